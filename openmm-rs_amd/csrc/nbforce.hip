@@ -1057,6 +1057,8 @@ void NbOperator::autotune(const double* pos_dev, unsigned* status, hipStream_t s
         for (int plane : {0, 1}) {
             if (!pme_set_fft_plane(pme_, sys_h_, prec, plane) && plane) continue;
             for (int cap : {16, 8, 4, 2}) {
+                // Matrix-core passes only: nothing to choose.
+                if (pme_.plane_blocks[prec] == 0 && best < 1e30) continue;
                 pme_set_fft_lines(pme_, sys_h_, prec, cap, s);
                 patch_layout(s);
                 const double t = timed(phase(PME_FFT));

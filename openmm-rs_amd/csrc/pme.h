@@ -8,12 +8,25 @@
 
 namespace ommhip {
 
+// What the matrix-core passes read of a system's record.  A lone system's is passed by
+// value: its workgroups start loading data without waiting for the table.
+struct MeshShape {
+    int grid[3], nzh, roots_off[3];
+    long long qgrid_off, cgrid_off;
+    __host__ __device__ static MeshShape of(const SysInfo& S) {
+        return MeshShape{{S.grid[0], S.grid[1], S.grid[2]}, S.nzh, {S.roots_off[0], S.roots_off[1], S.roots_off[2]},
+                         S.qgrid_off, S.cgrid_off};
+    }
+};
+
 struct PmeDev {
     int nsys = 0;
     long long qpoints = 0, cpoints = 0;  // real / half-spectrum points over all systems
     DevBuf<long long> qgrid_fx;  // mixed: fixed-point charge grids
     DevBuf<double> qgrid_d;      // plain: FP64 charge grids
-    DevBuf<float> cgrid_f;       // complex half-spectra [nx][ny][nzh] (interleaved re, im)
+    // Complex half-spectra: [nx][ny][nzh] (interleaved re, im), or the tiles of
+    // the matrix-core passes.
+    DevBuf<float> cgrid_f;
     DevBuf<double> cgrid_d;
     DevBuf<float> phi_f;         // real-space potentials [nx][ny][nz]
     DevBuf<double> phi_d;
@@ -31,8 +44,8 @@ struct PmeDev {
     // transform is three launches instead of five.  Available per precision
     // when every system's plane fits in LDS; results are the same bits as
     // the five-pass form.
-    DevBuf<int> plane_off;  // nsys + 1 prefix of x planes
-    int plane_blocks = 0;
+    DevBuf<int> plane_off[2];  // nsys + 1 prefix of x planes, per precision
+    int plane_blocks[2] = {};
     size_t plane_shmem[2] = {};  // dynamic LDS per plane workgroup, 0: unavailable
     bool plane[2] = {};          // use the plane decomposition
     int spread_edge = 0;  // spread tile edge
@@ -40,6 +53,14 @@ struct PmeDev {
     // of the tile-owned one; both write the same bits.
     bool spread_atoms = false;
     size_t fft_shmem[2][3] = {};  // dynamic LDS per axis
+    // Matrix-core passes (dft.h), for the systems of dft_system: workgroup
+    // prefix tables of the three passes per precision (the staged passes'
+    // tables hold no workgroups for these systems) and their dynamic LDS.
+    DevBuf<int> dft_off[2][3];
+    int dft_blocks[2][3] = {};
+    size_t dft_shmem[2][3] = {};
+    bool dft_wide[2] = {};  // eight waves per workgroup (some axis has more than 64 points)
+    MeshShape shape{};      // system 0's
     // Spread: per-atom stencils (base point, weights) and per-tile atom bins.
     int natoms = 0, ntiles = 0, bin_cap = 0;
     double max_charge = 0.0;        // largest |q| (selects the spread's int32 rounds)
@@ -60,6 +81,32 @@ struct PmeDev {
     int order_gen = -1;
     int order_sel = 0;
 };
+
+// Which systems transform by dense products on the matrix cores (DFT_COLS kz
+// values per tile) instead of the staged passes, per precision (0: FP32, 1:
+// FP64).  The dense products' work grows with n, the staged passes' with the
+// sum of n's prime factors (4 and 8 preferred).  Both transforms and the
+// convolution of n^3 points, staged then dense, microseconds:
+//   FP32: 19: 25, 14   55: 31, 21   72: 54, 39   96: 77, 71   120: 116, 104
+//         128: 129, 137   but 101: 228, 79 and 127: 430, 112
+//   FP64: 19: 27, 17   55: 37, 27   64: 46, 40   72: 68, 70   96: 110, 120
+//         but 101: 403, 130
+// so every axis has at most 120 (FP32) or 64 points (FP64), or at most DFT_MAX
+// with a prime factor above 16.  The rule depends on the system alone: a
+// replica's results are the same in any batch.
+constexpr int DFT_MAX = 128;
+constexpr int DFT_COLS = 8;
+__host__ __device__ inline int dft_tiles(int nzh) { return (nzh + DFT_COLS - 1) / DFT_COLS; }
+inline bool dft_axis(int n, int prec) {
+    if (n <= (prec ? 64 : 120)) return true;
+    int largest = 1, m = n;
+    for (int p = 2; p * p <= m; ++p)
+        for (; m % p == 0; m /= p) largest = p;
+    return n <= DFT_MAX && std::max(largest, m) > 16;
+}
+inline bool dft_system(const SysInfo& S, int prec) {
+    return dft_axis(S.grid[0], prec) && dft_axis(S.grid[1], prec) && dft_axis(S.grid[2], prec);
+}
 
 // Grid dimensions must each be >= 5 (pme.rs:222-225) and at most 1024.
 // Reads sys[s].grid and sys[s].alpha; writes the grid offsets, radices,

@@ -15,6 +15,7 @@
 #include <complex>
 #include <type_traits>
 
+#include "dft.h"
 #include "fmath.h"
 #include "pme.h"
 #include "spline.h"
@@ -24,11 +25,6 @@ namespace ommhip {
 namespace {
 
 constexpr int FFT_THREADS = 256;
-
-template <class R>
-struct Cx {
-    R x, y;
-};
 
 // Spread without atomics on the grid.  The grid of every system is cut into tiles
 // of ptile = 8 or 6 points per axis (the last tile of an axis takes the
@@ -524,19 +520,6 @@ __global__ __launch_bounds__(GATHER_ATOMS * 5) void k_gather5(const int* __restr
 
 enum : int { MODE_Z_R2C = 0, MODE_Y_FWD = 1, MODE_X_CONV = 2, MODE_Y_INV = 3, MODE_Z_C2R = 4 };
 
-
-__device__ __forceinline__ double grid_real(long long v) { return (double)v * (1.0 / GRID_SCALE); }
-__device__ __forceinline__ double grid_real(double v) { return v; }
-
-// x / d for 0 <= x < 2^20 and 1 <= d: a single-precision estimate corrected
-// by one step either way.
-__device__ __forceinline__ int div_small(int x, int d, float inv_d) {
-    int q = (int)((float)x * inv_d);
-    if (q * d > x) --q;
-    else if ((q + 1) * d <= x) ++q;
-    return q;
-}
-
 // Batched Stockham FFT of `lines` lines of length n held line-major in a/b,
 // T threads per line.  A stage of radix R is a direct DFT per output:
 // out[(j - k) R + k + q Ns] = sum_r in[j + r m] W_n^{r (k n/(Ns R) + q m)},
@@ -697,99 +680,22 @@ __global__ __launch_bounds__(FFT_THREADS) void k_fft(const int* __restrict__ blk
 
     if (MODE == MODE_X_CONV) {
         // Reciprocal convolution and energy (pme.rs:332-372) on the half spectrum.
-        const Box& b = S.box;
-        const R* mod_x = moduli_all + S.moduli_off[0];
-        const R* mod_y = moduli_all + S.moduli_off[1];
-        const R* mod_z = moduli_all + S.moduli_off[2];
-        const double pi2_a2 = PI * PI / (S.alpha * S.alpha);
-        const double pref = ONE_4PI_EPS0 / (PI * b.volume);
-        // Dispersion mesh (pme.rs:358-362): I(k) = -pi^1.5 / (3 V B(k))
-        // (2 pi^3 sqrt(pi) erfc(b) k^3 + e^{-b^2} (alpha^3 - 2 alpha pi^2 k^2)),
-        // b = pi k / alpha, with the k = 0 term kept.
-        const bool disp = S.dispersion != 0;
-        const double dpref = -PI * sqrt(PI) / (3.0 * b.volume);
-        const double dc1 = 2.0 * PI * PI * PI * sqrt(PI), da3 = S.alpha * S.alpha * S.alpha;
-        const double dc2 = 2.0 * S.alpha * PI * PI, pi_a = PI / S.alpha;
-        // The FP32 mesh serves force-only evaluations: the influence function
-        // in FP32 (exp2 of the hardware), no energy.  The FP64 meshes evaluate
-        // it in FP64 and sum the energy.
-        //
-        // The half spectrum stands for each point k and its mirror -k.  The
-        // reference sums the influence over the full grid and keeps the real
-        // part of the inverse transform, which is the half spectrum weighted
-        // by the mean influence of k and its mirror.  The mirror's frequency
-        // is -m on every axis except at a Nyquist index (2 k = n), where it is
-        // m itself; in a triclinic box |k|^2 then differs between the two, so
-        // those points take the mean of both influences.
         constexpr bool F32 = sizeof(R) == 4;
-        float rf[9];
-        for (int k = 0; k < 9; ++k) rf[k] = (float)b.recip[k];
-        const bool tric = b.triclinic != 0;
-        const float pi2_a2_log2e = (float)(pi2_a2 * 1.4426950408889634);
-        const float pref_f = (float)pref;
+        const Influence<R> I(S, moduli_all);
         double eacc = 0.0;
         for (int e = threadIdx.x; e < LINES * n; e += FFT_THREADS) {
             const int li = e % LINES, kx = e / LINES;
             const int L = line0 + li;
             if (L >= nlines) continue;
             const int y = L / nzh, kz = L - y * nzh;
-            Cx<R>& S = res[li * n + kx];
-            if (kx == 0 && y == 0 && kz == 0 && !disp) {
-                S = Cx<R>{0, 0};
-                continue;
+            Cx<R>& v = res[li * n + kx];
+            const R infl = I(kx, y, kz);
+            if (!F32) {
+                const double wz = (kz == 0 || 2 * kz == nz) ? 1.0 : 2.0;
+                eacc += wz * 0.5 * (double)infl * ((double)v.x * v.x + (double)v.y * v.y);
             }
-            // Mirror signs: the mirror's frequency is -m except at a Nyquist index.
-            const bool nyq = tric && (2 * kx == nx || 2 * y == ny || 2 * kz == nz);
-            const int sx = 2 * kx == nx ? 1 : -1, sy = 2 * y == ny ? 1 : -1, sz = 2 * kz == nz ? 1 : -1;
-            if (F32) {
-                const float mx = (float)(kx < (nx + 1) / 2 ? kx : kx - nx);
-                const float my = (float)(y < (ny + 1) / 2 ? y : y - ny);
-                const float mz = (float)(kz < (nz + 1) / 2 ? kz : kz - nz);
-                const float mod = (float)mod_x[kx] * (float)mod_y[y] * (float)mod_z[kz];
-                auto influence = [&](float ax, float ay, float az) {
-                    float k2 = 0.0f;
-                    for (int a = 0; a < 3; ++a) {
-                        const float kv = ax * rf[a] + ay * rf[3 + a] + az * rf[6 + a];
-                        k2 += kv * kv;
-                    }
-                    if (disp) {
-                        const float kk = __builtin_sqrtf(k2);
-                        float ec, ex;
-                        Math<float>::erfc_exp((float)pi_a * kk, ec, ex);
-                        return (float)dpref * ((float)dc1 * ec * kk * k2 + ex * ((float)da3 - (float)dc2 * k2)) /
-                               mod;
-                    }
-                    return pref_f * __builtin_amdgcn_exp2f(-pi2_a2_log2e * k2) / (k2 * mod);
-                };
-                float infl = influence(mx, my, mz);
-                if (nyq) infl = 0.5f * (infl + influence(-sx * mx, -sy * my, -sz * mz));
-                S.x = (R)((float)S.x * infl);
-                S.y = (R)((float)S.y * infl);
-                continue;
-            }
-            const double mx = kx < (nx + 1) / 2 ? kx : kx - nx;
-            const double my = y < (ny + 1) / 2 ? y : y - ny;
-            const double mz = kz < (nz + 1) / 2 ? kz : kz - nz;
-            const double mod = (double)mod_x[kx] * (double)mod_y[y] * (double)mod_z[kz];
-            auto influence = [&](double ax, double ay, double az) {
-                double k2 = 0.0;
-                for (int a = 0; a < 3; ++a) {
-                    double kv = ax * b.recip[0 * 3 + a] + ay * b.recip[1 * 3 + a] + az * b.recip[2 * 3 + a];
-                    k2 += kv * kv;
-                }
-                if (disp) {
-                    const double kk = sqrt(k2), bb = pi_a * kk;
-                    return dpref / mod * (dc1 * erfc(bb) * kk * k2 + exp(-bb * bb) * (da3 - dc2 * k2));
-                }
-                return pref * exp(-pi2_a2 * k2) / (k2 * mod);
-            };
-            double infl = influence(mx, my, mz);
-            if (nyq) infl = 0.5 * (infl + influence(-sx * mx, -sy * my, -sz * mz));
-            const double wz = (kz == 0 || 2 * kz == nz) ? 1.0 : 2.0;
-            const double s2 = (double)S.x * S.x + (double)S.y * S.y;
-            eacc += wz * 0.5 * infl * s2;
-            S.x = (R)(S.x * infl);
-            S.y = (R)(S.y * infl);
+            v.x *= infl;
+            v.y *= infl;
         }
         if (!F32) {
             double et = wave_sum(eacc);
@@ -1038,9 +944,35 @@ template <class R, class G, int DIR>
 void launch_plane(const PmeDev& pm, const SysInfo* sys, G* qgrid, Cx<R>* cgrid, R* phi, const R* roots,
                   hipStream_t s, int* clear = nullptr, int nclear = 0) {
     constexpr int prec = sizeof(R) == 8 ? 1 : 0;
-    hipLaunchKernelGGL((k_fft_plane<R, G, DIR>), dim3(pm.plane_blocks), dim3(PLANE_THREADS), pm.plane_shmem[prec], s,
-                       pm.plane_off.p, pm.nsys, sys, qgrid, cgrid, phi, reinterpret_cast<const Cx<R>*>(roots), clear,
+    hipLaunchKernelGGL((k_fft_plane<R, G, DIR>), dim3(pm.plane_blocks[prec]), dim3(PLANE_THREADS), pm.plane_shmem[prec], s,
+                       pm.plane_off[prec].p, pm.nsys, sys, qgrid, cgrid, phi, reinterpret_cast<const Cx<R>*>(roots), clear,
                        nclear);
+}
+
+// The matrix-core passes over the systems that take them.
+template <int W, class R, class G, class A>
+void launch_dft_w(const PmeDev& pm, const SysInfo* sys, G* qgrid, R* cgrid, R* phi, const Cx<R>* roots,
+                  const R* moduli, A* energy, unsigned* status, hipStream_t s, int* clear, int nclear) {
+    constexpr int prec = sizeof(R) == 8 ? 1 : 0;
+    const dim3 wg(64 * W);
+    hipLaunchKernelGGL((k_dft_zy<W, R, G>), dim3(pm.dft_blocks[prec][0]), wg, pm.dft_shmem[prec][0], s, pm.dft_off[prec][0].p,
+                       pm.nsys, sys, qgrid, cgrid, roots, pm.shape, clear, nclear);
+    hipLaunchKernelGGL((k_dft_x<W, R, G, A>), dim3(pm.dft_blocks[prec][1]), wg, pm.dft_shmem[prec][1], s, pm.dft_off[prec][1].p,
+                       pm.nsys, sys, qgrid, cgrid, roots, moduli, pm.shape, energy, status);
+    hipLaunchKernelGGL((k_dft_yz<W, R>), dim3(pm.dft_blocks[prec][2]), wg, pm.dft_shmem[prec][2], s, pm.dft_off[prec][2].p,
+                       pm.nsys, sys, cgrid, phi, roots, pm.shape);
+}
+
+template <class R, class G, class A>
+void launch_dft(const PmeDev& pm, const SysInfo* sys, G* qgrid, R* cgrid, R* phi, const R* roots_r, const R* moduli,
+                A* energy, unsigned* status, hipStream_t s, int* clear, int nclear) {
+    const Cx<R>* roots = reinterpret_cast<const Cx<R>*>(roots_r);
+    constexpr int prec = sizeof(R) == 8 ? 1 : 0;
+    if (pm.dft_wide[prec])
+        launch_dft_w<DFT_WAVES_WIDE, R, G, A>(pm, sys, qgrid, cgrid, phi, roots, moduli, energy, status, s, clear,
+                                              nclear);
+    else
+        launch_dft_w<DFT_WAVES, R, G, A>(pm, sys, qgrid, cgrid, phi, roots, moduli, energy, status, s, clear, nclear);
 }
 
 template <class R>
@@ -1095,7 +1027,13 @@ void run_t(PmeDev& pm, const NlistDev& nl, bool atom_order, const double* pos, c
         Cx<R>* cg = reinterpret_cast<Cx<R>*>(cgrid);
         int* clear = (phases & PME_SPREAD) ? pm.bin_count.p : nullptr;
         constexpr int prec = sizeof(R) == 8 ? 1 : 0;
-        if (pm.plane[prec]) {
+        if (pm.dft_blocks[prec][0] > 0) {
+            launch_dft<R, G, A>(pm, sys, qgrid, cgrid, phi, roots, moduli, energy, status, s, clear, pm.ntiles);
+            clear = nullptr;
+        }
+        if (pm.plane_blocks[prec] == 0) {
+            // Every system takes the matrix-core passes.
+        } else if (pm.plane[prec]) {
             launch_plane<R, G, 0>(pm, sys, qgrid, cg, phi, roots, s, clear, pm.ntiles);
             launch_fft<R, G, A, MODE_X_CONV>(pm, sys, qgrid, cg, phi, roots, moduli, energy, status, s);
             launch_plane<R, G, 1>(pm, sys, qgrid, cg, phi, roots, s);
@@ -1228,6 +1166,47 @@ int fft_nlines(const SysInfo& S, int a) {
 }
 }  // namespace
 
+namespace {
+// Workgroup tables and LDS of the matrix-core passes.
+void dft_setup(PmeDev& pm, const std::vector<SysInfo>& sys, hipStream_t s) {
+    pm.shape = MeshShape::of(sys[0]);
+    for (int prec = 0; prec < 2; ++prec) {
+        pm.dft_wide[prec] = false;
+        for (const SysInfo& S : sys)
+            for (int a = 0; a < 3; ++a)
+                if (dft_system(S, prec) && S.grid[a] > 16 * DFT_WAVES) pm.dft_wide[prec] = true;
+        const int waves = pm.dft_wide[prec] ? DFT_WAVES_WIDE : DFT_WAVES;
+        std::vector<int> off[3];
+        size_t lds[3] = {0, 0, 0};
+        for (int k = 0; k < 3; ++k) off[k].assign(1, 0);
+        for (const SysInfo& S : sys) {
+            const bool on = dft_system(S, prec);
+            const int nx = S.grid[0], ny = S.grid[1], nz = S.grid[2], tiles = dft_tiles(S.nzh);
+            const int blocks[3] = {nx * tiles, ny * tiles, nx * ((ny + 15) / 16)};
+            const size_t need[3] = {DftLds::zy(ny, nz, waves), DftLds::x(nx), DftLds::yz(ny, nz, tiles, waves)};
+            for (int k = 0; k < 3; ++k) {
+                off[k].push_back(off[k].back() + (on ? blocks[k] : 0));
+                if (on) lds[k] = std::max(lds[k], need[k]);
+            }
+        }
+        for (int k = 0; k < 3; ++k) {
+            pm.dft_off[prec][k].upload(off[k], s);
+            pm.dft_blocks[prec][k] = off[k].back();
+            pm.dft_shmem[prec][k] = lds[k] * (prec ? sizeof(double) : sizeof(float));
+        }
+    }
+    // Dynamic LDS above 64 KB per workgroup.
+    auto allow = [](const void* f) {
+        OMM_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)PLANE_LDS_MAX));
+    };
+    allow((const void*)&k_dft_zy<DFT_WAVES_WIDE, float, long long>);
+    allow((const void*)&k_dft_zy<DFT_WAVES_WIDE, double, long long>);
+    allow((const void*)&k_dft_zy<DFT_WAVES_WIDE, double, double>);
+    allow((const void*)&k_dft_yz<DFT_WAVES_WIDE, float>);
+    allow((const void*)&k_dft_yz<DFT_WAVES_WIDE, double>);
+}
+}  // namespace
+
 int pme_set_fft_lines(PmeDev& pm, std::vector<SysInfo>& sys, int prec, int cap, hipStream_t s) {
     const size_t csize = prec ? 2 * sizeof(double) : 2 * sizeof(float);
     if (cap <= 0) {
@@ -1257,8 +1236,9 @@ int pme_set_fft_lines(PmeDev& pm, std::vector<SysInfo>& sys, int prec, int cap, 
                 std::max(pm.fft_shmem[prec][a], (2 * (size_t)S.fft_lines[prec][a] * S.grid[a] + S.grid[a]) * csize);
         }
         for (int k = 0; k < 5; ++k) {
-            const int a = PASS_AXIS[k];
-            off[k].push_back(off[k].back() + (fft_nlines(S, a) + S.fft_lines[prec][a] - 1) / S.fft_lines[prec][a]);
+            const int l = S.fft_lines[prec][PASS_AXIS[k]];
+            const int blocks = (fft_nlines(S, PASS_AXIS[k]) + l - 1) / l;
+            off[k].push_back(off[k].back() + (dft_system(S, prec) ? 0 : blocks));
         }
     }
     for (int k = 0; k < 5; ++k) {
@@ -1356,7 +1336,8 @@ void pme_setup(PmeDev& pm, std::vector<SysInfo>& sys, int natoms, const int* ato
         S.qgrid_off = qpts;
         S.cgrid_off = cpts;
         qpts += (long long)S.grid[0] * S.grid[1] * S.grid[2];
-        cpts += (long long)S.grid[0] * S.grid[1] * S.nzh;
+        // The matrix-core passes pad kz to whole tiles.
+        cpts += (long long)S.grid[0] * S.grid[1] * (dft_system(S, 0) || dft_system(S, 1) ? DFT_COLS * dft_tiles(S.nzh) : S.nzh);
         for (int a = 0; a < 3; ++a) {
             const int n = S.grid[a];
             std::vector<int> f = factorize(n);
@@ -1380,10 +1361,12 @@ void pme_setup(PmeDev& pm, std::vector<SysInfo>& sys, int natoms, const int* ato
     pme_set_fft_lines(pm, sys, 0, 0, s);
     pme_set_fft_lines(pm, sys, 1, 0, s);
     {
-        std::vector<int> poff{0};
-        for (const SysInfo& S : sys) poff.push_back(poff.back() + S.grid[0]);
-        pm.plane_off.upload(poff, s);
-        pm.plane_blocks = poff.back();
+        for (int prec = 0; prec < 2; ++prec) {
+            std::vector<int> poff{0};
+            for (const SysInfo& S : sys) poff.push_back(poff.back() + (dft_system(S, prec) ? 0 : S.grid[0]));
+            pm.plane_off[prec].upload(poff, s);
+            pm.plane_blocks[prec] = poff.back();
+        }
         // Dynamic LDS above 64 KB per workgroup.
         const int lds = (int)PLANE_LDS_MAX;
         OMM_HIP(hipFuncSetAttribute((const void*)&k_fft_plane<float, long long, 0>,
@@ -1400,6 +1383,7 @@ void pme_setup(PmeDev& pm, std::vector<SysInfo>& sys, int natoms, const int* ato
                                     hipFuncAttributeMaxDynamicSharedMemorySize, lds));
         for (int prec = 0; prec < 2; ++prec) pme_set_fft_plane(pm, sys, prec, -1);
     }
+    dft_setup(pm, sys, s);
     pme_set_spread_edge(pm, sys, 0, s);
     pm.st_idx.alloc(4 * (size_t)pm.natoms);
     if (mixed) pm.st_wf.alloc(16 * (size_t)pm.natoms);
