@@ -46,9 +46,10 @@ struct BaroState {
 // constraints in the reference's order (constraints only couple atoms of a
 // component, so this is the reference's global Gauss-Seidel loop).
 struct ConstraintDev {
-    int ncomp = 0, ncons = 0;
+    int ncomp = 0, ncons = 0, natoms = 0;  // natoms: constrained atoms
+    int shape_count[2] = {0, 0};  // triangles, then stars: the first components (k_constrained_shape)
     double tolerance = 1e-5;
-    DevBuf<int> atom_off, atoms;  // [ncomp + 1] prefix, atoms of each component (ascending)
+    DevBuf<int> atom_off, atoms;  // [ncomp + 1] prefix, atoms of each component (in its shape's order, or ascending)
     DevBuf<int> cons_off;         // [ncomp + 1] prefix into the constraint arrays
     DevBuf<int> c1, c2;           // global particle indices, reference order within a component
     DevBuf<double> d2, w1, w2;    // distance^2, inverse masses
@@ -187,6 +188,9 @@ public:
 
 private:
     double default_box_[9] = {};  // a non-periodic system's default box vectors
+    template <class A>
+    void launch_constraints(A* force, double tolerance, int mode, double decay, double variance, int offset,
+                            double lim2, int check, hipStream_t s);
     void enqueue_forces(hipStream_t s, bool energy, int rebuild);
     void enqueue_forces_into(hipStream_t s, bool energy, int rebuild, long long* force_fx, double* force_d,
                              long long* energy_fx, double* energy_d);

@@ -135,3 +135,34 @@ def test_constrained_batch_matches_single_contexts():
         c.set_velocities_to_temperature(300.0, 20 + r)
         c.step(30)
         assert np.array_equal(b.get_state(r)["positions"], c.get_state()["positions"])
+
+
+@pytest.mark.parametrize("precision,tol", [(ommhip.PRECISION_DOUBLE, 1e-11), (ommhip.PRECISION_MIXED, 1e-9)])
+def test_components_of_every_size_match_oracle(precision, tol):
+    # One system with triangles in several orders, stars of one to three bonds
+    # (both projected in registers), chains and larger components (through
+    # memory), mixed, against the oracle's solver over all constraints; bars as
+    # for rigid water.
+    s = rigid(water(300, 2.1, seed=75))
+    full = s.constraints
+    keep = []
+    for m in range(300):
+        c = full[3 * m : 3 * m + 3]
+        keep += [c[:1], c[:2], c, [c[2], c[0]], [c[1], c[2], c[0]], [(c[0][1], c[0][0], c[0][2]), c[2], c[1]], c][m % 7]
+    for m in range(0, 290, 10):  # this molecule's oxygen to atoms of the next one, or of the next two
+        for a, b in ((3 * m, 3 * m + 3), (3 * m, 3 * m + 7 if m % 20 else 3 * m + 4)):
+            keep.append((a, b, float(np.linalg.norm(s.positions[a] - s.positions[b]))))
+    s.constraints = keep
+    rng = np.random.default_rng(8)
+    v0 = rng.normal(scale=0.4, size=s.positions.shape)
+    ctx = ommhip.Context(s, temperature=0.0, friction=0.0, step_size=0.0005, precision=precision)
+    ctx.set_velocities(v0)
+    ctx.step(1)
+    st = ctx.get_state()
+    F, _ = orc.water_energy_forces(s)
+    x1, v1 = orc.lfmiddle_step_constrained(s.positions, v0, F, s.masses, 0.0005, 0.0, 0.0, s.constraints, 1e-5)
+    dx = np.abs(st["positions"] - x1.reshape(-1, 3)).max()
+    dv = np.abs(st["velocities"] - v1.reshape(-1, 3)).max()
+    print(f"max |dx| = {dx:.3e} nm, max |dv| = {dv:.3e} nm/ps")
+    assert dx < tol
+    assert dv < 1e3 * tol
