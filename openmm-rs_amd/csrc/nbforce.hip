@@ -448,7 +448,9 @@ void NbOperator::setup_device(const std::vector<Box>& boxes) {
             pp_.crf = (3.0 * eps) / (2.0 * eps + 1.0) / rc;
         }
     }
-    pair_grid_ = std::max(64, std::min(8192, nl_.nblocks * 4));
+    // Waves of the pair kernels until a calibration counts the tasks: about
+    // eight tiles a cluster (waves past the last task leave at once).
+    pair_grid_ = std::max(64, std::min(65535, nl_.nclusters * 8 / nl_.tpt));
 
     if (nsys == 1) {
         pos_dev_.alloc(3 * (size_t)N);
@@ -1122,7 +1124,7 @@ bool NbOperator::calibrate(const double* pos_dev, unsigned* status, hipStream_t 
         long long tasks = 0;
         for (int c : ccounts) {
             mx = std::max(mx, c);
-            tasks += ((c + JTILE - 1) / JTILE + TPT - 1) / TPT;
+            tasks += ((c + JTILE - 1) / JTILE + nl_.tpt - 1) / nl_.tpt;
         }
         // One wave per task of the calibrated list (grid-stride beyond it):
         // enough resident waves to hide the latency of the pair loop.

@@ -28,7 +28,6 @@ constexpr int CPB = IBLOCK / CLUSTER;  // clusters per block
 constexpr int SUPER = 64;   // blocks per superblock (the coarse level of the candidate search)
 constexpr int SUPER_MIN = 1024;  // systems with more blocks search superblocks first
 constexpr int JTILE = 64;   // j-slots per tile
-constexpr int TPT = 4;      // tiles of one cluster per pair-kernel task
 constexpr int PME_CHUNK = 64;  // sorted slots per PME spread/gather workgroup
 
 // Squared displacement of an atom from its position at the last list build,
@@ -53,6 +52,7 @@ struct NlistDev {
     int natoms = 0, nslots = 0, nblocks = 0, nclusters = 0, nchunks = 0, cap = 0, nunits = 0, ncells = 0;
     int uniform = 0;  // atoms per unit when all units are the same size, else 0
     int closed = 0;   // every exception pair lies inside one unit
+    int tpt = 4;  // tiles of one cluster per pair-kernel task (see tiles_per_task)
     double cutoff = 0, skin = 0;
     DevBuf<int> unit_ptr, unit_atoms, unit_pos, unit_sys, unit_key, cell_rank, cell_count, cell_start, cell_cursor;
     DevBuf<int> sorted_units, unit_size_sorted, unit_offset;

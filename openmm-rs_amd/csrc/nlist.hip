@@ -497,7 +497,7 @@ __global__ __launch_bounds__(64) void k_super_bounds(int nsuper, const int* __re
 // the cluster's own atoms and of every atom of those blocks within reach
 // (the pair kernel takes an entry of the cluster's own slots only after the
 // i-atom), and the cluster appends its pair-kernel tasks: one run of up
-// to TPT tiles of JTILE entries per task, packed as cluster * 256 + first
+// to tpt tiles of JTILE entries per task, packed as cluster * 256 + first
 // tile (their order in the table does not matter, as forces are fixed-point
 // sums; one atomic per workgroup reserves the runs of its clusters).  The
 // atoms of four passing blocks are loaded together, so their loads overlap.
@@ -620,8 +620,8 @@ __global__ __launch_bounds__(64 * W) void k_clist(
     const int* __restrict__ super_off, const double* __restrict__ super_center,
     const float* __restrict__ super_half, const int* __restrict__ atom_slot, const int* __restrict__ excl_ptr,
     const int* __restrict__ excl_idx, const int2* __restrict__ excl_range, const int* __restrict__ minimg,
-    const float4* __restrict__ slot_pos, double reach, int cap, int nclusters, int2* clist, unsigned char* clist_ex,
-    int* ccount, int* tasks, int* ntasks, unsigned* status, const int* flag) {
+    const float4* __restrict__ slot_pos, double reach, int cap, int nclusters, int tpt, int2* clist,
+    unsigned char* clist_ex, int* ccount, int* tasks, int* ntasks, unsigned* status, const int* flag) {
     __shared__ int s_runs[W];
     __shared__ int s_base;
     if (!flag[0]) return;
@@ -801,7 +801,7 @@ __global__ __launch_bounds__(64 * W) void k_clist(
     } else if (C < nclusters) {
         if (lane == 0) ccount[C] = 0;  // a cluster of padding only
     }
-    const int runs = ((count + JTILE - 1) / JTILE + TPT - 1) / TPT;
+    const int runs = ((count + JTILE - 1) / JTILE + tpt - 1) / tpt;
     if (lane == 0) s_runs[wave] = runs;
     __syncthreads();
     if (threadIdx.x == 0) {
@@ -812,7 +812,7 @@ __global__ __launch_bounds__(64 * W) void k_clist(
     __syncthreads();
     int base = s_base;
     for (int w = 0; w < wave; ++w) base += s_runs[w];
-    for (int k = lane; k < runs; k += 64) tasks[base + k] = (C << 8) | (k * TPT);
+    for (int k = lane; k < runs; k += 64) tasks[base + k] = (C << 8) | (k * tpt);
 }
 
 // Position of cell (x, y, z) along a 3-D Hilbert curve over a 2^bits cube
@@ -844,6 +844,13 @@ uint64_t hilbert3(uint32_t x, uint32_t y, uint32_t z, int bits) {
         for (int i = 0; i < 3; ++i) h = (h << 1) | ((X[i] >> b) & 1u);
     return h;
 }
+
+// Tiles per pair-kernel task, for nblocks blocks over all systems: four where
+// the tasks fill the chip, fewer where they would leave SIMDs idle (pair kernel,
+// four tiles and these: 900 atoms 13.4 -> 7.0 us, 3,000 15.1 -> 10.9, 9,000 19.1 ->
+// 17.5; at 23,550 fewer than four were slower).  Forces and energies do not
+// depend on it: the tiles' sums are exact in any grouping.
+inline int tiles_per_task(int nblocks) { return nblocks <= 64 ? 1 : (nblocks <= 384 ? 2 : 4); }
 
 inline int blocks_for(long long n, int t) { return (int)((n + t - 1) / t); }
 
@@ -987,6 +994,7 @@ void nlist_setup(NlistDev& nl, const std::vector<NlistSystem>& systems, std::vec
     nl.nclusters = nblocks * CPB;
     nl.nslots = nblocks * IBLOCK;
     nl.nchunks = nchunks;
+    nl.tpt = tiles_per_task(nblocks);
     nl.nunits = (int)uptr.size() - 1;
     nl.ncells = ncells;
     // List capacity: the atoms within reach of a compact cluster at liquid
@@ -1038,7 +1046,7 @@ void nlist_setup(NlistDev& nl, const std::vector<NlistSystem>& systems, std::vec
     nl.cap = std::min(nl.cap, 255 * JTILE);
     nl.clist.alloc((size_t)nl.nclusters * nl.cap);
     nl.clist_ex.alloc((size_t)nl.nclusters * nl.cap);
-    nl.tasks.alloc((size_t)nl.nclusters * ((nl.cap / JTILE + TPT - 1) / TPT));
+    nl.tasks.alloc((size_t)nl.nclusters * ((nl.cap / JTILE + nl.tpt - 1) / nl.tpt));
     nl.ntasks.alloc(1);
     nl.ccount.alloc(nl.nclusters);
     nl.fslot_fx.alloc(3 * (size_t)nl.nslots);
@@ -1057,7 +1065,7 @@ void nlist_resize(NlistDev& nl, int cap) {
     nl.cap = cap;
     nl.clist.alloc((size_t)nl.nclusters * nl.cap);
     nl.clist_ex.alloc((size_t)nl.nclusters * nl.cap);
-    nl.tasks.alloc((size_t)nl.nclusters * ((nl.cap / JTILE + TPT - 1) / TPT));
+    nl.tasks.alloc((size_t)nl.nclusters * ((nl.cap / JTILE + nl.tpt - 1) / nl.tpt));
 }
 
 void nlist_check(NlistDev& nl, const double* pos, int force, hipStream_t s) {
@@ -1123,7 +1131,7 @@ void nlist_build(NlistDev& nl, const double* pos, const SysInfo* sys_dev, unsign
         hipLaunchKernelGGL(kernel, dim3(blocks_for(nl.nclusters, w)), dim3(64 * w), 0, s, pos, nl.sorted_atom.p,
                            nl.block_sys.p, sys_dev, nl.block_center.p, nl.block_half.p, nl.super_off.p,
                            nl.super_center.p, nl.super_half.p, nl.atom_slot.p, nl.excl_ptr.p, nl.excl_idx.p,
-                           nl.excl_range.p, nl.block_minimg.p, nl.slot_pos.p, reach, nl.cap, nl.nclusters, nl.clist.p,
+                           nl.excl_range.p, nl.block_minimg.p, nl.slot_pos.p, reach, nl.cap, nl.nclusters, nl.tpt, nl.clist.p,
                            nl.clist_ex.p, nl.ccount.p, nl.tasks.p, nl.ntasks.p, status, flag);
     };
     if (nl.nsys == 1)

@@ -1,7 +1,7 @@
 // Direct-space LJ + Ewald-screened Coulomb over the tile list, and the
 // exception kernel (nonbonded.rs:842-924, 995-1036).
 //
-// One wave64 per task = (cluster of 8 i-atoms, up to TPT consecutive tiles
+// One wave64 per task = (cluster of 8 i-atoms, up to tpt consecutive tiles
 // of 64 entries of the cluster's list); the loads of the next tiles are in
 // flight while a tile is evaluated.  Lane l owns i-atom l%8 and the group of entries
 // 8*(l/8) .. 8*(l/8)+7; in step k (0..7) it pairs with entry 8*(l/8) + (l%8 ^ k),
@@ -14,9 +14,9 @@
 // Near-cutoff pairs (|r^2 - rc^2| < 1e-5 rc^2) are re-decided in FP64 with
 // the reference's exact arithmetic, which makes the pair set bit-exact.
 //
-// Energy mode: forces stay on the FP32 path, and each pair's energy is
-// evaluated in FP64 from FP64 offsets.  The Coulomb classes of a water box
-// (O-O, O-H, H-H) are each ~1e6 kJ/mol and cancel to ~1e2-1e3, so any
+// Energies of the mixed form: k_pair_energy evaluates each pair in FP64 from
+// FP64 offsets, beside the FP32 forces.  The Coulomb classes of a water box (O-O,
+// O-H, H-H) are each ~1e6 kJ/mol and cancel to ~1e2-1e3, so any
 // distance-dependent FP32 rounding bias would survive in the sum; FP64 pair
 // energies remove it.  The MD step does not request energies and never pays
 // for this.
@@ -66,16 +66,19 @@ __device__ __forceinline__ void lj_switch(R r, const PairParams& P, R& s, R& ds)
     ds = (R)-30 * t * t * ((R)1 - t) * ((R)1 - t) * inv_width;
 }
 
-// FP64 energy of one pair (nonbonded.rs:1203-1214, 1219-1273) from offsets.
+// FP64 energy of one pair (nonbonded.rs:1203-1214, 1219-1273) at squared distance r2.
 template <int KIND>
-__device__ __forceinline__ double pair_energy_fp64(double dx, double dy, double dz, double sig, double eps4,
-                                                   double ss, double qq, const PairParams& P) {
+__device__ __forceinline__ double pair_energy_fp64(double r2, double sig, double eps4, double ss, double qq,
+                                                   const PairParams& P) {
     constexpr int ELEC = KIND & ELEC_MASK;
-    const double r2 = dx * dx + dy * dy + dz * dz;
-    const double r = sqrt(r2);
+    // Straight-line: nearly every wave holds pairs with and without LJ and
+    // charge, whose terms vanish by their factors eps4 and qq.
+    using M = PairF64;
+    const double inv_r = M::rsqrt(r2);
+    const double r = r2 * inv_r;
     double e = 0.0;
-    if (eps4 != 0.0) {
-        const double s2 = sig * sig / r2;
+    {
+        const double s2 = sig * sig * (inv_r * inv_r);
         const double s6 = s2 * s2 * s2;
         e = eps4 * (s6 * s6 - s6);
         if (KIND & PAIR_LJPME) {
@@ -93,18 +96,22 @@ __device__ __forceinline__ double pair_energy_fp64(double dx, double dy, double 
             e *= sw;
         }
     }
-    if (qq != 0.0) {
-        if (ELEC == ELEC_EWALD) e += qq * erfc(P.alpha * r) / r;
-        else if (ELEC == ELEC_REACTION_FIELD) e += qq * (1.0 / r + P.krf * r2 - P.crf);
-        else e += qq / r;
+    if (ELEC == ELEC_EWALD) {
+        double ec, ex;
+        M::erfc_exp(P.alpha * r, ec, ex);
+        e += qq * ec * inv_r;
+    } else if (ELEC == ELEC_REACTION_FIELD) {
+        e += qq * (inv_r + P.krf * r2 - P.crf);
+    } else {
+        e += qq * inv_r;
     }
     return e;
 }
 
 // Lane permutations by DPP inside each row of 16 lanes: quad_perm [1,0,3,2]
 // is lane ^ 1, quad_perm [3,2,1,0] is lane ^ 3, row_half_mirror is lane ^ 7
-// (each group of 8 reversed), row_ror:8 is lane ^ 8.
-constexpr int DPP_XOR1 = 0xB1, DPP_XOR3 = 0x1B, DPP_XOR7 = 0x141, DPP_XOR8 = 0x128;
+// (each group of 8 reversed).
+constexpr int DPP_XOR1 = 0xB1, DPP_XOR3 = 0x1B, DPP_XOR7 = 0x141;
 
 // Every control used here reads a lane of the same row, so no lane falls
 // back to an old value and the move needs none.
@@ -131,59 +138,114 @@ __device__ __forceinline__ void rotate_j(R& gx, R& gy, R& gz) {
 }
 
 // Raw data of one tile entry as loaded from HBM, before it is staged in LDS.
-template <class R, bool E64>
+template <class R>
 struct EntryRaw {
     double x = 0, y = 0, z = 0;
     R q = 0, s = 0, e = 0;
-    double qd = 0, sd = 0, ed = 0;  // the energy path's FP64 parameters
 };
 
 // Loads the data of atom a >= 0 with no branch: the entries past the end of
 // a list load some real atom's data and are masked when their tile is staged,
 // so the loads of a tile never wait on a branch's merge.
-template <class R, bool E64>
+template <class R>
 __device__ __forceinline__ void load_entry(const int a, const double* __restrict__ pos, const R* __restrict__ qk,
-                                           const R* __restrict__ sh, const R* __restrict__ e2,
-                                           const double* __restrict__ qk_d, const double* __restrict__ sh_d,
-                                           const double* __restrict__ e2_d, EntryRaw<R, E64>& r) {
+                                           const R* __restrict__ sh, const R* __restrict__ e2, EntryRaw<R>& r) {
     r.x = pos[3 * a];
     r.y = pos[3 * a + 1];
     r.z = pos[3 * a + 2];
     r.q = qk[a];
     r.s = sh[a];
     r.e = e2[a];
-    if (E64) {
-        r.qd = qk_d[a];
-        r.sd = sh_d[a];
-        r.ed = e2_d[a];
+}
+
+// Valid entries of the lane's group for i-atom `is` (slot): present, not
+// excluded, and after the i-atom where they are of its own cluster (entries
+// before the cluster's first slot come from blocks the cluster takes
+// cyclically).  il: the i-atom's index in the cluster.
+__device__ __forceinline__ unsigned valid_entries(const int* js, const unsigned char* ex, int is, int il) {
+    const int4* g4 = reinterpret_cast<const int4*>(js);
+    const int4 lo = g4[0], hi = g4[1];
+    const int jv[CLUSTER] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+    const int cfirst = is & ~(CLUSTER - 1);
+    unsigned vmask = 0;
+#pragma unroll
+    for (int s8 = 0; s8 < CLUSTER; ++s8)
+        if (jv[s8] != INT_MAX && (jv[s8] > is || jv[s8] < cfirst)) vmask |= 1u << s8;
+    // Bit il of each of the group's eight exclusion bytes, gathered into bits
+    // 0-7: each byte's bit il moves to the byte's bit 0, and a multiply by
+    // 2^0 + 2^7 + 2^14 + 2^21 carries the bits of bytes 0-3 (positions 0, 8, 16,
+    // 24) to positions 21-24 without collisions.
+    const unsigned long long xb = *reinterpret_cast<const unsigned long long*>(ex);
+    const unsigned long long sel = (xb >> il) & 0x0101010101010101ull;
+    const unsigned lo4 = (((unsigned)sel * 0x00204081u) >> 21) & 0xFu;
+    const unsigned hi4 = (((unsigned)(sel >> 32) * 0x00204081u) >> 21) & 0xFu;
+    return vmask & ~(lo4 | (hi4 << 4));
+}
+
+// A lane's force on its i-atom over a task.  Mixed form: each tile's FP32 sum
+// is rounded to multiples of 2^-28 (3.7e-9 kJ/mol/nm) by adding and subtracting
+// 1.5 x 2^24, where FP64 has that step, and the multiples are added in FP64,
+// exactly in any grouping while sums stay below 2^24; so the total does not
+// depend on how many tiles a task holds.  Four instructions per component and
+// tile; converting each tile's sum to the accumulators' fixed point cost 5% of
+// the kernel at 300,000 atoms.
+struct FixedForce {
+    static constexpr double STEP = 25165824.0;  // 1.5 x 2^24
+    double x = 0, y = 0, z = 0;
+    static __device__ __forceinline__ double rounded(float f) { return ((double)f + STEP) - STEP; }
+    __device__ __forceinline__ void add(float fx, float fy, float fz) {
+        x += rounded(fx);
+        y += rounded(fy);
+        z += rounded(fz);
     }
+    static __device__ __forceinline__ long long total(double v, unsigned* status) {
+        return to_fixed(v, FORCE_SCALE, status);
+    }
+};
+struct PlainForce {
+    double x = 0, y = 0, z = 0;
+    __device__ __forceinline__ void add(double fx, double fy, double fz) {
+        x += fx;
+        y += fy;
+        z += fz;
+    }
+    static __device__ __forceinline__ double total(double v, unsigned*) { return v; }
+};
+// Sum over the eight groups (lanes l, l ^ 8, l ^ 16, ...).
+template <class T>
+__device__ __forceinline__ T group_sum(T v) {
+    for (int o = CLUSTER; o < 64; o <<= 1) v += __shfl_xor(v, o, 64);
+    return v;
+}
+__device__ __forceinline__ void add_total(long long* p, long long v) {
+    if (v) atomicAdd(reinterpret_cast<unsigned long long*>(p), (unsigned long long)v);
+}
+__device__ __forceinline__ void add_total(double* p, double v) {
+    if (v != 0.0) unsafeAtomicAdd(p, v);
 }
 
 template <class R, class A, int KIND, bool STATS, bool ENERGY>
 __global__ __launch_bounds__(64) void k_pairs(const double* __restrict__ pos, const R* __restrict__ qk,
                                               const R* __restrict__ sh, const R* __restrict__ e2,
-                                              const double* __restrict__ qk_d, const double* __restrict__ sh_d,
-                                              const double* __restrict__ e2_d, const int* __restrict__ sorted_atom,
+                                              const int* __restrict__ sorted_atom,
                                               const unsigned char* __restrict__ clist_ex,
                                               const double* __restrict__ center,
                                               const int* __restrict__ minimg, const int2* __restrict__ clist,
                                               const int* __restrict__ ccount, const int* __restrict__ tasks,
                                               const int* __restrict__ ntasks, const int* __restrict__ block_sys,
-                                              const SysInfo* __restrict__ sys, PairParams P, A* fslot, A* energy,
+                                              const SysInfo* __restrict__ sys, PairParams P, int tpt, A* fslot, A* energy,
                                               unsigned* status, unsigned long long* stats, int* list_flag,
                                               int nflags) {
     using M = Math<R>;
     constexpr int ELEC = KIND & ELEC_MASK;
     constexpr bool SWITCH = (KIND & PAIR_SWITCH) != 0;
     constexpr bool LJPME = (KIND & PAIR_LJPME) != 0;
-    constexpr bool E64 = ENERGY && sizeof(R) == 4;  // separate FP64 energy path
+    static_assert(!ENERGY || sizeof(R) == 8, "the mixed form's energies: k_pair_energy");
     __shared__ Q4<R> s_pq[JTILE];
     __shared__ Q2<R> s_se[JTILE];
     __shared__ __align__(16) int s_js[JTILE];
     __shared__ int s_ja[JTILE];
     __shared__ __align__(8) unsigned char s_ex[JTILE];  // exclusion bits of each entry (bit k: i-atom k)
-    __shared__ Q4<double> s_pd[E64 ? JTILE : 1];
-    __shared__ Q2<double> s_sd[E64 ? JTILE : 1];
 
     const int lane = threadIdx.x;
     const int grp = lane / CLUSTER;  // the lane's group of 8 tile entries
@@ -208,7 +270,7 @@ __global__ __launch_bounds__(64) void k_pairs(const double* __restrict__ pos, co
         const int first = task & 255;
         const int I = C / CPB;
         const int count = ccount[C];
-        const int ntile = min(TPT, (count + JTILE - 1) / JTILE - first);
+        const int ntile = min(tpt, (count + JTILE - 1) / JTILE - first);
         const int sidx = block_sys[I];
         const Box& bx = sys[sidx].box;
         const double c0 = center[3 * I], c1 = center[3 * I + 1], c2 = center[3 * I + 2];
@@ -235,17 +297,10 @@ __global__ __launch_bounds__(64) void k_pairs(const double* __restrict__ pos, co
         const int ia0 = max(ia, 0);
         const double pxi = pos[3 * ia0], pyi = pos[3 * ia0 + 1], pzi = pos[3 * ia0 + 2];
         const R qi_raw = qk[ia0], si_raw = sh[ia0], ei_raw = e2[ia0];
-        double qid_raw = 0, sid_raw = 0, eid_raw = 0;
-        if (E64) {
-            qid_raw = qk_d[ia0];
-            sid_raw = sh_d[ia0];
-            eid_raw = e2_d[ia0];
-        }
-        EntryRaw<R, E64> r0;
-        load_entry<R, E64>(max(e0.y, 0), pos, qk, sh, e2, qk_d, sh_d, e2_d, r0);
+        EntryRaw<R> r0;
+        load_entry<R>(max(e0.y, 0), pos, qk, sh, e2, r0);
 
         R xi = 0, yi = 0, zi = 0, qi = 0, si = 0, ei = 0;
-        double xid = 0, yid = 0, zid = 0, qid = 0, sid = 0, eid = 0;
         if (ia >= 0) {
             double d[3] = {pxi - c0, pyi - c1, pzi - c2};
             if (P.periodic) wrap_nearest(d, bx);
@@ -255,14 +310,6 @@ __global__ __launch_bounds__(64) void k_pairs(const double* __restrict__ pos, co
             qi = qi_raw;
             si = si_raw;
             ei = ei_raw;
-            if (E64) {
-                xid = d[0];
-                yid = d[1];
-                zid = d[2];
-                qid = qid_raw;
-                sid = sid_raw;
-                eid = eid_raw;
-            }
         }
         // The pair steps read the i-atom's parameters inside divergent
         // branches, where the compiler cannot prove an earlier wait and
@@ -270,7 +317,6 @@ __global__ __launch_bounds__(64) void k_pairs(const double* __restrict__ pos, co
         // included, in each step.  Reading them here once, on every path,
         // completes their loads before the tiles start.
         asm volatile("" ::"v"(qi), "v"(si), "v"(ei));
-        if (E64) asm volatile("" ::"v"(qid), "v"(sid), "v"(eid));
         const bool mi = P.periodic && minimg[I];
         R bv[9], ib0 = 0, ib4 = 0, ib8 = 0;
         if (mi) {
@@ -280,14 +326,15 @@ __global__ __launch_bounds__(64) void k_pairs(const double* __restrict__ pos, co
             ib8 = (R)(1.0 / bx.v[8]);
         }
 
-        R fx = 0, fy = 0, fz = 0;
+        using Force = typename std::conditional<sizeof(R) == 4, FixedForce, PlainForce>::type;
+        Force ftot;
         double eacc = 0.0;
         unsigned long long npair = 0, hsum = 0;
         for (int k = 0; k < ntile; ++k) {
             const int2 e2n = entry(k + 2);
             const unsigned x2n = entry_ex(k + 2);
-            EntryRaw<R, E64> r1;
-            load_entry<R, E64>(max(e1.y, 0), pos, qk, sh, e2, qk_d, sh_d, e2_d, r1);
+            EntryRaw<R> r1;
+            load_entry<R>(max(e1.y, 0), pos, qk, sh, e2, r1);
 
             // Stage tile k in LDS as offsets from the block centre.
             {
@@ -297,55 +344,24 @@ __global__ __launch_bounds__(64) void k_pairs(const double* __restrict__ pos, co
                 }
                 Q4<R> pq = {0, 0, 0, 0};
                 Q2<R> se = {0, 0};
-                Q4<double> pd = {0, 0, 0, 0};
-                Q2<double> sd = {0, 0};
                 if (e0.y >= 0) {
                     double d[3] = {r0.x - c0, r0.y - c1, r0.z - c2};
                     if (P.periodic) wrap_nearest(d, bx);
                     pq = {(R)d[0], (R)d[1], (R)d[2], r0.q};
                     se = {r0.s, r0.e};
-                    if (E64) {
-                        pd = {d[0], d[1], d[2], r0.qd};
-                        sd = {r0.sd, r0.ed};
-                    }
                 }
                 s_pq[lane] = pq;
                 s_se[lane] = se;
                 s_js[lane] = e0.x;
                 s_ja[lane] = e0.y;
                 s_ex[lane] = (unsigned char)x0;
-                if (E64) {
-                    s_pd[lane] = pd;
-                    s_sd[lane] = sd;
-                }
             }
             __syncthreads();
 
-            // Valid entries of the lane's group: present, not excluded, and
-            // after the i-atom where they are of its own cluster (entries
-            // before the cluster's first slot come from blocks the cluster
-            // takes cyclically).
             unsigned vmask = 0;
-            if (ia >= 0) {
-                const int4* g4 = reinterpret_cast<const int4*>(s_js + grp * CLUSTER);
-                const int4 lo = g4[0], hi = g4[1];
-                const int jv[CLUSTER] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
-                const int cfirst = is & ~(CLUSTER - 1);
-#pragma unroll
-                for (int s8 = 0; s8 < CLUSTER; ++s8)
-                    if (jv[s8] != INT_MAX && (jv[s8] > is || jv[s8] < cfirst)) vmask |= 1u << s8;
-                // Bit il of each of the group's eight exclusion bytes, gathered
-                // into bits 0-7: each byte's bit il moves to the byte's bit 0,
-                // and a multiply by 2^0 + 2^7 + 2^14 + 2^21 carries the bits of
-                // bytes 0-3 (positions 0, 8, 16, 24) to positions 21-24
-                // without collisions.
-                const unsigned long long xb = *reinterpret_cast<const unsigned long long*>(s_ex + grp * CLUSTER);
-                const unsigned long long sel = (xb >> il) & 0x0101010101010101ull;
-                const unsigned lo4 = (((unsigned)sel * 0x00204081u) >> 21) & 0xFu;
-                const unsigned hi4 = (((unsigned)(sel >> 32) * 0x00204081u) >> 21) & 0xFu;
-                vmask &= ~(lo4 | (hi4 << 4));
-            }
+            if (ia >= 0) vmask = valid_entries(s_js + grp * CLUSTER, s_ex + grp * CLUSTER, is, il);
 
+            R fx = 0, fy = 0, fz = 0;
             R gx = 0, gy = 0, gz = 0;
             // Offset of the entry at pj from the lane's i-atom, with the FP32
             // minimum image when MI (the block is near half the box).
@@ -389,8 +405,7 @@ __global__ __launch_bounds__(64) void k_pairs(const double* __restrict__ pos, co
                     const R poly = (R)1 + x * ((R)1 + (R)0.5 * x);
                     const R c6r6 = c6 * inv_r2 * inv_r2 * inv_r2;
                     f -= (R)6 * c6r6 * inv_r2 * ((R)1 - ex * (poly + x * x * x * (R)(1.0 / 6.0)));
-                    if (ENERGY && !E64) {
-                        // The plain form's energy (the mixed form's is the FP64 pair energy).
+                    if (ENERGY) {
                         const R rc2 = (R)(P.cutoff * P.cutoff);
                         const R sc2 = sig * sig / rc2, sc6 = sc2 * sc2 * sc2;
                         const R xc = lj_a2 * rc2;
@@ -432,22 +447,7 @@ __global__ __launch_bounds__(64) void k_pairs(const double* __restrict__ pos, co
             };
             // Energy and statistics of an accepted pair (their variants only).
             auto pair_extra = [&](const int slot, const R e) {
-                if (E64) {
-                    const Q4<double> pjd = s_pd[slot];
-                    const Q2<double> sjd = s_sd[slot];
-                    double ddx = pjd.x - xid, ddy = pjd.y - yid, ddz = pjd.z - zid;
-                    if (mi) {
-                        double dd[3] = {ddx, ddy, ddz};
-                        wrap_nearest(dd, bx);
-                        ddx = dd[0];
-                        ddy = dd[1];
-                        ddz = dd[2];
-                    }
-                    eacc += pair_energy_fp64<KIND>(ddx, ddy, ddz, sid + sjd.x, eid * sjd.y, sid * sjd.x, qid * pjd.w,
-                                                   P);
-                } else if (ENERGY) {
-                    eacc += (double)e;
-                }
+                if (ENERGY) eacc += (double)e;
                 if (STATS) {
                     const int ja = s_ja[slot];
                     ++npair;
@@ -539,6 +539,7 @@ __global__ __launch_bounds__(64) void k_pairs(const double* __restrict__ pos, co
                 acc_add(fslot + P.nslots + js, (double)gy, FORCE_SCALE, status);
                 acc_add(fslot + 2 * P.nslots + js, (double)gz, FORCE_SCALE, status);
             }
+            ftot.add(fx, fy, fz);
             __syncthreads();
             e0 = e1;
             e1 = e2n;
@@ -546,20 +547,13 @@ __global__ __launch_bounds__(64) void k_pairs(const double* __restrict__ pos, co
             x1 = x2n;
             r0 = r1;
         }
-        // i-forces: the eight groups' partial sums, in a fixed order.
-        fx += dpp<DPP_XOR8>(fx);
-        fy += dpp<DPP_XOR8>(fy);
-        fz += dpp<DPP_XOR8>(fz);
-        fx += __shfl_xor(fx, 16, 64);
-        fy += __shfl_xor(fy, 16, 64);
-        fz += __shfl_xor(fz, 16, 64);
-        fx += __shfl_xor(fx, 32, 64);
-        fy += __shfl_xor(fy, 32, 64);
-        fz += __shfl_xor(fz, 32, 64);
+        // i-forces: the eight groups' sums, in a fixed order.
+        const A tx = group_sum(Force::total(ftot.x, status)), ty = group_sum(Force::total(ftot.y, status)),
+                tz = group_sum(Force::total(ftot.z, status));
         if (grp == 0 && ia >= 0) {
-            acc_add(fslot + is, (double)fx, FORCE_SCALE, status);
-            acc_add(fslot + P.nslots + is, (double)fy, FORCE_SCALE, status);
-            acc_add(fslot + 2 * P.nslots + is, (double)fz, FORCE_SCALE, status);
+            add_total(fslot + is, tx);
+            add_total(fslot + P.nslots + is, ty);
+            add_total(fslot + 2 * P.nslots + is, tz);
         }
         if (ENERGY) {
             double etot = wave_sum(eacc);
@@ -572,6 +566,132 @@ __global__ __launch_bounds__(64) void k_pairs(const double* __restrict__ pos, co
                 atomicAdd(stats + 2 * sidx, npair);
                 atomicAdd(stats + 2 * sidx + 1, hsum);
             }
+        }
+    }
+}
+
+// Pair energies of the mixed form in FP64, over the pair kernel's tasks and
+// pair set: FP64 offsets and parameters, the cutoff decided as the pair kernel
+// decides it (exactly, near the cutoff).  A kernel of its own: within the pair
+// kernel the FP64 values took its registers to one or two waves per SIMD.
+// Waves loop over tasks; each tile's sum is added in fixed point, so neither
+// the tasks' size nor their order changes the total.  Adds to one energy
+// serialise (12 ns each: one per task was 60 us at 9,000 atoms), so few waves
+// are launched and a workgroup adds once when its waves saw one system.
+// Bound: FP64 issue (about 150 instructions per step of 64 slots).  Pair forces
+// and energies together, in one kernel and now in two: 58 -> 17 us at 900 atoms,
+// 91 -> 47 at 9,000, 132 -> 104 at 23,550.
+constexpr int ENERGY_WAVES = 4;           // waves per workgroup
+constexpr int ENERGY_WORKGROUPS = 768;    // at most: three waves per SIMD of the chip
+
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+template <int KIND>
+__global__ __launch_bounds__(64 * ENERGY_WAVES) void k_pair_energy(
+    const double* __restrict__ pos, const double* __restrict__ qk, const double* __restrict__ sh,
+    const double* __restrict__ e2, const int* __restrict__ sorted_atom, const unsigned char* __restrict__ clist_ex,
+    const double* __restrict__ center, const int* __restrict__ minimg, const int2* __restrict__ clist,
+    const int* __restrict__ ccount, const int* __restrict__ tasks, const int* __restrict__ ntasks,
+    const int* __restrict__ block_sys, const SysInfo* __restrict__ sys, PairParams P, int tpt, long long* energy,
+    unsigned* status) {
+    __shared__ Q4<double> s_pw[ENERGY_WAVES][JTILE];
+    __shared__ Q2<double> s_sew[ENERGY_WAVES][JTILE];
+    __shared__ __align__(16) int s_jsw[ENERGY_WAVES][JTILE];
+    __shared__ int s_jaw[ENERGY_WAVES][JTILE];
+    __shared__ __align__(8) unsigned char s_exw[ENERGY_WAVES][JTILE];
+    __shared__ long long s_sum[ENERGY_WAVES];
+    __shared__ int s_of[ENERGY_WAVES];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    Q4<double>* s_p = s_pw[wave];
+    Q2<double>* s_se = s_sew[wave];
+    int *s_js = s_jsw[wave], *s_ja = s_jaw[wave];
+    unsigned char* s_ex = s_exw[wave];
+    const int lane = threadIdx.x & 63, grp = lane / CLUSTER, il = lane % CLUSTER;
+    const double cutoff2 = P.cutoff * P.cutoff;
+    const double rc2_lo = cutoff2 * (1.0 - 1e-12), rc2_hi = cutoff2 * (1.0 + 1e-12);
+    long long esum = 0;  // lane 0: fixed-point energy of system esys
+    int esys = -1;
+    const int total = ntasks[0];
+    for (int t = blockIdx.x * ENERGY_WAVES + wave; t < total; t += gridDim.x * ENERGY_WAVES) {
+        const int task = tasks[t], C = task >> 8, first = task & 255, I = C / CPB;
+        const int count = ccount[C];
+        const int ntile = min(tpt, (count + JTILE - 1) / JTILE - first);
+        const int sidx = block_sys[I];
+        const Box& bx = sys[sidx].box;
+        const double c0 = center[3 * I], c1 = center[3 * I + 1], c2 = center[3 * I + 2];
+        const int2* list = clist + (size_t)C * P.cap + (size_t)first * JTILE;
+        const unsigned char* list_ex = clist_ex + (size_t)C * P.cap + (size_t)first * JTILE;
+        const int nentries = count - first * JTILE, last = max(nentries - 1, 0);
+        auto entry = [&](int tl) { return list[min(tl * JTILE + lane, last)]; };
+        auto entry_ex = [&](int tl) -> unsigned { return list_ex[min(tl * JTILE + lane, last)]; };
+        const int is = C * CLUSTER + il;
+        const int ia = sorted_atom[is], ia0 = max(ia, 0);
+        int2 e0 = entry(0);
+        unsigned x0 = entry_ex(0);
+        double di[3] = {pos[3 * ia0] - c0, pos[3 * ia0 + 1] - c1, pos[3 * ia0 + 2] - c2};
+        const double qi = qk[ia0], si = sh[ia0], ei = e2[ia0];
+        if (P.periodic) wrap_nearest(di, bx);
+        const bool mi = P.periodic && minimg[I];
+        if (sidx != esys) {
+            if (lane == 0 && esys >= 0) add_total(energy + esys * E_SLOTS + E_DIRECT, esum);
+            esum = 0;
+            esys = sidx;
+        }
+        for (int k = 0; k < ntile; ++k) {
+            EntryRaw<double> r0;
+            load_entry<double>(max(e0.y, 0), pos, qk, sh, e2, r0);
+            const int2 e1 = entry(k + 1);
+            const unsigned x1 = entry_ex(k + 1);
+            const bool live = k * JTILE + lane < nentries;
+            double d[3] = {r0.x - c0, r0.y - c1, r0.z - c2};
+            if (P.periodic) wrap_nearest(d, bx);
+            s_p[lane] = {d[0], d[1], d[2], r0.q};
+            s_se[lane] = {r0.s, r0.e};
+            s_js[lane] = live && e0.y >= 0 ? e0.x : INT_MAX;
+            s_ja[lane] = e0.y;
+            s_ex[lane] = (unsigned char)x0;
+            wave_sync();
+            const unsigned present = valid_entries(s_js + grp * CLUSTER, s_ex + grp * CLUSTER, is, il);
+            const unsigned vmask = ia >= 0 ? present : 0u;
+            double eacc = 0.0;
+#pragma unroll 1
+            for (int s8 = 0; s8 < CLUSTER; ++s8) {
+                const int slot = grp * CLUSTER + s8;
+                const Q4<double> pj = s_p[slot];
+                const Q2<double> sj = s_se[slot];
+                double dd[3] = {pj.x - di[0], pj.y - di[1], pj.z - di[2]};
+                if (mi) wrap_nearest(dd, bx);
+                const double r2 = dd[0] * dd[0] + dd[1] * dd[1] + dd[2] * dd[2];
+                const bool valid = (vmask >> s8) & 1u;
+                bool in = valid && (!P.use_cutoff || r2 < rc2_lo);
+                if (valid && !in && r2 < rc2_hi)
+                    in = within_cutoff_exact(pos, ia, s_ja[slot], bx, P.periodic, cutoff2);
+                // A rejected slot is evaluated away from the singularity.
+                const double e = pair_energy_fp64<KIND>(in ? r2 : 1.0, si + sj.x, ei * sj.y, si * sj.x, qi * pj.w, P);
+                eacc += in ? e : 0.0;
+            }
+            const double et = wave_sum(eacc);
+            esum += to_fixed(et, ENERGY_SCALE, status);
+            wave_sync();
+            e0 = e1;
+            x0 = x1;
+        }
+    }
+    if (lane == 0) {
+        s_sum[wave] = esum;
+        s_of[wave] = esys;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        // Waves 0, 1, ... took the first tasks: an idle wave follows a busy one.
+        for (int w = 0; w < ENERGY_WAVES && s_of[w] >= 0;) {
+            long long sum = 0;
+            const int of = s_of[w];
+            for (; w < ENERGY_WAVES && s_of[w] == of; ++w) sum += s_sum[w];
+            add_total(energy + of * E_SLOTS + E_DIRECT, sum);
         }
     }
 }
@@ -637,10 +757,17 @@ void launch_one(const NlistDev& nl, const PairParams& p, const R* qk, const R* s
                 const ParticleDev& part, const double* pos, const SysInfo* sys_dev, A* force, A* energy,
                 unsigned* status, unsigned long long* stats, int grid, bool combine, int* const* order_out,
                 hipStream_t s) {
-    hipLaunchKernelGGL((k_pairs<R, A, ELEC, STATS, ENERGY>), dim3(grid), dim3(64), 0, s, pos, qk, sh, e2,
-                       part.qk_d.p, part.sh_d.p, part.e2_d.p, nl.sorted_atom.p, nl.clist_ex.p, nl.block_center.p,
-                       nl.block_minimg.p, nl.clist.p, nl.ccount.p, nl.tasks.p, nl.ntasks.p, nl.block_sys.p, sys_dev, p,
-                       slot_buffer<A>(nl), energy, status, stats, nl.flag.p, nl.nsys + 1);
+    constexpr bool MIXED = sizeof(R) == 4;
+    hipLaunchKernelGGL((k_pairs<R, A, ELEC, STATS, ENERGY && !MIXED>), dim3(grid), dim3(64), 0, s, pos, qk, sh, e2,
+                       nl.sorted_atom.p, nl.clist_ex.p, nl.block_center.p, nl.block_minimg.p, nl.clist.p, nl.ccount.p,
+                       nl.tasks.p, nl.ntasks.p, nl.block_sys.p, sys_dev, p, nl.tpt, slot_buffer<A>(nl), energy, status,
+                       stats, nl.flag.p, nl.nsys + 1);
+    if constexpr (ENERGY && MIXED)
+        hipLaunchKernelGGL((k_pair_energy<ELEC>), dim3(std::min((grid + ENERGY_WAVES - 1) / ENERGY_WAVES, ENERGY_WORKGROUPS)),
+                           dim3(64 * ENERGY_WAVES), 0, s, pos, part.qk_d.p,
+                           part.sh_d.p, part.e2_d.p, nl.sorted_atom.p, nl.clist_ex.p, nl.block_center.p,
+                           nl.block_minimg.p, nl.clist.p, nl.ccount.p, nl.tasks.p, nl.ntasks.p, nl.block_sys.p,
+                           sys_dev, p, nl.tpt, energy, status);
     if (combine)
         hipLaunchKernelGGL(k_slot_forces<A>, dim3((nl.nslots + 255) / 256), dim3(256), 0, s, nl.sorted_atom.p,
                            nl.nslots, slot_buffer<A>(nl), force, order_out[0], order_out[1]);

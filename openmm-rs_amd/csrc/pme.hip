@@ -1190,20 +1190,21 @@ void dft_setup(PmeDev& pm, const std::vector<SysInfo>& sys, hipStream_t s) {
             }
         }
         for (int k = 0; k < 3; ++k) {
-            pm.dft_off[prec][k].upload(off[k], s);
+            if (pm.nsys > 1) pm.dft_off[prec][k].upload(off[k], s);  // a lone system's workgroups start at 0
             pm.dft_blocks[prec][k] = off[k].back();
             pm.dft_shmem[prec][k] = lds[k] * (prec ? sizeof(double) : sizeof(float));
         }
     }
     // Dynamic LDS above 64 KB per workgroup.
-    auto allow = [](const void* f) {
-        OMM_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)PLANE_LDS_MAX));
+    auto allow = [&](const void* f, int prec, int k) {
+        if (pm.dft_shmem[prec][k] > 64 * 1024)
+            OMM_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)PLANE_LDS_MAX));
     };
-    allow((const void*)&k_dft_zy<DFT_WAVES_WIDE, float, long long>);
-    allow((const void*)&k_dft_zy<DFT_WAVES_WIDE, double, long long>);
-    allow((const void*)&k_dft_zy<DFT_WAVES_WIDE, double, double>);
-    allow((const void*)&k_dft_yz<DFT_WAVES_WIDE, float>);
-    allow((const void*)&k_dft_yz<DFT_WAVES_WIDE, double>);
+    allow((const void*)&k_dft_zy<DFT_WAVES_WIDE, float, long long>, 0, 0);
+    allow((const void*)&k_dft_zy<DFT_WAVES_WIDE, double, long long>, 1, 0);
+    allow((const void*)&k_dft_zy<DFT_WAVES_WIDE, double, double>, 1, 0);
+    allow((const void*)&k_dft_yz<DFT_WAVES_WIDE, float>, 0, 2);
+    allow((const void*)&k_dft_yz<DFT_WAVES_WIDE, double>, 1, 2);
 }
 }  // namespace
 
