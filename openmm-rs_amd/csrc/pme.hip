@@ -325,11 +325,12 @@ __global__ __launch_bounds__(ATOM_SPREAD_THREADS) void k_spread_atoms(const int*
             const int lead = __ffsll((long long)live) - 1;
             const int lsys = __shfl(si, lead, 64);
             const SysInfo& L = sys[lsys];
-            int rel[3], lo[3], ext[3];
+            int rel[3], lo[3], ext[3], org[3];
             for (int d = 0; d < 3; ++d) {
                 // Offsets from the lead atom's base point, taken in (-n/2, n/2].
                 const int n = L.grid[d];
-                int r = idx[d] - __shfl(idx[d], lead, 64);
+                org[d] = __shfl(idx[d], lead, 64);  // with every lane on: the lead need not be lane 0
+                int r = idx[d] - org[d];
                 if (r > n / 2) r -= n;
                 else if (r <= -(n - n / 2)) r += n;
                 rel[d] = r;
@@ -342,7 +343,7 @@ __global__ __launch_bounds__(ATOM_SPREAD_THREADS) void k_spread_atoms(const int*
             for (int d = 0; d < 3; ++d) s_base[d][t] = fit ? rel[d] - lo[d] : idx[d];
             if (t == 0) {
                 for (int d = 0; d < 3; ++d) {
-                    s_org[d] = wrap_index(__shfl(idx[d], lead, 64) + lo[d], L.grid[d]);
+                    s_org[d] = wrap_index(org[d] + lo[d], L.grid[d]);
                     s_ext[d] = ext[d];
                 }
                 s_lsys = lsys;

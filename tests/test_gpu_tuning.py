@@ -5,7 +5,8 @@ import numpy as np
 import pytest
 
 import ommhip
-from helpers import water
+import oracle as orc
+from helpers import force_rms_rel, water
 
 pytestmark = pytest.mark.gpu
 
@@ -151,3 +152,29 @@ def test_tuning_cache_replays_a_timed_tuning(tmp_path):
         assert len(path.read_text().splitlines()) == 2
     finally:
         ommhip.set_tuning_cache(None)
+
+
+def test_atom_owned_spread_with_uncharged_atoms():
+    # Chunks whose first atoms carry no charge (they do not spread): the oxygens
+    # of every other molecule, and whole molecules, against the tile spread and
+    # the oracle.
+    s = water(500, 2.5, seed=41)
+    p = s.nonbonded.particles
+    for m in range(500):
+        if m % 2:
+            p[3 * m] = (0.0,) + p[3 * m][1:]
+        if m % 5 == 0:
+            for k in range(3):
+                p[3 * m + k] = (0.0,) + p[3 * m + k][1:]
+    forces = []
+    for edge in (8, 0):
+        c = ommhip.Context(s, temperature=0.0, friction=0.0, step_size=1e-5)
+        c.set_launch_tuning(edge, 8, 0, 1)
+        c.set_velocities(np.zeros_like(s.positions))
+        first = c.get_state()
+        c.step(1)
+        forces.append((first["forces"], c.get_state()["velocities"]))
+    assert np.array_equal(forces[0][0], forces[1][0])
+    assert np.array_equal(forces[0][1], forces[1][1])
+    f_ref, _ = orc.water_energy_forces(s)
+    assert force_rms_rel(forces[1][0], f_ref) <= 2e-6
