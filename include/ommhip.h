@@ -158,9 +158,8 @@ omm_status omm_nb_get_ljpme_parameters(const omm_nb* nb, double* alpha, int32_t 
 /* Force::calc_forces_and_energy (nonbonded.rs:1125-1131): direct space if
  * include_direct_space, reciprocal always.  pos: host N x 3; box: host 9 or
  * NULL; forces_out: host N x 3 (overwritten, may be NULL); energy_out: kJ/mol.
- * With energy_out == NULL only forces are evaluated, on the MD step's path
- * (MIXED: FP32 pair and mesh arithmetic); with an energy requested, MIXED
- * evaluates each pair energy and the whole mesh in FP64 as well. */
+ * With energy_out == NULL no energies are evaluated.  MIXED: FP32 pair forces
+ * and an FP64 mesh either way, FP64 pair energies when one is requested. */
 omm_status omm_nb_calc_forces_and_energy(omm_nb* nb, const double* pos, const double* box,
                                          double* forces_out, double* energy_out);
 

@@ -26,7 +26,6 @@ using ommhip::guarded;
 
 struct omm_nb {
     ommhip::NbOperator op;
-    double parts[5] = {0, 0, 0, 0, 0};
     omm_nb(const omm_nb_desc* d, int precision) : op(&d, 1, precision) {}
 };
 
@@ -169,7 +168,7 @@ omm_status omm_nb_calc_forces_and_energy(omm_nb* nb, const double* pos, const do
     return guarded([&]() -> omm_status {
         if (!nb) throw Error(OMM_ERR_INVALID, "null handle");
         std::lock_guard<std::mutex> lock(nb->op.mutex);
-        nb->op.compute(pos, box, nb->op.settings().include_direct, true, forces_out, energy_out, nb->parts, nullptr,
+        nb->op.compute(pos, box, nb->op.settings().include_direct, true, forces_out, energy_out, nullptr, nullptr,
                        nullptr);
         return OMM_OK;
     });
@@ -188,7 +187,7 @@ omm_status omm_nb_calc_forces_and_energy_groups(omm_nb* nb, const double* pos, c
                      (groups & (1u << rg)) != 0;
         if (evaluated) *evaluated = (direct || recip) ? 1 : 0;
         if (!(direct || recip)) return OMM_OK;
-        nb->op.compute(pos, box, direct, recip, forces_out, energy_out, nb->parts, nullptr, nullptr);
+        nb->op.compute(pos, box, direct, recip, forces_out, energy_out, nullptr, nullptr, nullptr);
         return OMM_OK;
     });
 }
@@ -208,7 +207,7 @@ omm_status omm_nb_calc_forces_and_energy_device(omm_nb* nb, const double* d_pos,
                      (groups & (1u << rg)) != 0;
         if (evaluated) *evaluated = (direct || recip) ? 1 : 0;
         if (!(direct || recip)) return OMM_OK;
-        nb->op.compute(nullptr, box, direct, recip, nullptr, energy_out, nb->parts, nullptr, nullptr, d_pos, d_forces,
+        nb->op.compute(nullptr, box, direct, recip, nullptr, energy_out, nullptr, nullptr, nullptr, d_pos, d_forces,
                        static_cast<hipStream_t>(stream));
         return OMM_OK;
     });

@@ -173,6 +173,9 @@ struct DevBuf {
         if (count) OMM_HIP(hipMalloc(reinterpret_cast<void**>(&p), count * sizeof(T)));
         n = count;
     }
+    void alloc_at_least(size_t count) {
+        if (count > n) alloc(count);
+    }
     // Host-to-device copy ordered on stream s; returns once the copy is done,
     // so the host buffer may be released immediately.
     void upload(const T* host, size_t count, hipStream_t s) {
@@ -185,6 +188,30 @@ struct DevBuf {
     void upload(const std::vector<T>& host, hipStream_t s) { upload(host.data(), host.size(), s); }
     void download(T* host, size_t count, hipStream_t s) const {
         if (count) OMM_HIP(hipMemcpyAsync(host, p, count * sizeof(T), hipMemcpyDeviceToHost, s));
+    }
+};
+
+// Page-locked host memory that kernels read and write in place: the staging of
+// a call's inputs and results.  Held by its owner and grown on demand.
+template <class T>
+struct PinnedBuf {
+    T* p = nullptr;
+    size_t n = 0;
+    PinnedBuf() = default;
+    PinnedBuf(const PinnedBuf&) = delete;
+    PinnedBuf& operator=(const PinnedBuf&) = delete;
+    ~PinnedBuf() {
+        if (p) (void)hipHostFree(p);
+    }
+    T* at_least(size_t count) {
+        if (count > n) {
+            if (p) (void)hipHostFree(p);
+            p = nullptr;
+            n = 0;
+            OMM_HIP(hipHostMalloc(reinterpret_cast<void**>(&p), count * sizeof(T), hipHostMallocDefault));
+            n = count;
+        }
+        return p;
     }
 };
 

@@ -225,14 +225,16 @@ private:
                       const std::vector<double>& ath, const std::vector<double>& ak);
     void clear_accumulators(hipStream_t s);
     void capture_graph();
-    // Evaluates forces (all atoms, FP64 out, nullable) and the potential
-    // energy of every replica (nullable).
-    void evaluate(double* forces, double* energy, bool want_energy);
+    // Evaluates the forces, of which `count` values from `first` on are returned
+    // (in page-locked memory of this context, until its next evaluation), and the
+    // potential energy of every replica (nullable).
+    const double* evaluate(size_t first, size_t count, double* energy, bool want_energy);
     void check_status();
+    void check_status(unsigned status);
     unsigned read_status();
     void enqueue_snapshot(hipStream_t s);
     void restore_snapshot();
-    void run_steps(int count, bool graph);
+    unsigned run_steps(int count, bool graph);  // returns the run's status
     void drop_graph();
     // Sizes the neighbour list for the current positions once they are all set.
     void prepare();
@@ -247,7 +249,7 @@ private:
     double dt_ = 0.001, temperature_ = 0.0, friction_ = 0.0;
     int64_t step_count_ = 0;
     int graph_steps_ = 10;
-    DevBuf<double> pos_, vel_, inv_mass_, out_;
+    DevBuf<double> pos_, vel_, inv_mass_;
     // Positions each system's neighbour list is built from at the next
     // preparation, and which systems were set since the last one (the others
     // rebuild from the positions of their current list, which reproduces it).
@@ -263,6 +265,8 @@ private:
     DevBuf<long long> force_fx_, energy_fx_;
     DevBuf<double> force_d_, energy_d_;
     DevBuf<unsigned> status_;
+    PinnedBuf<unsigned> host_status_;  // status_ after the last run of steps
+    PinnedBuf<double> host_pos_, host_vel_, host_frc_, host_report_;
     DevBuf<unsigned long long> step_dev_, snap_step_;
     DevBuf<double> snap_pos_, snap_vel_, snap_list_;
     int64_t overflow_replays_ = 0;

@@ -4,6 +4,7 @@
 #include <cfloat>
 #include <climits>
 #include <cmath>
+#include <cstring>
 #include <functional>
 #include <random>
 #include <map>
@@ -160,9 +161,15 @@ __device__ __forceinline__ void philox4x32_10(uint32_t c[4], uint32_t k0, uint32
 // graph): advance the step counter, clear the energies.  Inside the run, step
 // k's integrator draws at counter step[0] + k + 1, so a graph needs one such
 // node rather than one per step.
+// The run's status goes to the host's copy (page-locked), which the host reads
+// once the stream is idle.
 template <class A>
-__global__ void k_step_advance(unsigned long long* step, int count, A* energy, int nslots) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) step[0] += (unsigned long long)count;
+__global__ void k_step_advance(unsigned long long* step, int count, A* energy, int nslots,
+                               const unsigned* __restrict__ status, unsigned* status_host) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        step[0] += (unsigned long long)count;
+        *status_host = *status;
+    }
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < nslots; i += gridDim.x * blockDim.x) energy[i] = (A)0;
 }
 
@@ -184,6 +191,29 @@ __global__ void k_snapshot(const double* __restrict__ pos, double* __restrict__ 
 
 inline __device__ double force_value(long long f) { return (double)f * (1.0 / FORCE_SCALE); }
 inline __device__ double force_value(double f) { return f; }
+inline __device__ double energy_value(long long e) { return (double)e * (1.0 / ENERGY_SCALE); }
+inline __device__ double energy_value(double e) { return e; }
+
+// Last kernel of an evaluation: the count force values from `first` on to `out`
+// (page-locked host memory), the report (status, E_SLOTS energies and the volume of every
+// system) likewise, and the accumulators cleared for the next step.
+template <class A>
+__global__ void k_evaluation_out(size_t n3, A* force, double* out, size_t first, size_t count, A* energy, int nsys,
+                                 const SysInfo* __restrict__ sys, const unsigned* __restrict__ status,
+                                 double* report) {
+    const size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
+    if (i < n3) {
+        if (i - first < count) out[i - first] = force_value(force[i]);
+        force[i] = (A)0;
+    }
+    for (size_t k = i; k < (size_t)nsys * E_SLOTS; k += gridDim.x * (size_t)blockDim.x) {
+        report[1 + k] = energy_value(energy[k]);
+        energy[k] = (A)0;
+    }
+    for (size_t k = i; k < (size_t)nsys; k += gridDim.x * (size_t)blockDim.x)
+        report[1 + (size_t)nsys * E_SLOTS + k] = sys[k].box.volume;
+    if (i == 0) report[0] = (double)*status;
+}
 
 // The three standard normals of atom i (global index) at the current step:
 // Philox keyed by the system's seed, counter (index within the system,
@@ -808,8 +838,6 @@ __global__ void k_baro_scale(int nmol, const int* __restrict__ mol_start, const 
     }
 }
 
-inline __device__ double energy_value(long long e) { return (double)e * (1.0 / ENERGY_SCALE); }
-inline __device__ double energy_value(double e) { return e; }
 
 // Potential energy of one system from its energy slots plus the volume terms.
 template <class A>
@@ -1026,8 +1054,8 @@ MdContext::MdContext(const omm_md_desc* descs, int nsys, int precision) {
         force_d_.alloc(3 * (size_t)n_);
         energy_d_.alloc(eslots);
     }
-    out_.alloc(3 * (size_t)n_);
     status_.alloc(1);
+    *host_status_.at_least(1) = 0u;
     fill_async<unsigned>(status_.p, 1, 0u, s_);
     step_dev_.alloc(1);
     fill_async<unsigned long long>(step_dev_.p, 1, 0ull, s_);
@@ -1150,10 +1178,12 @@ void MdContext::capacity(int* list_cap, int* bin_cap, int64_t* replays) {
 void MdContext::list_positions(int r, double* out) {
     if (r < 0 || r >= nsys_) throw Error(OMM_ERR_INVALID, "replica index out of range");
     prepare();
-    const size_t off3 = 3 * (size_t)nb_->atom_offset(r), bytes = 3 * (size_t)nb_->num_particles(r) * sizeof(double);
+    const size_t off3 = 3 * (size_t)nb_->atom_offset(r), n3 = 3 * (size_t)nb_->num_particles(r);
     const double* built = nb_->settings().include_direct ? nb_->pos_build() : nullptr;
-    OMM_HIP(hipMemcpyAsync(out, (built ? built : pos_.p) + off3, bytes, hipMemcpyDeviceToHost, s_));
+    double* p = host_pos_.at_least(n3);
+    launch_copy_out((built ? built : pos_.p) + off3, p, n3, s_);
     OMM_HIP(hipStreamSynchronize(s_));
+    std::memcpy(out, p, n3 * sizeof(double));
 }
 
 void MdContext::set_tuning(const NbOperator::Tuning& t) {
@@ -1596,7 +1626,7 @@ void MdContext::energies_at(const std::vector<double>& transforms, const std::ve
         OMM_HIP(hipStreamSynchronize(s_));
     };
     try {
-        evaluate(nullptr, energies, true);
+        evaluate(0, 0, energies, true);
     } catch (...) {
         restore();
         throw;
@@ -1804,10 +1834,10 @@ void MdContext::enqueue_step(hipStream_t s, int rebuild, bool barostat, int offs
         const int eb = std::min(64, (eslots + 255) / 256);
         if (mixed_)
             hipLaunchKernelGGL(k_step_advance<long long>, dim3(eb), dim3(256), 0, s, step_dev_.p, advance,
-                               energy_fx_.p, eslots);
+                               energy_fx_.p, eslots, status_.p, host_status_.p);
         else
             hipLaunchKernelGGL(k_step_advance<double>, dim3(eb), dim3(256), 0, s, step_dev_.p, advance, energy_d_.p,
-                               eslots);
+                               eslots, status_.p, host_status_.p);
     }
     OMM_HIP(hipGetLastError());
 }
@@ -1996,8 +2026,9 @@ unsigned MdContext::read_status() {
     return st;
 }
 
-void MdContext::check_status() {
-    const unsigned st = read_status();
+void MdContext::check_status() { check_status(read_status()); }
+
+void MdContext::check_status(unsigned st) {
     if (st & (ST_LIST_OVERFLOW | ST_BIN_OVERFLOW)) {
         fill_async<unsigned>(status_.p, 1, 0u, s_);
         throw Error(OMM_ERR_OVERFLOW, "neighbour list or PME bin capacity exceeded during the step");
@@ -2101,7 +2132,7 @@ void MdContext::set_integrator(double temperature, double friction, double step_
 // overflow during them restores the snapshot, grows the storage, rebuilds the
 // lists the snapshot had and replays the steps eagerly: the trajectory is that
 // of a run that never overflowed (the noise is counter-based).
-void MdContext::run_steps(int count, bool graph) {
+unsigned MdContext::run_steps(int count, bool graph) {
     TraceRange range(graph ? "omm.graph_steps" : "omm.eager_steps");
     BaroDev& B = baro_;
     const int phase0 = B.phase;
@@ -2120,9 +2151,10 @@ void MdContext::run_steps(int count, bool graph) {
         enqueue_snapshot(s_);
         eager();
     }
-    unsigned st = read_status();
+    OMM_HIP(hipStreamSynchronize(s_));
+    unsigned st = *host_status_.p;  // written by the run's last kernel
     for (int attempt = 0; st & (ST_LIST_OVERFLOW | ST_BIN_OVERFLOW | ST_VBOX); ++attempt) {
-        if (attempt == 8) check_status();  // throws
+        if (attempt == 8) check_status(st);  // throws
         TraceRange replay("omm.overflow_replay");
         ++overflow_replays_;
         drop_graph();
@@ -2138,8 +2170,10 @@ void MdContext::run_steps(int count, bool graph) {
         restore_snapshot();
         B.phase = phase0;
         eager();
-        st = read_status();
+        OMM_HIP(hipStreamSynchronize(s_));
+        st = *host_status_.p;
     }
+    return st;
 }
 
 void MdContext::step(int nsteps) {
@@ -2151,6 +2185,7 @@ void MdContext::step(int nsteps) {
     const bool graphs = mixed_ && graph_steps_ > 0 && len > 0;
     const int chunk = graph_steps_ > 0 ? graph_steps_ : 10;  // eager steps per snapshot
     int done = 0;
+    unsigned st = 0;
     while (done < nsteps) {
         const int left = nsteps - done;
         // A period graph starts at an attempt boundary; an attempt-free graph
@@ -2168,20 +2203,33 @@ void MdContext::step(int nsteps) {
         } else {
             k = std::min(left, graphs ? len : chunk);
         }
-        run_steps(k, g);
+        st = run_steps(k, g);
         done += k;
     }
     step_count_ += nsteps;
-    check_status();
+    check_status(nsteps > 0 ? st : read_status());
 }
 
-void MdContext::evaluate(double* forces, double* energy, bool want_energy) {
+const double* MdContext::evaluate(size_t first, size_t count, double* energy, bool want_energy) {
     TraceRange range("omm.evaluate");
     prepare();
+    const size_t n3 = 3 * (size_t)n_, eslots = (size_t)E_SLOTS * nsys_;
+    double* out = count ? host_frc_.at_least(count) : nullptr;
+    double* report = host_report_.at_least(1 + eslots + nsys_);
+    unsigned st = 0;
+    clear_accumulators(s_);
     for (int attempt = 0;; ++attempt) {
-        clear_accumulators(s_);
         enqueue_forces(s_, want_energy, NbOperator::REBUILD_FLAG);
-        const unsigned st = read_status();
+        const dim3 wgs((unsigned)((n3 + 255) / 256));
+        if (mixed_)
+            hipLaunchKernelGGL(k_evaluation_out<long long>, wgs, dim3(256), 0, s_, n3, force_fx_.p, out, first,
+                               count, energy_fx_.p, nsys_, nb_->systems_dev(), status_.p, report);
+        else
+            hipLaunchKernelGGL(k_evaluation_out<double>, wgs, dim3(256), 0, s_, n3, force_d_.p, out, first,
+                               count, energy_d_.p, nsys_, nb_->systems_dev(), status_.p, report);
+        OMM_HIP(hipGetLastError());
+        OMM_HIP(hipStreamSynchronize(s_));
+        st = (unsigned)report[0];
         if (!(st & (ST_LIST_OVERFLOW | ST_BIN_OVERFLOW)) || attempt == 4) break;
         if (attempt == 3)
             throw Error(OMM_ERR_OVERFLOW, "evaluation kept overflowing (status " + std::to_string(st) + ")");
@@ -2190,44 +2238,25 @@ void MdContext::evaluate(double* forces, double* energy, bool want_energy) {
         nb_->force_rebuild(s_);
         drop_graph();
     }
-    const size_t eslots = (size_t)E_SLOTS * nsys_;
-    std::vector<double> e(eslots);
-    if (mixed_) {
-        std::vector<long long> efx(eslots);
-        energy_fx_.download(efx.data(), eslots, s_);
-        if (forces) {
-            launch_fixed_to_double(force_fx_.p, out_.p, 3 * (size_t)n_, s_);
-            out_.download(forces, 3 * (size_t)n_, s_);
-        }
-        OMM_HIP(hipStreamSynchronize(s_));
-        for (size_t k = 0; k < eslots; ++k) e[k] = (double)efx[k] * (1.0 / ENERGY_SCALE);
-    } else {
-        energy_d_.download(e.data(), eslots, s_);
-        if (forces) force_d_.download(forces, 3 * (size_t)n_, s_);
-        OMM_HIP(hipStreamSynchronize(s_));
-    }
-    clear_accumulators(s_);  // the step expects a zero force accumulator
-    check_status();
+    check_status(st);
     if (energy) {
         const NbSettings& c = nb_->settings();
-        std::vector<SysInfo> sys(nsys_);
-        OMM_HIP(hipMemcpyAsync(sys.data(), nb_->systems_dev(), nsys_ * sizeof(SysInfo), hipMemcpyDeviceToHost, s_));
-        OMM_HIP(hipStreamSynchronize(s_));
         for (int r = 0; r < nsys_; ++r) {
-            const double* er = e.data() + (size_t)E_SLOTS * r;
-            HostTerms ht = nb_->host_terms(r, sys[r].box.volume, c.include_direct, true);
+            const double* er = report + 1 + (size_t)E_SLOTS * r;
+            HostTerms ht = nb_->host_terms(r, report[1 + eslots + r], c.include_direct, true);
             energy[r] = er[E_DIRECT] + er[E_RECIP] + ht.self + ht.dispersion + er[E_EXCEPT] + er[E_BOND] + er[E_ANGLE];
         }
     }
+    return out;
 }
 
-void MdContext::energies(double* out) { evaluate(nullptr, out, true); }
+void MdContext::energies(double* out) { evaluate(0, 0, out, true); }
 
 void MdContext::set_velocities_to_temperature(double temperature, uint64_t seed) {
     // context.rs:182-223
     if (!(std::isfinite(temperature) && temperature >= 0.0))
         throw Error(OMM_ERR_INVALID, "temperature must be nonnegative and finite");
-    std::vector<double> v(3 * (size_t)n_), f(3 * (size_t)n_);
+    std::vector<double> v(3 * (size_t)n_);
     for (int r = 0; r < nsys_; ++r) {
         std::mt19937_64 rng(seed + (uint64_t)r);
         std::normal_distribution<double> normal(0.0, 1.0);
@@ -2237,7 +2266,7 @@ void MdContext::set_velocities_to_temperature(double temperature, uint64_t seed)
             for (int a = 0; a < 3; ++a) v[3 * (size_t)i + a] = normal(rng) * scale;
         }
     }
-    evaluate(f.data(), nullptr, false);
+    const double* f = evaluate(0, 3 * (size_t)n_, nullptr, false);
     double offset = 0.5 * dt_;  // LangevinMiddle velocity_time_offset (langevin.rs:204-206)
     for (int i = 0; i < n_; ++i) {
         double im = masses_[i] == 0.0 ? 0.0 : 1.0 / masses_[i];
@@ -2249,15 +2278,21 @@ void MdContext::set_velocities_to_temperature(double temperature, uint64_t seed)
 void MdContext::get_state(int r, double* pos, double* vel, double* forces, double* energy, int64_t* step) {
     if (r < 0 || r >= nsys_) throw Error(OMM_ERR_INVALID, "replica index out of range");
     const size_t off3 = 3 * (size_t)nb_->atom_offset(r), n3 = 3 * (size_t)nb_->num_particles(r);
+    // Everything leaves through page-locked memory under one synchronisation.
+    double* p = pos ? host_pos_.at_least(n3) : nullptr;
+    double* v = vel ? host_vel_.at_least(n3) : nullptr;
+    if (p) launch_copy_out(pos_.p + off3, p, n3, s_);
+    if (v) launch_copy_out(vel_.p + off3, v, n3, s_);
     if (forces || energy) {
-        std::vector<double> f(forces ? 3 * (size_t)n_ : 0), e(nsys_);
-        evaluate(forces ? f.data() : nullptr, energy ? e.data() : nullptr, energy != nullptr);
-        if (forces) std::copy(f.begin() + off3, f.begin() + off3 + n3, forces);
+        std::vector<double> e(nsys_);
+        const double* f = evaluate(off3, forces ? n3 : 0, energy ? e.data() : nullptr, energy != nullptr);
+        if (forces) std::memcpy(forces, f, n3 * sizeof(double));
         if (energy) *energy = e[r];
+    } else {
+        OMM_HIP(hipStreamSynchronize(s_));
     }
-    if (pos) OMM_HIP(hipMemcpyAsync(pos, pos_.p + off3, n3 * sizeof(double), hipMemcpyDeviceToHost, s_));
-    if (vel) OMM_HIP(hipMemcpyAsync(vel, vel_.p + off3, n3 * sizeof(double), hipMemcpyDeviceToHost, s_));
-    OMM_HIP(hipStreamSynchronize(s_));
+    if (p) std::memcpy(pos, p, n3 * sizeof(double));
+    if (v) std::memcpy(vel, v, n3 * sizeof(double));
     if (step) *step = step_count_;
 }
 

@@ -70,6 +70,16 @@ struct HostTerms {
 // OMMHIP_TUNING_CACHE environment variable.
 void set_tuning_cache_path(const char* path);
 
+// What an evaluation reports to the host, written by its last kernel.
+struct EvalResult {
+    unsigned status = 0;
+    double energy[E_SLOTS] = {};
+    unsigned long long stats[2] = {};
+};
+
+// Copies count doubles to page-locked host memory (a kernel, in stream order).
+void launch_copy_out(const double* src, double* host, size_t count, hipStream_t s);
+
 class NbOperator {
 public:
     // A batch of nsys systems.  Method, cutoff, tolerance, dielectric,
@@ -311,18 +321,18 @@ private:
 
     // Host-API scratch.
     DevBuf<double> pos_dev_;
-    DevBuf<double> mesh_q_, mesh_out_;  // mesh_charges: charges, potentials
+    DevBuf<double> mesh_q_;  // mesh_charges: charges
     DevBuf<int> mesh_atoms_;
     DevBuf<long long> force_fx_, energy_fx_;
     DevBuf<double> force_d_, energy_d_;
     DevBuf<unsigned> status_;
     DevBuf<unsigned long long> stats_;
-    DevBuf<double> out_forces_;
+    PinnedBuf<double> host_in_, host_out_;  // staged positions (and charges), forces
+    PinnedBuf<int> host_idx_;
+    PinnedBuf<EvalResult> host_res_;
     Box last_box_{};
     bool have_box_ = false;
 };
 
-// Converts int64 fixed-point forces to FP64 (n3 values).
-void launch_fixed_to_double(const long long* fx, double* out, size_t n3, hipStream_t s);
 
 }  // namespace ommhip

@@ -19,9 +19,93 @@ constexpr double LIST_SKIN = 0.13;
 
 namespace {
 
-__global__ void k_fixed_to_double(const long long* __restrict__ fx, double* __restrict__ out, size_t n3) {
-    size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
-    if (i < n3) out[i] = (double)fx[i] * (1.0 / FORCE_SCALE);
+// First kernel of an evaluation, 256 atoms per workgroup: positions taken from
+// `src` (page-locked host memory, the caller's device array, or `pos` itself on a
+// retry), accumulators cleared, and the list's displacement check
+// (pos_build nullable: none; force_all: a rebuild whatever the check says).
+// One launch for the upload, five fills and the check, which were nine
+// launches and a synchronisation.
+constexpr int EVAL_WG = 256;
+template <class A>
+__global__ __launch_bounds__(EVAL_WG) void k_eval_begin(int n, const double* src, double* pos,
+                                                        const double* __restrict__ pos_build, A* force, A* energy,
+                                                        unsigned* status, unsigned long long* stats, double lim2,
+                                                        int force_all, int* flag) {
+    __shared__ double s_x[3 * EVAL_WG];
+    const int first = blockIdx.x * EVAL_WG, cnt = min(EVAL_WG, n - first);
+    const size_t base = 3 * (size_t)first;
+    for (int k = threadIdx.x; k < 3 * cnt; k += EVAL_WG) {
+        const double v = src[base + k];
+        s_x[k] = v;
+        pos[base + k] = v;
+        force[base + k] = (A)0;
+    }
+    if (blockIdx.x == 0) {
+        if (threadIdx.x < E_SLOTS) energy[threadIdx.x] = (A)0;
+        if (threadIdx.x < 2) stats[threadIdx.x] = 0ull;
+        if (threadIdx.x == 0) *status = 0u;
+        if (force_all && threadIdx.x < 2) flag[threadIdx.x] = 1;
+    }
+    if (!pos_build) return;
+    __syncthreads();
+    bool moved = false;
+    if ((int)threadIdx.x < cnt) {
+        const double *x = s_x + 3 * threadIdx.x, *b = pos_build + base + 3 * threadIdx.x;
+        moved = !(skin_d2(x[0] - b[0], x[1] - b[1], x[2] - b[2]) <= lim2);  // NaN also requests a rebuild
+    }
+    wave_raise_flags(flag, moved, 0);
+}
+
+__device__ __forceinline__ double force_out(long long v) { return (double)v * (1.0 / FORCE_SCALE); }
+__device__ __forceinline__ double force_out(double v) { return v; }
+__device__ __forceinline__ double energy_out(long long v) { return (double)v * (1.0 / ENERGY_SCALE); }
+__device__ __forceinline__ double energy_out(double v) { return v; }
+
+// Last kernel of an evaluation: forces to `out` (the caller's device array or
+// page-locked host memory, nullable; left alone when the status reports an
+// error), status, energies and statistics to the host's record.
+template <class A>
+__global__ void k_eval_end(size_t n3, const A* __restrict__ force, double* __restrict__ out,
+                           const A* __restrict__ energy, const unsigned* __restrict__ status,
+                           const unsigned long long* __restrict__ stats, EvalResult* res) {
+    const size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
+    if (out && i < n3 && *status == 0u) out[i] = force_out(force[i]);
+    if (blockIdx.x == 0) {
+        if (threadIdx.x < E_SLOTS) res->energy[threadIdx.x] = energy_out(energy[threadIdx.x]);
+        if (stats && threadIdx.x < 2) res->stats[threadIdx.x] = stats[threadIdx.x];
+        if (threadIdx.x == 0) res->status = *status;
+    }
+}
+
+__global__ void k_copy_out(const double* __restrict__ src, double* __restrict__ dst, size_t n) {
+    const size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
+    if (i < n) dst[i] = src[i];
+}
+
+// Charge mesh inputs from page-locked host memory (positions, then charges).
+__global__ void k_mesh_begin(int n, const double* __restrict__ src, double* pos, double* q, double* force,
+                             double* energy, unsigned* status) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < 3 * n) {
+        pos[i] = src[i];
+        force[i] = 0.0;
+    }
+    if (i < n) q[i] = src[3 * (size_t)n + i];
+    if (i < E_SLOTS) energy[i] = 0.0;
+    if (i == 0) *status = 0u;
+}
+
+// Copies finite values; false when one is not.
+bool copy_finite(const double* src, double* dst, size_t n) {
+    uint64_t worst = 0;
+    for (size_t i = 0; i < n; ++i) {
+        uint64_t u;
+        std::memcpy(&u, src + i, 8);
+        const uint64_t e = u & 0x7ff0000000000000ull;
+        worst = worst > e ? worst : e;
+        dst[i] = src[i];
+    }
+    return worst != 0x7ff0000000000000ull;
 }
 
 void validate_particle(double q, double s, double e) {
@@ -70,9 +154,9 @@ Box make_box(const double* v) {
     return b;
 }
 
-void launch_fixed_to_double(const long long* fx, double* out, size_t n3, hipStream_t s) {
-    if (!n3) return;
-    hipLaunchKernelGGL(k_fixed_to_double, dim3((unsigned)((n3 + 255) / 256)), dim3(256), 0, s, fx, out, n3);
+void launch_copy_out(const double* src, double* host, size_t count, hipStream_t s) {
+    if (!count) return;
+    hipLaunchKernelGGL(k_copy_out, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, s, src, host, count);
     OMM_HIP(hipGetLastError());
 }
 
@@ -463,7 +547,6 @@ void NbOperator::setup_device(const std::vector<Box>& boxes) {
         }
         status_.alloc(1);
         stats_.alloc(2);
-        out_forces_.alloc(3 * (size_t)N);
     }
     OMM_HIP(hipStreamSynchronize(s));
     have_box_ = false;
@@ -1223,8 +1306,9 @@ double NbOperator::mesh_charges(const double* pos, const double* box, double alp
         if (!std::isfinite(charges[i])) throw Error(OMM_ERR_NONFINITE, "charges must be finite");
         qmax = std::max(qmax, std::fabs(charges[i]));
     }
-    for (int i = 0; i < 3 * n; ++i)
-        if (!std::isfinite(pos[i])) throw Error(OMM_ERR_NONFINITE, "particle positions must be finite");
+    double* in = host_in_.at_least(4 * (size_t)n);
+    if (!copy_finite(pos, in, 3 * (size_t)n)) throw Error(OMM_ERR_NONFINITE, "particle positions must be finite");
+    std::memcpy(in + 3 * (size_t)n, charges, (size_t)n * sizeof(double));
     for (int k = 0; k < count; ++k)
         if (atoms[k] < 0 || atoms[k] >= n) throw Error(OMM_ERR_INVALID, "particle index out of range");
     hipStream_t s = stream_;
@@ -1236,20 +1320,31 @@ double NbOperator::mesh_charges(const double* pos, const double* box, double alp
         last_box_ = b;
         have_box_ = true;
     }
-    pos_dev_.upload(pos, 3 * (size_t)n, s);
-    mesh_q_.upload(charges, (size_t)n, s);
+    mesh_q_.alloc((size_t)n);
+    if (count > 0) {
+        mesh_atoms_.alloc_at_least((size_t)count);
+        std::memcpy(host_idx_.at_least((size_t)count), atoms, (size_t)count * sizeof(int));
+        OMM_HIP(hipMemcpyAsync(mesh_atoms_.p, host_idx_.p, (size_t)count * sizeof(int), hipMemcpyHostToDevice, s));
+    }
     const double saved_max = pme_.max_charge;
     pme_.max_charge = qmax;  // selects the spread's staging; the FP64 grid is exact either way
     const int phases = count > 0 ? (PME_SPREAD | PME_FFT) : PME_ALL;
+    double* out = host_out_.at_least(std::max(3 * (size_t)n, (size_t)count));
+    EvalResult* res = host_res_.at_least(1);
     unsigned st = 0;
     for (int attempt = 0; attempt < 8; ++attempt) {
-        fill_async<unsigned>(status_.p, 1, 0u, s);
-        fill_async<double>(force_d_.p, 3 * (size_t)n, 0.0, s);
-        fill_async<double>(energy_d_.p, E_SLOTS, 0.0, s);
+        hipLaunchKernelGGL(k_mesh_begin, dim3((3 * n + 255) / 256), dim3(256), 0, s, n, in, pos_dev_.p, mesh_q_.p,
+                           force_d_.p, energy_d_.p, status_.p);
         pme_run(pme_, MESH_F64, nl_, pos_dev_.p, mesh_q_.p, sys_dev_.p, nullptr, force_d_.p, nullptr, energy_d_.p,
                 status_.p, s, phases);
-        status_.download(&st, 1, s);
+        // The potentials or the forces go straight to page-locked memory.
+        if (count > 0) pme_potential_at(pme_, sys_dev_.p, pos_dev_.p, mesh_atoms_.p, count, out, s);
+        const size_t n3 = count > 0 ? 0 : 3 * (size_t)n;
+        hipLaunchKernelGGL(k_eval_end<double>, dim3((unsigned)std::max<size_t>(1, (n3 + 255) / 256)), dim3(256), 0, s,
+                           n3, force_d_.p, forces ? out : nullptr, energy_d_.p, status_.p, nullptr, res);
+        OMM_HIP(hipGetLastError());
         OMM_HIP(hipStreamSynchronize(s));
+        st = res->status;
         if (!(st & ST_BIN_OVERFLOW)) break;
         grow(st);
     }
@@ -1257,22 +1352,12 @@ double NbOperator::mesh_charges(const double* pos, const double* box, double alp
     if (st & ST_BIN_OVERFLOW) throw Error(OMM_ERR_OVERFLOW, "PME spread bins kept overflowing");
     if (st & ST_NONFINITE) throw Error(OMM_ERR_NONFINITE, "non-finite mesh result");
     if (count > 0) {
-        mesh_atoms_.upload(atoms, (size_t)count, s);
-        mesh_out_.alloc((size_t)count);
-        pme_potential_at(pme_, sys_dev_.p, pos_dev_.p, mesh_atoms_.p, count, mesh_out_.p, s);
-        std::vector<double> pot(count);
-        mesh_out_.download(pot.data(), (size_t)count, s);
-        OMM_HIP(hipStreamSynchronize(s));
-        for (int k = 0; k < count; ++k) derivatives[k] += pot[k];
+        for (int k = 0; k < count; ++k) derivatives[k] += out[k];
         return 0.0;
     }
-    double e[E_SLOTS];
-    energy_d_.download(e, E_SLOTS, s);
-    std::vector<double> f(forces ? 3 * (size_t)n : 0);
-    if (forces) force_d_.download(f.data(), 3 * (size_t)n, s);
-    OMM_HIP(hipStreamSynchronize(s));
-    for (size_t i = 0; i < f.size(); ++i) forces[i] += f[i];
-    return e[E_RECIP];
+    if (forces)
+        for (size_t i = 0; i < 3 * (size_t)n; ++i) forces[i] += out[i];
+    return res->energy[E_RECIP];
 }
 
 void NbOperator::set_box(int s, const double* box9, hipStream_t st) {
@@ -1459,9 +1544,8 @@ void NbOperator::compute(const double* pos, const double* box, bool direct, bool
         OMM_HIP(hipStreamSynchronize(caller));
         pos = host_pos.data();
     }
-    if (pos)
-        for (int i = 0; i < 3 * n; ++i)
-            if (!std::isfinite(pos[i])) throw Error(OMM_ERR_NONFINITE, "particle positions must be finite");
+    if (pos && !copy_finite(pos, host_in_.at_least(3 * (size_t)std::max(n, 1)), 3 * (size_t)n))
+        throw Error(OMM_ERR_NONFINITE, "particle positions must be finite");
     Box b{};
     bool vchanged = false;
     if (n > 0 && virtual_) {
@@ -1491,73 +1575,78 @@ void NbOperator::compute(const double* pos, const double* box, bool direct, bool
         // once the results are complete, as the host form does.
         OMM_HIP(hipEventRecord(ev_caller_, caller));
         OMM_HIP(hipStreamWaitEvent(s, ev_caller_, 0));
-        OMM_HIP(hipMemcpyAsync(pos_dev_.p, pos_dev_in, 3 * (size_t)n * sizeof(double), hipMemcpyDeviceToDevice, s));
-    } else {
-        pos_dev_.upload(pos, 3 * (size_t)n, s);
     }
     const bool want_stats = num_pairs || pair_hash;
     // Pair statistics are gathered by a force-only pass; energies by the
-    // energy pass (FP64 pair energies and FP64 mesh in the mixed form).
+    // energy pass (FP64 pair energies).  The mesh runs in FP64 either way.
     const bool want_energy = !want_stats && (energy || parts);
+    const int mode = mesh_mode(!want_stats);
     const NbSettings& c = cfg_[0];
+    const size_t n3 = 3 * (size_t)n;
+    double* out = forces_dev_out ? forces_dev_out : (forces ? host_out_.at_least(n3) : nullptr);
+    EvalResult* res = host_res_.at_least(1);
+    const double lim = 0.5 * nl_.skin;
     for (int attempt = 0; attempt < 6; ++attempt) {
-        fill_async<unsigned>(status_.p, 1, 0u, s);
-        if (want_stats) fill_async<unsigned long long>(stats_.p, 2, 0ull, s);
-        if (mixed_) {
-            fill_async<long long>(force_fx_.p, 3 * (size_t)n, 0ll, s);
-            fill_async<long long>(energy_fx_.p, E_SLOTS, 0ll, s);
-        } else {
-            fill_async<double>(force_d_.p, 3 * (size_t)n, 0.0, s);
-            fill_async<double>(energy_d_.p, E_SLOTS, 0.0, s);
+        const double* src = attempt > 0 ? pos_dev_.p : (pos_dev_in ? pos_dev_in : host_in_.p);
+        const double* built = direct ? nl_.pos_build.p : nullptr;
+        const int rebuild = direct && (box_changed || attempt > 0) ? 1 : 0;
+        const dim3 wgs((n + EVAL_WG - 1) / EVAL_WG);
+        if (mixed_)
+            hipLaunchKernelGGL(k_eval_begin<long long>, wgs, dim3(EVAL_WG), 0, s, n, src, pos_dev_.p, built,
+                               force_fx_.p, energy_fx_.p, status_.p, stats_.p, lim * lim, rebuild, nl_.flag.p);
+        else
+            hipLaunchKernelGGL(k_eval_begin<double>, wgs, dim3(EVAL_WG), 0, s, n, src, pos_dev_.p, built, force_d_.p,
+                               energy_d_.p, status_.p, stats_.p, lim * lim, rebuild, nl_.flag.p);
+        OMM_HIP(hipGetLastError());
+        if (direct) nlist_build(nl_, pos_dev_.p, sys_dev_.p, status_.p, s);
+        // The reciprocal space runs on the side stream beside the pairs, after
+        // the build: a call's conformation may be unrelated to the last one's,
+        // whose order would not be a spatial one here.
+        const bool beside = direct && recip && c.screened();
+        hipStream_t rs = beside ? side_ : s;
+        if (beside) {
+            OMM_HIP(hipEventRecord(ev_fork_, s));
+            OMM_HIP(hipStreamWaitEvent(side_, ev_fork_, 0));
         }
+        if (recip && c.pme_mesh())
+            pme_run(pme_, mode, nl_, pos_dev_.p, part_.charge.p, sys_dev_.p, force_fx_.p, force_d_.p, energy_fx_.p,
+                    energy_d_.p, status_.p, rs);
+        if (recip && ljpme())
+            lj_mesh(mode, pos_dev_.p, force_fx_.p, force_d_.p, energy_fx_.p, energy_d_.p, status_.p, rs);
+        if (recip && c.method == OMM_NB_EWALD)
+            ewald_run(ewald_, pos_dev_.p, part_.charge.p, sys_dev_.p, alpha_[0], force_fx_.p, force_d_.p,
+                      energy_fx_.p, energy_d_.p, status_.p, mixed_, rs);
+        if (beside) OMM_HIP(hipEventRecord(ev_join_, side_));
         if (direct) {
-            nlist_check(nl_, pos_dev_.p, (box_changed || attempt > 0) ? 1 : 0, s);
-            nlist_build(nl_, pos_dev_.p, sys_dev_.p, status_.p, s);
             launch_pairs(mixed_, want_energy, nl_, pp_, part_, pos_dev_.p, sys_dev_.p, force_fx_.p, force_d_.p,
                          energy_fx_.p, energy_d_.p, status_.p, want_stats ? stats_.p : nullptr, pair_grid_, s);
             launch_exceptions(mixed_, exc_, part_, pos_dev_.p, sys_dev_.p, c.exceptions_pbc ? 1 : 0,
                               c.screened() ? 1 : 0, alpha_[0], ljpme() ? lj_alpha_[0] : 0.0, force_fx_.p,
                               force_d_.p, energy_fx_.p, energy_d_.p, status_.p, s);
         }
-        if (recip && c.pme_mesh())
-            pme_run(pme_, mesh_mode(want_energy), nl_, pos_dev_.p, part_.charge.p, sys_dev_.p, force_fx_.p,
-                    force_d_.p, energy_fx_.p, energy_d_.p, status_.p, s);
-        if (recip && ljpme())
-            lj_mesh(mesh_mode(want_energy), pos_dev_.p, force_fx_.p, force_d_.p, energy_fx_.p, energy_d_.p, status_.p, s);
-        if (recip && c.method == OMM_NB_EWALD)
-            ewald_run(ewald_, pos_dev_.p, part_.charge.p, sys_dev_.p, alpha_[0], force_fx_.p, force_d_.p,
-                      energy_fx_.p, energy_d_.p, status_.p, mixed_, s);
-        unsigned st = 0;
-        status_.download(&st, 1, s);
+        if (beside) OMM_HIP(hipStreamWaitEvent(s, ev_join_, 0));
+        const size_t nout = out ? n3 : 0;
+        const dim3 ends((unsigned)std::max<size_t>(1, (nout + 255) / 256));
+        if (mixed_)
+            hipLaunchKernelGGL(k_eval_end<long long>, ends, dim3(256), 0, s, nout, force_fx_.p, out, energy_fx_.p,
+                               status_.p, stats_.p, res);
+        else
+            hipLaunchKernelGGL(k_eval_end<double>, ends, dim3(256), 0, s, nout, force_d_.p, out, energy_d_.p,
+                               status_.p, stats_.p, res);
+        OMM_HIP(hipGetLastError());
         OMM_HIP(hipStreamSynchronize(s));
+        const unsigned st = res->status;
         if (st & (ST_LIST_OVERFLOW | ST_BIN_OVERFLOW)) {
             grow(st);
             continue;
         }
         if (st & ST_NONFINITE) throw Error(OMM_ERR_NONFINITE, "non-finite force or energy on the device");
         if (st & ST_OVERFLOW) throw Error(OMM_ERR_OVERFLOW, "fixed-point force/energy accumulator overflow");
-        double e[E_SLOTS];
-        if (mixed_) {
-            long long efx[E_SLOTS];
-            energy_fx_.download(efx, E_SLOTS, s);
-            launch_fixed_to_double(force_fx_.p, forces_dev_out ? forces_dev_out : out_forces_.p, 3 * (size_t)n, s);
-            if (forces) out_forces_.download(forces, 3 * (size_t)n, s);
-            OMM_HIP(hipStreamSynchronize(s));
-            for (int k = 0; k < E_SLOTS; ++k) e[k] = (double)efx[k] * (1.0 / ENERGY_SCALE);
-        } else {
-            energy_d_.download(e, E_SLOTS, s);
-            if (forces) force_d_.download(forces, 3 * (size_t)n, s);
-            if (forces_dev_out)
-                OMM_HIP(hipMemcpyAsync(forces_dev_out, force_d_.p, 3 * (size_t)n * sizeof(double),
-                                       hipMemcpyDeviceToDevice, s));
-            OMM_HIP(hipStreamSynchronize(s));
-        }
+        const double* e = res->energy;
+        if (forces) std::memcpy(forces, out, n3 * sizeof(double));
         if (want_stats) {
-            unsigned long long st2[2];
-            stats_.download(st2, 2, s);
-            OMM_HIP(hipStreamSynchronize(s));
-            if (num_pairs) *num_pairs = (int64_t)st2[0];
-            if (pair_hash) *pair_hash = st2[1];
+            if (num_pairs) *num_pairs = (int64_t)res->stats[0];
+            if (pair_hash) *pair_hash = res->stats[1];
         }
         HostTerms ht = host_terms(0, b.volume, direct, recip);
         double p[5] = {e[E_DIRECT], e[E_EXCEPT], e[E_RECIP], ht.self, ht.dispersion};

@@ -1327,6 +1327,9 @@ void pme_setup(PmeDev& pm, std::vector<SysInfo>& sys, int natoms, const int* ato
     pm.nsys = nsys;
     pm.natoms = natoms;
     pm.atom_sys = atom_sys;
+    // Until an autotuner chooses: atom-owned where the grid is fixed point (at
+    // 900 atoms 18 us against 33 for the tiles, at 9,000 18 against 53).
+    pm.spread_atoms = mixed;
     std::vector<double> roots, moduli;
     long long qpts = 0, cpts = 0;
     for (int si = 0; si < nsys; ++si) {
