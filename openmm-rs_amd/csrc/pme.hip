@@ -241,20 +241,27 @@ __global__ __launch_bounds__(SPREAD_THREADS) void k_spread_tiles(const int* __re
     }
 }
 
-// Atom-owned spread (the autotuner's alternative to the tile-owned one): one
-// workgroup per chunk of PME_CHUNK sorted slots, or of PME_CHUNK atoms in
-// index order while no sorted order is available.  The chunk's stencils are
-// computed once.  When the chunk lies in one system and its stencil points
-// fit a box of at most SPREAD_BOX_BYTES of LDS, the contributions are summed
-// in that box and the box is added to the grid with one device atomic per
-// non-zero point; otherwise every contribution is added to the grid
-// directly.  Each contribution is the tile-owned spread's fixed-point value,
-// and integer sums do not depend on their order, so both spreads write the
-// same bits.  The grid is zero at the launch (the forward transform after
-// the previous spread cleared every point it read).
+// Atom-owned spread (the autotuner's alternative to the tile-owned one): chunks
+// of PME_CHUNK sorted slots, whose stencils lie in a small box of the grid.
+// The contributions are summed in the box in LDS and the box is added to the
+// grid with one device atomic per non-zero point; a chunk whose box does not
+// fit SPREAD_BOX_BYTES adds every contribution to the grid.  Each contribution
+// is the tile-owned spread's value, and integer sums do not depend on their
+// order, so on a fixed-point grid both spreads write the same bits (FP64 grids
+// sum in a varying order either way).  The grid is zero at the launch (the
+// transform after the previous spread cleared every point).
+//
+// One workgroup per chunk; its four waves hold the same 64 atoms, one per lane,
+// with their weights in registers, and share the stencil's 25 rows.  Bound:
+// latency at small systems, the device atomics of the box (27 points per atom at
+// 100 atoms/nm^3) at large ones.  Kept in LDS with a thread per row of an atom's
+// stencil, and with tiles for FP64 grids, it took (here): 3,000 unsorted atoms on
+// an FP64 grid 57 us (22), 9,000 sorted ones 50 (14); FP32 stencils at 300,000
+// atoms 91 (83).  Four chunks per workgroup in one box add a third fewer points
+// and take twice as long below 60,000 atoms (36 us against 16 at 23,550).
 constexpr int SPREAD_BOX_BYTES = 32768;
-constexpr int ATOM_SPREAD_THREADS = 256;
-static_assert(PME_CHUNK == 64, "the atom-owned spread computes a chunk's stencils in one wave");
+constexpr int ATOM_SPREAD_WAVES = 4, ATOM_SPREAD_THREADS = 64 * ATOM_SPREAD_WAVES;
+static_assert(PME_CHUNK == 64, "a wave of the atom-owned spread holds a chunk");
 
 __device__ __forceinline__ int wave_min(int v) {
     for (int o = 32; o >= 1; o >>= 1) v = min(v, __shfl_xor(v, o, 64));
@@ -264,187 +271,196 @@ __device__ __forceinline__ int wave_max(int v) {
     for (int o = 32; o >= 1; o >>= 1) v = max(v, __shfl_xor(v, o, 64));
     return v;
 }
-__device__ __forceinline__ int wrap_index(int i, int n) {
-    i %= n;
-    return i < 0 ? i + n : i;
+// r reduced to (-n/2, n/2], for r in (-n, n).
+__device__ __forceinline__ int nearest_offset(int r, int n) {
+    if (r > n / 2) return r - n;
+    return r <= -(n - n / 2) ? r + n : r;
+}
+// i reduced to [0, n), for i in [-n, 3n) (a box is at most n + 4 points long).
+__device__ __forceinline__ int wrap_near(int i, int n) {
+    if (i < 0) i += n;
+    if (i >= n) i -= n;
+    return i >= n ? i - n : i;
+}
+// w[i] for an i known at run time, without an indexed register.
+template <class R>
+__device__ __forceinline__ R pick(const R w[5], int i) {
+    return i == 0 ? w[0] : (i == 1 ? w[1] : (i == 2 ? w[2] : (i == 3 ? w[3] : w[4])));
 }
 __device__ __forceinline__ void grid_add(long long* p, unsigned long long v) {
     atomicAdd(reinterpret_cast<unsigned long long*>(p), v);
 }
-__device__ __forceinline__ void grid_add(double* p, double v) { atomicAdd(p, v); }
+__device__ __forceinline__ void grid_add(double* p, double v) { unsafeAtomicAdd(p, v); }
+
+// A contribution q w: an int at 2^-24, or an Acc.
+template <class R, class G>
+struct SpreadRow {
+    static constexpr bool FIXED = sizeof(G) == sizeof(long long) && G(0.5) == G(0);  // int64 grid
+    using Acc = typename std::conditional<FIXED, unsigned long long, double>::type;
+    static constexpr bool I32 = FIXED && sizeof(R) == 4;
+    static __device__ __forceinline__ int at24(double q, R wx, R wy, R wz) {
+        const float qx = (float)(q * SPREAD32_SCALE) * (float)wx;
+        const float qxy = qx * (float)wy;
+        return __float2int_rn(qxy * (float)wz);
+    }
+    static __device__ __forceinline__ Acc full(double q, R wx, R wy, R wz, unsigned* status) {
+        const R wxy = wx * wy;
+        const double c = q * (double)(wxy * wz);
+        if constexpr (FIXED) return (Acc)to_fixed(c, GRID_SCALE, status);
+        else return c;
+    }
+};
+
+// Adds one atom's row to the grid directly.
+template <class R, class G>
+__device__ __forceinline__ void spread_row_direct(double q, R wx, R wy, const R wz[5], G* row, int gz0, int nz,
+                                                  bool use32, unsigned* status) {
+    using Row = SpreadRow<R, G>;
+#pragma unroll
+    for (int iz = 0; iz < 5; ++iz) {
+        int gz = gz0 + iz;
+        if (gz >= nz) gz -= nz;
+        typename Row::Acc v;
+        if (Row::I32 && use32) v = (typename Row::Acc)((long long)Row::at24(q, wx, wy, wz[iz]) * 65536ll);
+        else v = Row::full(q, wx, wy, wz[iz], status);
+        if (v != (typename Row::Acc)0) grid_add(row + gz, v);
+    }
+}
 
 template <class R, class G>
 __global__ __launch_bounds__(ATOM_SPREAD_THREADS) void k_spread_atoms(const int* __restrict__ chunk_off, int nsys,
-                                                                      const int* __restrict__ order, int natoms,
+                                                                      const int* __restrict__ order,
                                                                       const double* __restrict__ pos,
                                                                       const double* __restrict__ charge,
-                                                                      const int* __restrict__ atom_sys,
                                                                       const SysInfo* __restrict__ sys, G* grid,
                                                                       int small_charges, unsigned* status) {
-    constexpr bool FIXED = sizeof(G) == sizeof(long long) && G(0.5) == G(0);  // int64 grid
-    using Acc = typename std::conditional<FIXED, unsigned long long, double>::type;
-    constexpr bool I32 = FIXED && sizeof(R) == 4;
-    const bool use32 = I32 && small_charges;
+    using Row = SpreadRow<R, G>;
+    using Acc = typename Row::Acc;
+    const bool use32 = Row::I32 && small_charges;
     // The box: int32 sums at 2^-24 (at most PME_CHUNK contributions of
     // |q| w <= 2 x 0.2153 per point stay below 2^31) or Acc sums.
     __shared__ __align__(8) unsigned char s_raw[SPREAD_BOX_BYTES];
     int* box32 = reinterpret_cast<int*>(s_raw);
     Acc* box = reinterpret_cast<Acc*>(s_raw);
-    __shared__ int s_base[3][PME_CHUNK];  // box-local (fit) or grid base point
-    __shared__ R s_w[15][PME_CHUNK];
-    __shared__ double s_q[PME_CHUNK];
-    __shared__ int s_sys[PME_CHUNK];
-    __shared__ int s_org[3], s_ext[3], s_fit, s_lsys;
-    const int t = threadIdx.x;
-    if (t < PME_CHUNK) {
-        int a = -1;
-        if (chunk_off) {
-            const SysInfo& S = sys[find_sys(chunk_off, nsys, blockIdx.x)];
-            const int slot = S.slot_off + (blockIdx.x - S.chunk_off) * PME_CHUNK + t;
-            a = slot < S.slot_off + S.nblocks * IBLOCK ? order[slot] : -1;
-        } else {
-            const int i = blockIdx.x * PME_CHUNK + t;
-            a = i < natoms ? i : -1;
-        }
-        const double q = a >= 0 ? charge[a] : 0.0;
-        const bool on = q != 0.0;  // uncharged atoms do not spread (pme.rs:315-330)
-        int si = 0, idx[3] = {0, 0, 0};
-        if (on) {
-            si = atom_sys[a];
-            const SysInfo& S = sys[si];
-            R w[3][5], dw[3][5];
-            stencil<R>(pos + 3 * a, S.box, S.grid, idx, w, dw);
-            for (int d = 0; d < 3; ++d)
-                for (int k = 0; k < 5; ++k) s_w[5 * d + k][t] = w[d][k];
-        }
-        s_q[t] = q;
-        s_sys[t] = si;
-        const unsigned long long live = __ballot(on);
-        int fit = -1;  // nothing to spread
-        if (live) {
-            const int lead = __ffsll((long long)live) - 1;
-            const int lsys = __shfl(si, lead, 64);
-            const SysInfo& L = sys[lsys];
-            int rel[3], lo[3], ext[3], org[3];
-            for (int d = 0; d < 3; ++d) {
-                // Offsets from the lead atom's base point, taken in (-n/2, n/2].
-                const int n = L.grid[d];
-                org[d] = __shfl(idx[d], lead, 64);  // with every lane on: the lead need not be lane 0
-                int r = idx[d] - org[d];
-                if (r > n / 2) r -= n;
-                else if (r <= -(n - n / 2)) r += n;
-                rel[d] = r;
-                lo[d] = wave_min(on ? r : INT_MAX);
-                ext[d] = wave_max(on ? r : INT_MIN) - lo[d] + 5;
-            }
-            const long long vol = (long long)ext[0] * ext[1] * ext[2];
-            const int cap = SPREAD_BOX_BYTES / (use32 ? (int)sizeof(int) : (int)sizeof(Acc));
-            fit = (__ballot(on && si != lsys) == 0 && vol <= cap) ? 1 : 0;
-            for (int d = 0; d < 3; ++d) s_base[d][t] = fit ? rel[d] - lo[d] : idx[d];
-            if (t == 0) {
-                for (int d = 0; d < 3; ++d) {
-                    s_org[d] = wrap_index(org[d] + lo[d], L.grid[d]);
-                    s_ext[d] = ext[d];
-                }
-                s_lsys = lsys;
-            }
-        }
-        if (t == 0) s_fit = fit;
+    const int t = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(t >> 6), lane = t & 63;
+    int si = 0, local = blockIdx.x;
+    if (nsys > 1) {
+        si = find_sys(chunk_off, nsys, blockIdx.x);
+        local -= chunk_off[si];
     }
-    __syncthreads();
-    const int fit = s_fit;
-    if (fit < 0) return;
-    if (fit) {
-        const int e1 = s_ext[1], e2 = s_ext[2];
-        const int vol = s_ext[0] * e1 * e2;
-        for (int i = t; i < vol; i += ATOM_SPREAD_THREADS) {
-            if (I32 && use32) box32[i] = 0;
-            else box[i] = (Acc)0;
-        }
-        __syncthreads();
-        for (int item = t; item < PME_CHUNK * 25; item += ATOM_SPREAD_THREADS) {
-            const int m = item / 25, r = item - 25 * m;
-            const int ix = r / 5, iy = r - 5 * ix;
-            const double q = s_q[m];
-            if (q == 0.0) continue;
-            const int row = ((s_base[0][m] + ix) * e1 + s_base[1][m] + iy) * e2 + s_base[2][m];
-            const R wx = s_w[ix][m];
-            if (I32 && use32) {
-                const float qx = (float)(q * SPREAD32_SCALE) * (float)wx;
-                const float qxy = qx * (float)s_w[5 + iy][m];
-                for (int iz = 0; iz < 5; ++iz) {
-                    const int v = __float2int_rn(qxy * (float)s_w[10 + iz][m]);
-                    if (v) atomicAdd(box32 + row + iz, v);
-                }
-            } else {
-                const R wxy = wx * s_w[5 + iy][m];
-                for (int iz = 0; iz < 5; ++iz) {
-                    const double c = q * (double)(wxy * s_w[10 + iz][m]);
-                    if (FIXED) lds_add(reinterpret_cast<unsigned long long*>(box) + row + iz,
-                                       (long long)to_fixed(c, GRID_SCALE, status));
-                    else lds_add(reinterpret_cast<double*>(box) + row + iz, c);
-                }
+    const SysInfo& S = sys[si];
+    const int slot = S.slot_off + local * PME_CHUNK + lane, end = S.slot_off + S.nblocks * IBLOCK;
+    const int listed = order[min(slot, end - 1)];
+    const int a = slot < end ? listed : -1, a0 = max(a, 0);
+    const double charge_a = charge[a0];
+    const double p[3] = {pos[3 * (size_t)a0], pos[3 * (size_t)a0 + 1], pos[3 * (size_t)a0 + 2]};
+    const int n[3] = {S.grid[0], S.grid[1], S.grid[2]};
+    int idx[3];
+    R w[3][5], dw[3][5];
+    stencil<R>(p, S.box, n, idx, w, dw);
+    const double q = a >= 0 ? charge_a : 0.0;
+    const bool on = q != 0.0;  // uncharged atoms do not spread (pme.rs:315-330)
+    const unsigned long long live = __ballot(on);
+    if (!live) return;  // the same in all four waves
+    // The box: offsets from the first charged atom, nearest images.
+    const int lead = __ffsll((long long)live) - 1;
+    int org[3], ext[3], at[3];
+    for (int d = 0; d < 3; ++d) {
+        const int first = __shfl(idx[d], lead, 64);
+        const int r = nearest_offset(idx[d] - first, n[d]);
+        const int lo = wave_min(on ? r : INT_MAX), hi = wave_max(on ? r : INT_MIN);
+        org[d] = wrap_near(first + lo, n[d]);
+        ext[d] = hi - lo + 5;
+        at[d] = r - lo;
+    }
+    G* g = grid + S.qgrid_off;
+    const int e1 = ext[1], e2 = ext[2], vol = ext[0] * e1 * e2;
+    if (vol > SPREAD_BOX_BYTES / (use32 ? (int)sizeof(int) : (int)sizeof(Acc))) {
+        if (!on) return;
+#pragma unroll 1
+        for (int ix = 0; ix < 5; ++ix) {
+            const R wx = pick(w[0], ix);
+            int gx = idx[0] + ix;
+            if (gx >= n[0]) gx -= n[0];
+#pragma unroll
+            for (int iy = 0; iy < 5; ++iy) {
+                if (((5 * ix + iy) & (ATOM_SPREAD_WAVES - 1)) != wave) continue;
+                int gy = idx[1] + iy;
+                if (gy >= n[1]) gy -= n[1];
+                spread_row_direct<R, G>(q, wx, w[1][iy], w[2], g + ((size_t)gx * n[1] + gy) * n[2], idx[2], n[2],
+                                        use32, status);
             }
-        }
-        __syncthreads();
-        const SysInfo& L = sys[s_lsys];
-        const int nx = L.grid[0], ny = L.grid[1], nz = L.grid[2];
-        G* g = grid + L.qgrid_off;
-        for (int i = t; i < vol; i += ATOM_SPREAD_THREADS) {
-            Acc v;
-            if (I32 && use32) {
-                const int v32 = box32[i];
-                if (!v32) continue;
-                v = (Acc)((long long)v32 * 65536ll);
-            } else {
-                v = box[i];
-                if (v == (Acc)0) continue;
-            }
-            const int lz = i % e2, rr = i / e2;
-            const int ly = rr % e1, lx = rr / e1;
-            const int gx = wrap_index(s_org[0] + lx, nx), gy = wrap_index(s_org[1] + ly, ny),
-                      gz = wrap_index(s_org[2] + lz, nz);
-            grid_add(g + ((size_t)gx * ny + gy) * nz + gz, v);
         }
         return;
     }
-    // Direct adds (a chunk spread over more than a box, or over systems).
-    for (int item = t; item < PME_CHUNK * 25; item += ATOM_SPREAD_THREADS) {
-        const int m = item / 25, r = item - 25 * m;
-        const int ix = r / 5, iy = r - 5 * ix;
-        const double q = s_q[m];
-        if (q == 0.0) continue;
-        const SysInfo& S = sys[s_sys[m]];
-        const int nx = S.grid[0], ny = S.grid[1], nz = S.grid[2];
-        int gx = s_base[0][m] + ix, gy = s_base[1][m] + iy;
-        if (gx >= nx) gx -= nx;
-        if (gy >= ny) gy -= ny;
-        G* grow = grid + S.qgrid_off + ((size_t)gx * ny + gy) * nz;
-        const int gz0 = s_base[2][m];
-        const R wx = s_w[ix][m];
-        if (I32 && use32) {
-            const float qx = (float)(q * SPREAD32_SCALE) * (float)wx;
-            const float qxy = qx * (float)s_w[5 + iy][m];
-            for (int iz = 0; iz < 5; ++iz) {
-                const int v = __float2int_rn(qxy * (float)s_w[10 + iz][m]);
-                int gz = gz0 + iz;
-                if (gz >= nz) gz -= nz;
-                if (v) grid_add(grow + gz, (unsigned long long)((long long)v * 65536ll));
-            }
-        } else {
-            const R wxy = wx * s_w[5 + iy][m];
-            for (int iz = 0; iz < 5; ++iz) {
-                const double c = q * (double)(wxy * s_w[10 + iz][m]);
-                int gz = gz0 + iz;
-                if (gz >= nz) gz -= nz;
-                if (FIXED) {
-                    const long long f = to_fixed(c, GRID_SCALE, status);
-                    if (f) grid_add(grow + gz, (unsigned long long)f);
-                } else if (c != 0.0) {
-                    grid_add(grow + gz, c);
+    for (int i = t; i < vol; i += ATOM_SPREAD_THREADS) {
+        if (Row::I32 && use32) box32[i] = 0;
+        else box[i] = (Acc)0;
+    }
+    __syncthreads();
+    if (on) {
+        const int base = (at[0] * e1 + at[1]) * e2 + at[2];
+#pragma unroll 1
+        for (int ix = 0; ix < 5; ++ix) {
+            const R wx = pick(w[0], ix);
+#pragma unroll
+            for (int iy = 0; iy < 5; ++iy) {
+                if (((5 * ix + iy) & (ATOM_SPREAD_WAVES - 1)) != wave) continue;
+                const int row = base + (ix * e1 + iy) * e2;
+#pragma unroll
+                for (int iz = 0; iz < 5; ++iz) {
+                    if (Row::I32 && use32) {
+                        const int v = Row::at24(q, wx, w[1][iy], w[2][iz]);
+                        if (v) atomicAdd(box32 + row + iz, v);
+                    } else {
+                        const Acc v = Row::full(q, wx, w[1][iy], w[2][iz], status);
+                        if (v != (Acc)0) atomicAdd(box + row + iz, v);
+                    }
                 }
             }
         }
+    }
+    __syncthreads();
+    // Sixteen threads per row of the box.
+    const float inv_e1 = 1.0f / (float)e1;
+    for (int row = t >> 4; row < ext[0] * e1; row += ATOM_SPREAD_THREADS / 16) {
+        const int lx = div_small(row, e1, inv_e1), ly = row - lx * e1;
+        G* grow = g + ((size_t)wrap_near(org[0] + lx, n[0]) * n[1] + wrap_near(org[1] + ly, n[1])) * n[2];
+        for (int lz = t & 15; lz < e2; lz += 16) {
+            Acc v;
+            if (Row::I32 && use32) v = (Acc)((long long)box32[row * e2 + lz] * 65536ll);
+            else v = box[row * e2 + lz];
+            if (v != (Acc)0) grid_add(grow + wrap_near(org[2] + lz, n[2]), v);
+        }
+    }
+}
+
+// Atoms in no spatial order: five threads per atom (one per x plane of the
+// stencil), every contribution added to the grid.
+template <class R, class G>
+__global__ __launch_bounds__(256) void k_spread_direct(int natoms, const double* __restrict__ pos,
+                                                       const double* __restrict__ charge,
+                                                       const int* __restrict__ atom_sys,
+                                                       const SysInfo* __restrict__ sys, G* grid, int small_charges,
+                                                       unsigned* status) {
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    const int a = t / 5, ix = t - 5 * a;
+    if (a >= natoms) return;
+    const double q = charge[a];
+    if (q == 0.0) return;  // pme.rs:315-330
+    const SysInfo& S = sys[atom_sys[a]];
+    int idx[3];
+    R w[3][5], dw[3][5];
+    stencil<R>(pos + 3 * (size_t)a, S.box, S.grid, idx, w, dw);
+    const R wx = pick(w[0], ix);
+    int gx = idx[0] + ix;
+    if (gx >= S.grid[0]) gx -= S.grid[0];
+#pragma unroll
+    for (int iy = 0; iy < 5; ++iy) {
+        int gy = idx[1] + iy;
+        if (gy >= S.grid[1]) gy -= S.grid[1];
+        spread_row_direct<R, G>(q, wx, w[1][iy], w[2], grid + S.qgrid_off + ((size_t)gx * S.grid[1] + gy) * S.grid[2],
+                                idx[2], S.grid[2], SpreadRow<R, G>::I32 && small_charges, status);
     }
 }
 
@@ -1001,16 +1017,14 @@ void run_t(PmeDev& pm, const NlistDev& nl, bool atom_order, const double* pos, c
     if (phases & PME_SPREAD) {
         const int* order = atom_order ? own : nl.sorted_atom.p;
         const int small = pm.max_charge <= SPREAD32_MAX_CHARGE ? 1 : 0;
-        // The atom-owned spread adds to the grid with device atomics, so it
-        // serves the fixed-point grids only (FP64 atomic sums would depend on
-        // their order).
-        constexpr bool fixed_grid = sizeof(G) == sizeof(long long) && G(0.5) == G(0);
-        if (pm.spread_atoms && fixed_grid) {
-            const int blocks = order ? nl.nchunks : (pm.natoms + PME_CHUNK - 1) / PME_CHUNK;
-            if (blocks > 0)
-                hipLaunchKernelGGL((k_spread_atoms<R, G>), dim3(blocks), dim3(ATOM_SPREAD_THREADS), 0, s,
-                                   order ? nl.chunk_off.p : nullptr, pm.nsys, order, pm.natoms, pos, charge,
-                                   pm.atom_sys, sys, qgrid, small, status);
+        if (pm.spread_atoms) {
+            if (!order) {
+                hipLaunchKernelGGL((k_spread_direct<R, G>), dim3((5 * pm.natoms + 255) / 256), dim3(256), 0, s,
+                                   pm.natoms, pos, charge, pm.atom_sys, sys, qgrid, small, status);
+            } else {
+                hipLaunchKernelGGL((k_spread_atoms<R, G>), dim3(nl.nchunks), dim3(ATOM_SPREAD_THREADS), 0, s,
+                                   nl.chunk_off.p, pm.nsys, order, pos, charge, sys, qgrid, small, status);
+            }
         } else {
             R* st_w = pme_weights<R>(pm);
             const int nitems = order ? nl.nslots : pm.natoms;
@@ -1026,7 +1040,7 @@ void run_t(PmeDev& pm, const NlistDev& nl, bool atom_order, const double* pos, c
     }
     if (phases & PME_FFT) {
         Cx<R>* cg = reinterpret_cast<Cx<R>*>(cgrid);
-        int* clear = (phases & PME_SPREAD) ? pm.bin_count.p : nullptr;
+        int* clear = (phases & PME_SPREAD) && !pm.spread_atoms ? pm.bin_count.p : nullptr;
         constexpr int prec = sizeof(R) == 8 ? 1 : 0;
         if (pm.dft_blocks[prec][0] > 0) {
             launch_dft<R, G, A>(pm, sys, qgrid, cgrid, phi, roots, moduli, energy, status, s, clear, pm.ntiles);
@@ -1327,9 +1341,9 @@ void pme_setup(PmeDev& pm, std::vector<SysInfo>& sys, int natoms, const int* ato
     pm.nsys = nsys;
     pm.natoms = natoms;
     pm.atom_sys = atom_sys;
-    // Until an autotuner chooses: atom-owned where the grid is fixed point (at
-    // 900 atoms 18 us against 33 for the tiles, at 9,000 18 against 53).
-    pm.spread_atoms = mixed;
+    // Until an autotuner chooses: atom-owned (9,000 atoms with FP64 stencils, 14
+    // us against 50 for the tiles).
+    pm.spread_atoms = true;
     std::vector<double> roots, moduli;
     long long qpts = 0, cpts = 0;
     for (int si = 0; si < nsys; ++si) {

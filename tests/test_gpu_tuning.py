@@ -178,3 +178,24 @@ def test_atom_owned_spread_with_uncharged_atoms():
     assert np.array_equal(forces[0][1], forces[1][1])
     f_ref, _ = orc.water_energy_forces(s)
     assert force_rms_rel(forces[1][0], f_ref) <= 2e-6
+
+
+@pytest.mark.parametrize("molecules,edge,tilt", [(21, 1.85, 0.0), (22, 1.85, 0.3), (300, 2.1, 0.0), (1500, 3.56, 0.3)])
+def test_atom_owned_spread_in_plain_fp64(molecules, edge, tilt):
+    # One chunk of 63 atoms, 64 + 2 atoms in scattered chunks (no box holds their
+    # stencils), several chunks, a tilted box.  FP64 grids are summed in a varying
+    # order: a point's sum of up to a few hundred contributions is off by at most
+    # their count times 2^-53, and the forces' sums add as much again.
+    s = water(molecules, edge, seed=17, cutoff=0.9)
+    s.box[2, 0] = tilt * edge
+    forces, energies = [], []
+    for tiles in (0, 8, 6):
+        c = ommhip.Context(s, temperature=0.0, friction=0.0, precision=ommhip.PRECISION_DOUBLE)
+        if tiles:
+            c.set_launch_tuning(tiles, 8, 0, 1)
+        state = c.get_state()
+        forces.append(state["forces"])
+        energies.append(state["potential_energy"])
+    for k in (1, 2):
+        assert np.abs(forces[k] - forces[0]).max() <= 1e-11 * np.abs(forces[0]).max()
+        assert abs(energies[k] - energies[0]) <= 1e-11 * abs(energies[0])
