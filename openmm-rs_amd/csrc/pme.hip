@@ -261,14 +261,21 @@ __global__ __launch_bounds__(SPREAD_THREADS) void k_spread_tiles(const int* __re
 // and take twice as long below 60,000 atoms (36 us against 16 at 23,550).
 constexpr int SPREAD_BOX_BYTES = 32768;
 constexpr int ATOM_SPREAD_WAVES = 4, ATOM_SPREAD_THREADS = 64 * ATOM_SPREAD_WAVES;
+// Smaller groups where that gives idle compute units work (chunks: time with 64,
+// 32 and 16 slots per workgroup, us): 15: 17, 12, 10; 141: 14, 11, 10; 368: 15, 14,
+// 20; 938: 24, 30, 40 (FP32 stencils).  FP64 ones at 360: 54, 43, 47.
+constexpr int SPREAD_16_CHUNKS = 192, SPREAD_32_CHUNKS = 256, SPREAD_32_CHUNKS_F64 = 512;
 static_assert(PME_CHUNK == 64, "a wave of the atom-owned spread holds a chunk");
 
-__device__ __forceinline__ int wave_min(int v) {
-    for (int o = 32; o >= 1; o >>= 1) v = min(v, __shfl_xor(v, o, 64));
+// Extrema over each N consecutive lanes.
+template <int N>
+__device__ __forceinline__ int group_min(int v) {
+    for (int o = N / 2; o >= 1; o >>= 1) v = min(v, __shfl_xor(v, o, 64));
     return v;
 }
-__device__ __forceinline__ int wave_max(int v) {
-    for (int o = 32; o >= 1; o >>= 1) v = max(v, __shfl_xor(v, o, 64));
+template <int N>
+__device__ __forceinline__ int group_max(int v) {
+    for (int o = N / 2; o >= 1; o >>= 1) v = max(v, __shfl_xor(v, o, 64));
     return v;
 }
 // r reduced to (-n/2, n/2], for r in (-n, n).
@@ -292,64 +299,69 @@ __device__ __forceinline__ void grid_add(long long* p, unsigned long long v) {
 }
 __device__ __forceinline__ void grid_add(double* p, double v) { unsafeAtomicAdd(p, v); }
 
-// A contribution q w: an int at 2^-24, or an Acc.
-template <class R, class G>
-struct SpreadRow {
+// A contribution q w to a grid of G: an int at 2^-24 (I32), or an Acc.
+template <class R, class G, bool I32>
+struct SpreadSum {
     static constexpr bool FIXED = sizeof(G) == sizeof(long long) && G(0.5) == G(0);  // int64 grid
     using Acc = typename std::conditional<FIXED, unsigned long long, double>::type;
-    static constexpr bool I32 = FIXED && sizeof(R) == 4;
-    static __device__ __forceinline__ int at24(double q, R wx, R wy, R wz) {
-        const float qx = (float)(q * SPREAD32_SCALE) * (float)wx;
-        const float qxy = qx * (float)wy;
-        return __float2int_rn(qxy * (float)wz);
+    using Box = typename std::conditional<I32, int, Acc>::type;  // a sum over one chunk
+    static __device__ __forceinline__ Box value(double q, R wx, R wy, R wz, unsigned* status) {
+        if constexpr (I32) {
+            const float qx = (float)(q * SPREAD32_SCALE) * (float)wx;
+            const float qxy = qx * (float)wy;
+            return __float2int_rn(qxy * (float)wz);
+        } else {
+            const R wxy = wx * wy;
+            const double c = q * (double)(wxy * wz);
+            if constexpr (FIXED) return (Acc)to_fixed(c, GRID_SCALE, status);
+            else return c;
+        }
     }
-    static __device__ __forceinline__ Acc full(double q, R wx, R wy, R wz, unsigned* status) {
-        const R wxy = wx * wy;
-        const double c = q * (double)(wxy * wz);
-        if constexpr (FIXED) return (Acc)to_fixed(c, GRID_SCALE, status);
-        else return c;
+    static __device__ __forceinline__ void to_grid(G* p, Box v) {
+        if constexpr (I32) grid_add(p, (unsigned long long)((long long)v * 65536ll));
+        else grid_add(p, v);
     }
 };
 
-// Adds one atom's row to the grid directly.
-template <class R, class G>
+// Adds one row of an atom's stencil to the grid directly.
+template <class R, class G, bool I32>
 __device__ __forceinline__ void spread_row_direct(double q, R wx, R wy, const R wz[5], G* row, int gz0, int nz,
-                                                  bool use32, unsigned* status) {
-    using Row = SpreadRow<R, G>;
+                                                  unsigned* status) {
+    using Sum = SpreadSum<R, G, I32>;
 #pragma unroll
     for (int iz = 0; iz < 5; ++iz) {
         int gz = gz0 + iz;
         if (gz >= nz) gz -= nz;
-        typename Row::Acc v;
-        if (Row::I32 && use32) v = (typename Row::Acc)((long long)Row::at24(q, wx, wy, wz[iz]) * 65536ll);
-        else v = Row::full(q, wx, wy, wz[iz], status);
-        if (v != (typename Row::Acc)0) grid_add(row + gz, v);
+        const typename Sum::Box v = Sum::value(q, wx, wy, wz[iz], status);
+        if (v != (typename Sum::Box)0) Sum::to_grid(row + gz, v);
     }
 }
 
-template <class R, class G>
+// ATOMS slots per workgroup: lane k of every ATOMS lanes holds slot k, and the
+// groups of ATOMS lanes share the rows.
+template <class R, class G, bool I32, int ATOMS>
 __global__ __launch_bounds__(ATOM_SPREAD_THREADS) void k_spread_atoms(const int* __restrict__ chunk_off, int nsys,
                                                                       const int* __restrict__ order,
                                                                       const double* __restrict__ pos,
                                                                       const double* __restrict__ charge,
                                                                       const SysInfo* __restrict__ sys, G* grid,
-                                                                      int small_charges, unsigned* status) {
-    using Row = SpreadRow<R, G>;
-    using Acc = typename Row::Acc;
-    const bool use32 = Row::I32 && small_charges;
-    // The box: int32 sums at 2^-24 (at most PME_CHUNK contributions of
-    // |q| w <= 2 x 0.2153 per point stay below 2^31) or Acc sums.
-    __shared__ __align__(8) unsigned char s_raw[SPREAD_BOX_BYTES];
-    int* box32 = reinterpret_cast<int*>(s_raw);
-    Acc* box = reinterpret_cast<Acc*>(s_raw);
-    const int t = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(t >> 6), lane = t & 63;
-    int si = 0, local = blockIdx.x;
+                                                                      unsigned* status) {
+    using Sum = SpreadSum<R, G, I32>;
+    using Box = typename Sum::Box;
+    constexpr int PARTS = PME_CHUNK / ATOMS, GROUPS = ATOM_SPREAD_THREADS / ATOMS;
+    // The box (int32 sums at 2^-24: at most PME_CHUNK contributions of
+    // |q| w <= 2 x 0.2153 per point stay below 2^31).
+    __shared__ Box box[SPREAD_BOX_BYTES / sizeof(Box)];
+    const int t = threadIdx.x, k = t & (ATOMS - 1), group = t / ATOMS;
+    const int chunk = blockIdx.x / PARTS;
+    int si = 0, local = chunk;
     if (nsys > 1) {
-        si = find_sys(chunk_off, nsys, blockIdx.x);
+        si = find_sys(chunk_off, nsys, chunk);
         local -= chunk_off[si];
     }
     const SysInfo& S = sys[si];
-    const int slot = S.slot_off + local * PME_CHUNK + lane, end = S.slot_off + S.nblocks * IBLOCK;
+    const int slot = S.slot_off + local * PME_CHUNK + (blockIdx.x & (PARTS - 1)) * ATOMS + k;
+    const int end = S.slot_off + S.nblocks * IBLOCK;
     const int listed = order[min(slot, end - 1)];
     const int a = slot < end ? listed : -1, a0 = max(a, 0);
     const double charge_a = charge[a0];
@@ -368,55 +380,37 @@ __global__ __launch_bounds__(ATOM_SPREAD_THREADS) void k_spread_atoms(const int*
     for (int d = 0; d < 3; ++d) {
         const int first = __shfl(idx[d], lead, 64);
         const int r = nearest_offset(idx[d] - first, n[d]);
-        const int lo = wave_min(on ? r : INT_MAX), hi = wave_max(on ? r : INT_MIN);
+        const int lo = group_min<ATOMS>(on ? r : INT_MAX), hi = group_max<ATOMS>(on ? r : INT_MIN);
         org[d] = wrap_near(first + lo, n[d]);
         ext[d] = hi - lo + 5;
         at[d] = r - lo;
     }
     G* g = grid + S.qgrid_off;
     const int e1 = ext[1], e2 = ext[2], vol = ext[0] * e1 * e2;
-    if (vol > SPREAD_BOX_BYTES / (use32 ? (int)sizeof(int) : (int)sizeof(Acc))) {
+    if (vol > SPREAD_BOX_BYTES / (int)sizeof(Box)) {
         if (!on) return;
-#pragma unroll 1
-        for (int ix = 0; ix < 5; ++ix) {
-            const R wx = pick(w[0], ix);
-            int gx = idx[0] + ix;
+        for (int r = group; r < 25; r += GROUPS) {
+            const int ix = r / 5, iy = r - 5 * ix;
+            int gx = idx[0] + ix, gy = idx[1] + iy;
             if (gx >= n[0]) gx -= n[0];
-#pragma unroll
-            for (int iy = 0; iy < 5; ++iy) {
-                if (((5 * ix + iy) & (ATOM_SPREAD_WAVES - 1)) != wave) continue;
-                int gy = idx[1] + iy;
-                if (gy >= n[1]) gy -= n[1];
-                spread_row_direct<R, G>(q, wx, w[1][iy], w[2], g + ((size_t)gx * n[1] + gy) * n[2], idx[2], n[2],
-                                        use32, status);
-            }
+            if (gy >= n[1]) gy -= n[1];
+            spread_row_direct<R, G, I32>(q, pick(w[0], ix), pick(w[1], iy), w[2],
+                                         g + ((size_t)gx * n[1] + gy) * n[2], idx[2], n[2], status);
         }
         return;
     }
-    for (int i = t; i < vol; i += ATOM_SPREAD_THREADS) {
-        if (Row::I32 && use32) box32[i] = 0;
-        else box[i] = (Acc)0;
-    }
+    for (int i = t; i < vol; i += ATOM_SPREAD_THREADS) box[i] = (Box)0;
     __syncthreads();
     if (on) {
         const int base = (at[0] * e1 + at[1]) * e2 + at[2];
-#pragma unroll 1
-        for (int ix = 0; ix < 5; ++ix) {
-            const R wx = pick(w[0], ix);
+        for (int r = group; r < 25; r += GROUPS) {
+            const int ix = r / 5, iy = r - 5 * ix;
+            const R wx = pick(w[0], ix), wy = pick(w[1], iy);
+            Box* row = box + base + (ix * e1 + iy) * e2;
 #pragma unroll
-            for (int iy = 0; iy < 5; ++iy) {
-                if (((5 * ix + iy) & (ATOM_SPREAD_WAVES - 1)) != wave) continue;
-                const int row = base + (ix * e1 + iy) * e2;
-#pragma unroll
-                for (int iz = 0; iz < 5; ++iz) {
-                    if (Row::I32 && use32) {
-                        const int v = Row::at24(q, wx, w[1][iy], w[2][iz]);
-                        if (v) atomicAdd(box32 + row + iz, v);
-                    } else {
-                        const Acc v = Row::full(q, wx, w[1][iy], w[2][iz], status);
-                        if (v != (Acc)0) atomicAdd(box + row + iz, v);
-                    }
-                }
+            for (int iz = 0; iz < 5; ++iz) {
+                const Box v = Sum::value(q, wx, wy, w[2][iz], status);
+                if (v != (Box)0) atomicAdd(row + iz, v);
             }
         }
     }
@@ -427,21 +421,19 @@ __global__ __launch_bounds__(ATOM_SPREAD_THREADS) void k_spread_atoms(const int*
         const int lx = div_small(row, e1, inv_e1), ly = row - lx * e1;
         G* grow = g + ((size_t)wrap_near(org[0] + lx, n[0]) * n[1] + wrap_near(org[1] + ly, n[1])) * n[2];
         for (int lz = t & 15; lz < e2; lz += 16) {
-            Acc v;
-            if (Row::I32 && use32) v = (Acc)((long long)box32[row * e2 + lz] * 65536ll);
-            else v = box[row * e2 + lz];
-            if (v != (Acc)0) grid_add(grow + wrap_near(org[2] + lz, n[2]), v);
+            const Box v = box[row * e2 + lz];
+            if (v != (Box)0) Sum::to_grid(grow + wrap_near(org[2] + lz, n[2]), v);
         }
     }
 }
 
 // Atoms in no spatial order: five threads per atom (one per x plane of the
 // stencil), every contribution added to the grid.
-template <class R, class G>
+template <class R, class G, bool I32>
 __global__ __launch_bounds__(256) void k_spread_direct(int natoms, const double* __restrict__ pos,
                                                        const double* __restrict__ charge,
                                                        const int* __restrict__ atom_sys,
-                                                       const SysInfo* __restrict__ sys, G* grid, int small_charges,
+                                                       const SysInfo* __restrict__ sys, G* grid,
                                                        unsigned* status) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     const int a = t / 5, ix = t - 5 * a;
@@ -459,8 +451,8 @@ __global__ __launch_bounds__(256) void k_spread_direct(int natoms, const double*
     for (int iy = 0; iy < 5; ++iy) {
         int gy = idx[1] + iy;
         if (gy >= S.grid[1]) gy -= S.grid[1];
-        spread_row_direct<R, G>(q, wx, w[1][iy], w[2], grid + S.qgrid_off + ((size_t)gx * S.grid[1] + gy) * S.grid[2],
-                                idx[2], S.grid[2], SpreadRow<R, G>::I32 && small_charges, status);
+        spread_row_direct<R, G, I32>(q, wx, w[1][iy], w[2], grid + S.qgrid_off + ((size_t)gx * S.grid[1] + gy) * S.grid[2],
+                                     idx[2], S.grid[2], status);
     }
 }
 
@@ -1003,6 +995,24 @@ double* pme_weights<double>(PmeDev& pm) {
     return pm.st_wd.p;
 }
 
+template <class R, class G, bool I32>
+void launch_spread_atoms(const PmeDev& pm, const NlistDev& nl, const int* order, const double* pos,
+                         const double* charge, const SysInfo* sys, G* qgrid, unsigned* status, hipStream_t s) {
+    auto chunks = [&](auto kernel, int atoms) {
+        hipLaunchKernelGGL(kernel, dim3(nl.nchunks * (PME_CHUNK / atoms)), dim3(ATOM_SPREAD_THREADS), 0, s,
+                           nl.chunk_off.p, pm.nsys, order, pos, charge, sys, qgrid, status);
+    };
+    if (!order)
+        hipLaunchKernelGGL((k_spread_direct<R, G, I32>), dim3((5 * pm.natoms + 255) / 256), dim3(256), 0, s, pm.natoms,
+                           pos, charge, pm.atom_sys, sys, qgrid, status);
+    else if (nl.nchunks < SPREAD_16_CHUNKS)
+        chunks(k_spread_atoms<R, G, I32, 16>, 16);
+    else if (nl.nchunks < (sizeof(R) == 8 ? SPREAD_32_CHUNKS_F64 : SPREAD_32_CHUNKS))
+        chunks(k_spread_atoms<R, G, I32, 32>, 32);
+    else
+        chunks(k_spread_atoms<R, G, I32, 64>, 64);
+}
+
 template <class R, class G, class A>
 void run_t(PmeDev& pm, const NlistDev& nl, bool atom_order, const double* pos, const double* charge,
            const SysInfo* sys, G* qgrid,
@@ -1018,13 +1028,9 @@ void run_t(PmeDev& pm, const NlistDev& nl, bool atom_order, const double* pos, c
         const int* order = atom_order ? own : nl.sorted_atom.p;
         const int small = pm.max_charge <= SPREAD32_MAX_CHARGE ? 1 : 0;
         if (pm.spread_atoms) {
-            if (!order) {
-                hipLaunchKernelGGL((k_spread_direct<R, G>), dim3((5 * pm.natoms + 255) / 256), dim3(256), 0, s,
-                                   pm.natoms, pos, charge, pm.atom_sys, sys, qgrid, small, status);
-            } else {
-                hipLaunchKernelGGL((k_spread_atoms<R, G>), dim3(nl.nchunks), dim3(ATOM_SPREAD_THREADS), 0, s,
-                                   nl.chunk_off.p, pm.nsys, order, pos, charge, sys, qgrid, small, status);
-            }
+            constexpr bool I32 = sizeof(R) == 4 && SpreadSum<R, G, false>::FIXED;
+            if (I32 && small) launch_spread_atoms<R, G, I32>(pm, nl, order, pos, charge, sys, qgrid, status, s);
+            else launch_spread_atoms<R, G, false>(pm, nl, order, pos, charge, sys, qgrid, status, s);
         } else {
             R* st_w = pme_weights<R>(pm);
             const int nitems = order ? nl.nslots : pm.natoms;
