@@ -9,18 +9,6 @@
 
 namespace ommhip {
 
-// Bonded terms of the MD step on the device: exceptions, harmonic bonds and
-// harmonic angles, grouped by small molecule (see MdContext::build_bonded).
-struct BondedDev {
-    int ngroups = 0, ne = 0, nb = 0, na = 0;  // groups; all exceptions / bonds / angles
-    int ge = 0, gb = 0, ga = 0;               // of which grouped (stored first)
-    DevBuf<int> grp_atoms;                    // [ngroups][4], -1 padded
-    DevBuf<int> grp_e, grp_b, grp_a;          // [ngroups + 1] term offsets per group
-    DevBuf<int> e1, e2, b1, b2, a1, a2, a3;
-    DevBuf<double> eqq, esig, eeps, blen, bk, ath, ak;
-    DevBuf<double> ec6;  // LJPME: exception particles' C6
-};
-
 // Monte Carlo barostat state of one system (barostat.rs:42-57, 129-195) plus
 // the record of its last attempt.
 struct BaroState {
@@ -210,7 +198,6 @@ private:
     // molecules of mass M > 0, 6 components per replica.
     void kinetic_tensor(std::vector<double>& out);
     void setup_constraints(const omm_md_desc* descs, int nsys, const std::vector<double>& inv);
-    void launch_bonded(hipStream_t s, long long* force_fx, double* force_d, long long* energy_fx, double* energy_d);
     // A barostat period of at most MAX_PERIOD_GRAPH steps is captured whole,
     // its attempt opening the last step; longer periods replay attempt-free
     // graphs of graph_steps_ steps and launch the attempt steps eagerly, so a
@@ -218,11 +205,6 @@ private:
     static constexpr int MAX_PERIOD_GRAPH = 1000;
     bool period_graph() const { return baro_.enabled && baro_.frequency <= MAX_PERIOD_GRAPH; }
     int graph_length() const { return period_graph() ? baro_.frequency : graph_steps_; }
-    void build_bonded(const std::vector<int>& e1, const std::vector<int>& e2, const std::vector<double>& eqq,
-                      const std::vector<double>& esig, const std::vector<double>& eeps, const std::vector<int>& b1,
-                      const std::vector<int>& b2, const std::vector<double>& blen, const std::vector<double>& bk,
-                      const std::vector<int>& a1, const std::vector<int>& a2, const std::vector<int>& a3,
-                      const std::vector<double>& ath, const std::vector<double>& ak);
     void clear_accumulators(hipStream_t s);
     void capture_graph();
     // Evaluates the forces, of which `count` values from `first` on are returned
@@ -255,9 +237,8 @@ private:
     // rebuild from the positions of their current list, which reproduces it).
     DevBuf<double> list_src_;
     std::vector<char> touched_;
-    BondedDev bonded_;
+    TermTiles bonded_;  // exceptions, bonds and angles
     ConstraintDev cons_;
-    std::vector<int> bonded_exc_order_;  // exception k of the bonded arrays = global exception order[k]
     BaroDev baro_;
     std::vector<int> bond1_h_, bond2_h_;  // bonds in global indices (molecules)
     std::vector<int> cons1_h_, cons2_h_;  // constraints in global indices (molecules)

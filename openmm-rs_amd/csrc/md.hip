@@ -22,125 +22,6 @@ namespace {
 // BOLTZMANN in kJ/mol/K (langevin.rs:12).
 const double BOLTZMANN = 1.380649e-23 * 6.02214076e23 / 1000.0;
 
-// Bonded terms in one launch.  Each small molecule (at most four atoms
-// joined by bonds, angles or exceptions, e.g. a water) takes GROUP_LANES
-// consecutive lanes: lane k evaluates the molecule's terms k, k + GROUP_LANES,
-// ... (its exceptions, then bonds, then angles) into per-atom sums in
-// registers, the lanes' sums are combined by a fixed butterfly of shuffles,
-// and the molecule's atoms receive one fixed-point add per component.  The
-// threads after the molecules' lanes take the terms outside such molecules
-// one each.  Indices are global over the batch; energies go to the term's
-// system.
-constexpr int GROUP_LANES = 8;
-__device__ __forceinline__ int group_slot(const int at[4], int i) {
-    return i == at[0] ? 0 : (i == at[1] ? 1 : (i == at[2] ? 2 : 3));
-}
-
-// f[slot] += v, with the slot chosen by selects (a register array; indexing
-// it with a run-time slot would put it in scratch memory).
-__device__ __forceinline__ void add_slot(double f[4][3], int slot, const double v[3]) {
-#pragma unroll
-    for (int k = 0; k < 4; ++k)
-#pragma unroll
-        for (int c = 0; c < 3; ++c) f[k][c] += slot == k ? v[c] : 0.0;
-}
-
-template <class A>
-__global__ __launch_bounds__(256) void k_bonded(
-    int ngroups, const int* __restrict__ grp_atoms, const int* __restrict__ grp_e, const int* __restrict__ grp_b,
-    const int* __restrict__ grp_a, int ne, int ge, const int* __restrict__ e1, const int* __restrict__ e2,
-    const double* __restrict__ eqq, const double* __restrict__ esig, const double* __restrict__ eeps, int nb, int gb,
-    const int* __restrict__ b1, const int* __restrict__ b2, const double* __restrict__ blen,
-    const double* __restrict__ bk, int na, int ga, const int* __restrict__ a1, const int* __restrict__ a2,
-    const int* __restrict__ a3, const double* __restrict__ ath, const double* __restrict__ ak,
-    const double* __restrict__ charge, int use_pbc, int has_pme, double alpha, const double* __restrict__ ec6,
-    double lj_alpha, const double* __restrict__ pos,
-    const int* __restrict__ atom_sys, const SysInfo* __restrict__ sys, A* force, A* energy, unsigned* status) {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    double ee = 0.0, eb = 0.0, ea = 0.0;
-    int se = -1, sb = -1, sa = -1;
-    const int grouped = ngroups * GROUP_LANES;  // a multiple of GROUP_LANES: a molecule's lanes share a branch
-    if (t < grouped) {
-        const int g = t / GROUP_LANES, lane = t % GROUP_LANES;
-        int at[4];
-        for (int k = 0; k < 4; ++k) at[k] = grp_atoms[4 * g + k];
-        const int si = atom_sys[at[0]];
-        const Box& box = sys[si].box;
-        const int e0 = grp_e[g], ne_g = grp_e[g + 1] - e0;
-        const int b0 = grp_b[g], nb_g = grp_b[g + 1] - b0;
-        const int a0 = grp_a[g], na_g = grp_a[g + 1] - a0;
-        double f[4][3] = {};
-        for (int k = lane; k < ne_g + nb_g + na_g; k += GROUP_LANES) {
-            if (k < ne_g) {
-                const int e = e0 + k, i = e1[e], j = e2[e];
-                double fi[3];
-                ee += exception_pair(i, j, eqq[e], esig[e], eeps[e], charge[i], charge[j], pos, box, use_pbc,
-                                     has_pme, alpha, ec6 ? ec6[e] : 0.0, lj_alpha, fi);
-                const double mi[3] = {-fi[0], -fi[1], -fi[2]};
-                add_slot(f, group_slot(at, i), fi);
-                add_slot(f, group_slot(at, j), mi);
-            } else if (k < ne_g + nb_g) {
-                const int b = b0 + k - ne_g, i = b1[b], j = b2[b];
-                double fi[3];
-                eb += bond_pair(i, j, blen[b], bk[b], pos, fi);
-                const double mi[3] = {-fi[0], -fi[1], -fi[2]};
-                add_slot(f, group_slot(at, i), fi);
-                add_slot(f, group_slot(at, j), mi);
-            } else {
-                const int a = a0 + k - ne_g - nb_g, i = a1[a], j = a2[a], l = a3[a];
-                double fi[3], fk[3];
-                ea += angle_triple(i, j, l, ath[a], ak[a], pos, fi, fk);
-                const double fj[3] = {-(fi[0] + fk[0]), -(fi[1] + fk[1]), -(fi[2] + fk[2])};
-                add_slot(f, group_slot(at, i), fi);
-                add_slot(f, group_slot(at, l), fk);
-                add_slot(f, group_slot(at, j), fj);
-            }
-        }
-#pragma unroll
-        for (int k = 0; k < 4; ++k)
-#pragma unroll
-            for (int c = 0; c < 3; ++c)
-#pragma unroll
-                for (int o = 1; o < GROUP_LANES; o <<= 1) f[k][c] += __shfl_xor(f[k][c], o, 64);
-        // Lane k adds the components k and k + GROUP_LANES of the 4 x 3.
-#pragma unroll
-        for (int q = 0; q < 12; q += GROUP_LANES) {
-            const int kc = q + lane;
-            if (kc < 12 && at[kc / 3] >= 0) {
-                double v = 0.0;
-#pragma unroll
-                for (int k = 0; k < 4; ++k)
-#pragma unroll
-                    for (int c = 0; c < 3; ++c) v = kc == 3 * k + c ? f[k][c] : v;
-                acc_add(force + 3 * at[kc / 3] + kc % 3, v, FORCE_SCALE, status);
-            }
-        }
-        se = ne_g > 0 ? si : -1;
-        sb = nb_g > 0 ? si : -1;
-        sa = na_g > 0 ? si : -1;
-    } else {
-        int u = t - grouped;
-        const int le = ne - ge, lb = nb - gb, la = na - ga;
-        if (u < le) {
-            const int e = ge + u, i = e1[e], j = e2[e];
-            se = atom_sys[i];
-            ee = exception_term(i, j, eqq[e], esig[e], eeps[e], charge[i], charge[j], pos, sys[se].box, use_pbc,
-                                has_pme, alpha, ec6 ? ec6[e] : 0.0, lj_alpha, force, status);
-        } else if ((u -= le) < lb) {
-            const int b = gb + u;
-            sb = atom_sys[b1[b]];
-            eb = bond_term(b1[b], b2[b], blen[b], bk[b], pos, force, status);
-        } else if ((u -= lb) < la) {
-            const int a = ga + u;
-            sa = atom_sys[a1[a]];
-            ea = angle_term(a1[a], a2[a], a3[a], ath[a], ak[a], pos, force, status);
-        }
-    }
-    wave_energy_add(energy, se, E_EXCEPT, ee, status);
-    wave_energy_add(energy, sb, E_BOND, eb, status);
-    wave_energy_add(energy, sa, E_ANGLE, ea, status);
-}
-
 // Philox4x32-10 (Salmon, Moraes, Dror, Shaw, SC'11), written from the paper.
 __device__ __forceinline__ void philox4x32_10(uint32_t c[4], uint32_t k0, uint32_t k1) {
     const uint32_t M0 = 0xD2511F53u, M1 = 0xCD9E8D57u, W0 = 0x9E3779B9u, W1 = 0xBB67AE85u;
@@ -977,7 +858,7 @@ MdContext::MdContext(const omm_md_desc* descs, int nsys, int precision) {
     n_ = nb_->total_particles();
     std::vector<double> inv;
     std::vector<int> b1, b2, a1, a2, a3;
-    std::vector<double> blen, bk, ath, ak;
+    std::vector<double> bp, ap;  // (length, k) of each bond, (theta0, k) of each angle
     for (int r = 0; r < nsys; ++r) {
         const omm_md_desc* d = descs + r;
         const int off = nb_->atom_offset(r), n = d->num_particles;
@@ -995,21 +876,21 @@ MdContext::MdContext(const omm_md_desc* descs, int nsys, int precision) {
         for (int k = 0; k < d->num_bonds; ++k) {
             b1.push_back(idx(d->bond_particle1, k));
             b2.push_back(idx(d->bond_particle2, k));
-            blen.push_back(d->bond_length[k]);
-            bk.push_back(d->bond_k[k]);
+            bp.push_back(d->bond_length[k]);
+            bp.push_back(d->bond_k[k]);
         }
         for (int k = 0; k < d->num_angles; ++k) {
             a1.push_back(idx(d->angle_particle1, k));
             a2.push_back(idx(d->angle_particle2, k));
             a3.push_back(idx(d->angle_particle3, k));
-            ath.push_back(d->angle_theta0[k]);
-            ak.push_back(d->angle_k[k]);
+            ap.push_back(d->angle_theta0[k]);
+            ap.push_back(d->angle_k[k]);
         }
         nb_->systems()[r].seed = d->seed;
     }
     nb_->upload_systems(s_);
     inv_mass_.upload(inv, s_);
-    // Exceptions in global indices (the bonded kernel evaluates them).
+    // Exceptions in global indices, evaluated with the bonded terms.
     std::vector<int> e1, e2;
     std::vector<double> eqq, esig, eeps, ec6;
     if (nb_->settings().include_direct)
@@ -1026,13 +907,10 @@ MdContext::MdContext(const omm_md_desc* descs, int nsys, int precision) {
                 eeps.push_back(c.exc_eps[k]);
             }
         }
-    build_bonded(e1, e2, eqq, esig, eeps, b1, b2, blen, bk, a1, a2, a3, ath, ak);
-    if (nb_->ljpme()) {
-        std::vector<double> p(bonded_exc_order_.size());
-        for (size_t k = 0; k < p.size(); ++k) p[k] = ec6[bonded_exc_order_[k]];
-        if (p.empty()) p.push_back(0.0);
-        bonded_.ec6.upload(p, s_);
-    }
+    std::vector<int> atom_sys;
+    for (int r = 0; r < nsys; ++r) atom_sys.insert(atom_sys.end(), nb_->num_particles(r), r);
+    bonded_.build(e1, e2, b1, b2, bp, a1, a2, a3, ap, atom_sys, s_);
+    bonded_.set_exceptions(eqq, esig, eeps, nb_->ljpme() ? ec6 : std::vector<double>(), s_);
     bond1_h_ = b1;
     bond2_h_ = b2;
     setup_constraints(descs, nsys, inv);
@@ -1208,153 +1086,6 @@ void MdContext::set_velocities(int r, const double* vel) {
     OMM_HIP(hipStreamSynchronize(s_));
 }
 
-// Groups the bonded terms by small molecule (connected components of at most
-// four atoms over bonds, angles and exceptions); terms of larger components
-// stay single.  Groups are ordered by their lowest atom, terms keep their
-// order within a group, so the layout is deterministic.
-void MdContext::build_bonded(const std::vector<int>& e1, const std::vector<int>& e2, const std::vector<double>& eqq,
-                             const std::vector<double>& esig, const std::vector<double>& eeps,
-                             const std::vector<int>& b1, const std::vector<int>& b2, const std::vector<double>& blen,
-                             const std::vector<double>& bk, const std::vector<int>& a1, const std::vector<int>& a2,
-                             const std::vector<int>& a3, const std::vector<double>& ath,
-                             const std::vector<double>& ak) {
-    std::vector<int> parent(n_), size(n_, 1);
-    for (int i = 0; i < n_; ++i) parent[i] = i;
-    std::function<int(int)> root = [&](int x) {
-        while (parent[x] != x) x = parent[x] = parent[parent[x]];
-        return x;
-    };
-    auto join = [&](int a, int b) {
-        a = root(a);
-        b = root(b);
-        if (a == b) return;
-        if (a > b) std::swap(a, b);
-        parent[b] = a;
-        size[a] += size[b];
-    };
-    for (size_t k = 0; k < e1.size(); ++k) join(e1[k], e2[k]);
-    for (size_t k = 0; k < b1.size(); ++k) join(b1[k], b2[k]);
-    for (size_t k = 0; k < a1.size(); ++k) {
-        join(a1[k], a2[k]);
-        join(a2[k], a3[k]);
-    }
-    // Group index of every small component that carries terms.
-    std::vector<int> group_of(n_, -1), roots;
-    auto small = [&](int a) { return size[root(a)] <= 4; };
-    auto mark = [&](int a) {
-        const int r = root(a);
-        if (group_of[r] < 0) {
-            group_of[r] = 0;
-            roots.push_back(r);
-        }
-    };
-    for (size_t k = 0; k < e1.size(); ++k)
-        if (small(e1[k])) mark(e1[k]);
-    for (size_t k = 0; k < b1.size(); ++k)
-        if (small(b1[k])) mark(b1[k]);
-    for (size_t k = 0; k < a1.size(); ++k)
-        if (small(a1[k])) mark(a1[k]);
-    std::sort(roots.begin(), roots.end());  // roots are the lowest atoms of their components
-    const int ng = (int)roots.size();
-    for (int g = 0; g < ng; ++g) group_of[roots[g]] = g;
-    std::vector<int> atoms(4 * (size_t)ng, -1), fill(ng, 0);
-    for (int i = 0; i < n_; ++i) {
-        const int r = root(i);
-        if (size[r] <= 4 && group_of[r] >= 0) {
-            const int g = group_of[r];
-            atoms[4 * g + fill[g]++] = i;
-        }
-    }
-    auto gid = [&](int a) { return small(a) ? group_of[root(a)] : -1; };
-    // Stable order: grouped terms by group, then the others.
-    auto order = [&](size_t count, auto&& group_fn, std::vector<int>& offsets) {
-        std::vector<int> idx(count);
-        for (size_t k = 0; k < count; ++k) idx[k] = (int)k;
-        std::stable_sort(idx.begin(), idx.end(), [&](int x, int y) {
-            int gx = group_fn(x), gy = group_fn(y);
-            gx = gx < 0 ? INT_MAX : gx;
-            gy = gy < 0 ? INT_MAX : gy;
-            return gx < gy;
-        });
-        offsets.assign(ng + 1, 0);
-        int grouped = 0;
-        for (size_t k = 0; k < count; ++k) {
-            const int g = group_fn((int)k);
-            if (g >= 0) {
-                ++offsets[g + 1];
-                ++grouped;
-            }
-        }
-        for (int g = 0; g < ng; ++g) offsets[g + 1] += offsets[g];
-        return std::make_pair(idx, grouped);
-    };
-    std::vector<int> oe, ob, oa;
-    auto [ie, ge] = order(e1.size(), [&](int k) { return gid(e1[k]); }, oe);
-    auto [ib, gb] = order(b1.size(), [&](int k) { return gid(b1[k]); }, ob);
-    auto [ia, ga] = order(a1.size(), [&](int k) { return gid(a1[k]); }, oa);
-    auto permute = [](const auto& v, const std::vector<int>& idx) {
-        std::remove_const_t<std::remove_reference_t<decltype(v)>> out(idx.size());
-        for (size_t k = 0; k < idx.size(); ++k) out[k] = v[idx[k]];
-        return out;
-    };
-    BondedDev& B = bonded_;
-    B.ngroups = ng;
-    B.ne = (int)e1.size();
-    B.nb = (int)b1.size();
-    B.na = (int)a1.size();
-    B.ge = ge;
-    B.gb = gb;
-    B.ga = ga;
-    B.grp_atoms.upload(atoms.empty() ? std::vector<int>{-1, -1, -1, -1} : atoms, s_);
-    B.grp_e.upload(oe, s_);
-    B.grp_b.upload(ob, s_);
-    B.grp_a.upload(oa, s_);
-    auto up_i = [&](DevBuf<int>& d, const std::vector<int>& v, const std::vector<int>& idx) {
-        std::vector<int> p = permute(v, idx);
-        if (p.empty()) p.push_back(0);
-        d.upload(p, s_);
-    };
-    auto up_d = [&](DevBuf<double>& d, const std::vector<double>& v, const std::vector<int>& idx) {
-        std::vector<double> p = permute(v, idx);
-        if (p.empty()) p.push_back(0.0);
-        d.upload(p, s_);
-    };
-    bonded_exc_order_ = ie;
-    up_i(B.e1, e1, ie);
-    up_i(B.e2, e2, ie);
-    up_d(B.eqq, eqq, ie);
-    up_d(B.esig, esig, ie);
-    up_d(B.eeps, eeps, ie);
-    up_i(B.b1, b1, ib);
-    up_i(B.b2, b2, ib);
-    up_d(B.blen, blen, ib);
-    up_d(B.bk, bk, ib);
-    up_i(B.a1, a1, ia);
-    up_i(B.a2, a2, ia);
-    up_i(B.a3, a3, ia);
-    up_d(B.ath, ath, ia);
-    up_d(B.ak, ak, ia);
-}
-
-void MdContext::launch_bonded(hipStream_t s, long long* force_fx, double* force_d, long long* energy_fx,
-                              double* energy_d) {
-    const BondedDev& B = bonded_;
-    const int total = B.ngroups * GROUP_LANES + (B.ne - B.ge) + (B.nb - B.gb) + (B.na - B.ga);
-    if (total == 0) return;
-    const int blocks = (total + 255) / 256;
-    auto go = [&](auto* force, auto* energy) {
-        using A = std::remove_pointer_t<decltype(force)>;
-        hipLaunchKernelGGL(k_bonded<A>, dim3(blocks), dim3(256), 0, s, B.ngroups, B.grp_atoms.p, B.grp_e.p,
-                           B.grp_b.p, B.grp_a.p, B.ne, B.ge, B.e1.p, B.e2.p, B.eqq.p, B.esig.p, B.eeps.p, B.nb, B.gb,
-                           B.b1.p, B.b2.p, B.blen.p, B.bk.p, B.na, B.ga, B.a1.p, B.a2.p, B.a3.p, B.ath.p, B.ak.p,
-                           nb_->charge_dev(), nb_->exceptions_pbc() ? 1 : 0, nb_->screened() ? 1 : 0, nb_->alpha(),
-                           nb_->ljpme() ? B.ec6.p : nullptr, nb_->ljpme() ? nb_->lj_alpha() : 0.0, pos_.p, nb_->atom_sys_dev(), nb_->systems_dev(), force, energy, status_.p);
-    };
-    if (mixed_) go(force_fx, energy_fx);
-    else go(force_d, energy_d);
-    OMM_HIP(hipGetLastError());
-}
-
 void MdContext::enqueue_forces(hipStream_t s, bool energy, int rebuild) {
     enqueue_forces_into(s, energy, rebuild, force_fx_.p, force_d_.p, energy_fx_.p, energy_d_.p);
 }
@@ -1362,11 +1093,9 @@ void MdContext::enqueue_forces(hipStream_t s, bool energy, int rebuild) {
 void MdContext::enqueue_forces_into(hipStream_t s, bool energy, int rebuild, long long* force_fx, double* force_d,
                                     long long* energy_fx, double* energy_d) {
     const NbSettings& c = nb_->settings();
-    nb_->enqueue(pos_.p, c.include_direct, true, energy, rebuild, false, force_fx, force_d, energy_fx, energy_d,
-                 status_.p, s, false);
-    // Concurrent with the mesh; force-only steps sum no bonded energies.
-    launch_bonded(s, force_fx, force_d, energy ? energy_fx : nullptr, energy ? energy_d : nullptr);
-    nb_->join(s);
+    // Force-only steps sum no bonded energies.
+    nb_->enqueue(pos_.p, c.include_direct, true, energy, rebuild, &bonded_, force_fx, force_d, energy_fx, energy_d,
+                 status_.p, s);
 }
 
 // One barostat attempt for every replica (context/program.rs:14-41): the
@@ -1544,7 +1273,7 @@ bool MdContext::set_parameter(const std::string& name, double value) {
     bool changed = false;
     const bool found = nb_->set_global_parameter(name, value, &changed);
     if (changed && nb_->settings().include_direct) {
-        // The bonded kernel keeps its own (grouped) copy of the exception parameters.
+        // The steps' terms keep their own copy of the exception parameters.
         std::vector<double> qq, sig, eps, c6;
         for (int r = 0; r < nsys_; ++r) {
             const NbSettings& c = nb_->settings(r);
@@ -1554,16 +1283,7 @@ bool MdContext::set_parameter(const std::string& name, double value) {
             sig.insert(sig.end(), c.exc_sig.begin(), c.exc_sig.end());
             eps.insert(eps.end(), c.exc_eps.begin(), c.exc_eps.end());
         }
-        auto permuted = [&](const std::vector<double>& v) {
-            std::vector<double> out(bonded_exc_order_.size());
-            for (size_t k = 0; k < out.size(); ++k) out[k] = v[bonded_exc_order_[k]];
-            if (out.empty()) out.push_back(0.0);
-            return out;
-        };
-        bonded_.eqq.upload(permuted(qq), s_);
-        bonded_.esig.upload(permuted(sig), s_);
-        bonded_.eeps.upload(permuted(eps), s_);
-        if (nb_->ljpme()) bonded_.ec6.upload(permuted(c6), s_);
+        bonded_.set_exceptions(qq, sig, eps, nb_->ljpme() ? c6 : std::vector<double>(), s_);
     }
     return found;
 }
@@ -2328,7 +2048,10 @@ void MdContext::profile(int reps, double ms[8], int64_t* num_pairs) {
         OMM_HIP(hipEventElapsedTime(&v, t0, t1));
         return (double)v / reps;
     };
-    ms[6] = timed([&] { launch_bonded(s_, force_fx_.p, force_d_.p, nullptr, nullptr); });
+    ms[6] = timed([&] {
+        nb_->enqueue(pos_.p, false, false, false, NbOperator::REBUILD_NONE, &bonded_, force_fx_.p, force_d_.p, nullptr,
+                     nullptr, status_.p, s_);
+    });
     // The integrator is timed on scratch copies of the state.
     DevBuf<double> px, vx;
     DevBuf<int> scratch_flag;  // stands in for the list's nsys + 1 rebuild flags

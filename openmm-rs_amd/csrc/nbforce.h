@@ -6,6 +6,7 @@
 #include <mutex>
 #include <string>
 
+#include "fold.h"
 #include "ewald.h"
 #include "pme.h"
 
@@ -134,24 +135,22 @@ public:
         REBUILD_FLAG = 3     // rebuild if the list's flag is set (raised by the integrator)
     };
     // Device-resident enqueue for the MD step: neighbour-list rebuild per the
-    // policy, direct pairs, exceptions (unless the caller evaluates them
-    // itself) and PME into the caller's accumulators (forces over all atoms,
+    // policy, direct pairs, the caller's terms (nullable) and PME into the caller's accumulators (forces over all atoms,
     // energies E_SLOTS per system).  Graph-capturable.  energy: also
     // accumulate energies (slower, accurate path in the mixed form).
     // The PME mesh runs on a side stream concurrently with the pairs; with
     // join_now false the caller enqueues more work on s and then calls join(s).
-    void enqueue(const double* pos_dev, bool direct, bool recip, bool energy, int rebuild, bool exceptions,
+    void enqueue(const double* pos_dev, bool direct, bool recip, bool energy, int rebuild, const TermTiles* terms,
                  long long* force_fx, double* force_d, long long* energy_fx, double* energy_d, unsigned* status,
                  hipStream_t s, bool join_now = true);
     void join(hipStream_t s);
     // PME arithmetic for a force-only or an energy evaluation.
     int mesh_mode(bool energy) const;
 
-    // Device data the MD step's fused kernels use.
-    const ExceptionDev& exceptions() const { return exc_; }
-    const double* charge_dev() const { return part_.charge.p; }
+    // How launch_fold evaluates this operator's terms.
+    TermParams term_params() const;
+    // Device data the MD step's kernels use.
     const int* atom_sys_dev() const { return part_.atom_sys.p; }
-    bool exceptions_pbc() const { return cfg_[0].exceptions_pbc; }
     // Non-periodic method on a virtual box (one system).
     bool is_virtual() const { return virtual_; }
     // MD contexts of a non-periodic method: keeps the virtual box while the
@@ -160,8 +159,6 @@ public:
     // it.  Writes the region the integrators check.  Returns true when the
     // device was set up (lists must be rebuilt, captured graphs dropped).
     bool fit_virtual_box(const double* pos, int count);
-    // Exceptions carry the reciprocal-space correction (PME or Ewald).
-    bool screened() const { return cfg_[0].screened(); }
     const double* pos_build() const { return nl_.pos_build.p; }
     int* list_flag() { return nl_.flag.p; }
     double skin() const { return nl_.skin; }
@@ -305,7 +302,7 @@ private:
     std::vector<SysInfo> sys_h_;
     DevBuf<SysInfo> sys_dev_;
     ParticleDev part_;
-    ExceptionDev exc_;
+    TermTiles exc_;
     NlistDev nl_;
     PmeDev pme_;
     EwaldDev ewald_;

@@ -474,9 +474,7 @@ void NbOperator::setup_device(const std::vector<Box>& boxes) {
         off += n_[si];
     }
     part_.atom_sys.upload(atom_sys, s);
-    exc_.count = (int)p1.size();
-    exc_.p1.upload(p1, s);
-    exc_.p2.upload(p2, s);
+    exc_.build(p1, p2, {}, {}, {}, {}, {}, {}, {}, atom_sys, s);
     upload_parameters(s);
 
     const NbSettings& c0 = cfg_[0];
@@ -690,8 +688,6 @@ void NbOperator::upload_parameters(hipStream_t s) {
         part_.c6amp.upload(amp, s);
         pme_lj_.max_charge = 0.0;
         for (double b : amp) pme_lj_.max_charge = std::max(pme_lj_.max_charge, std::fabs(b));
-        if (ec6.empty()) ec6.push_back(0.0);
-        exc_.c6.upload(ec6, s);
     }
     if (mixed_) {
         part_.qk.upload(qk, s);
@@ -701,9 +697,7 @@ void NbOperator::upload_parameters(hipStream_t s) {
     part_.qk_d.upload(qkd, s);
     part_.sh_d.upload(shd, s);
     part_.e2_d.upload(e2d, s);
-    exc_.qq.upload(eqq, s);
-    exc_.sig.upload(esig, s);
-    exc_.eps.upload(eeps, s);
+    exc_.set_exceptions(eqq, esig, eeps, ec6, s);
 }
 
 void NbOperator::refresh_parameters() {
@@ -1166,7 +1160,7 @@ void NbOperator::autotune(const double* pos_dev, unsigned* status, hipStream_t s
         for (int scale : {1, 2, -2}) {
             const int g = scale == 1 ? base : (scale == 2 ? std::min(65535, 2 * base) : std::max(64, base / 2));
             const double t = timed([&] {
-                launch_pairs(mixed_, false, nl_, pp_, part_, pos_dev, sys_dev_.p, f_fx.p, f_d.p, e_fx.p, e_d.p, status,
+                launch_pairs(mixed_, false, nl_, pp_, part_, pos_dev, sys_dev_.p, e_fx.p, e_d.p, status,
                              nullptr, g, s);
             });
             if (t < best) {
@@ -1176,6 +1170,8 @@ void NbOperator::autotune(const double* pos_dev, unsigned* status, hipStream_t s
             }
         }
         tuning_.pair_ms = best;
+        launch_fold(mixed_, nl_, true, nullptr, term_params(), part_.charge.p, pos_dev, sys_dev_.p, f_fx.p, f_d.p,
+                    nullptr, nullptr, status, s);  // clears the slots' sums
         pair_grid_ = tuning_.pair_grid;
     }
     tuning_.from_cache = 0;
@@ -1382,7 +1378,7 @@ int NbOperator::mesh_mode(bool energy) const {
     return energy ? MESH_F64_FIXED : MESH_F32;
 }
 
-void NbOperator::enqueue(const double* pos_dev, bool direct, bool recip, bool energy, int rebuild, bool exceptions,
+void NbOperator::enqueue(const double* pos_dev, bool direct, bool recip, bool energy, int rebuild, const TermTiles* terms,
                          long long* force_fx, double* force_d, long long* energy_fx, double* energy_d,
                          unsigned* status, hipStream_t s, bool join_now) {
     const NbSettings& c = cfg_[0];
@@ -1435,20 +1431,22 @@ void NbOperator::enqueue(const double* pos_dev, bool direct, bool recip, bool en
         OMM_HIP(hipEventRecord(ev_join_, side_));
         joined_ = false;
     }
+    int* next[2] = {nullptr, nullptr};
     if (direct) {
-        int* next[2] = {nullptr, nullptr};
         if (mesh && own_order && c.pme_mesh()) {
             next[0] = pme_next_order(pme_, nl_);
             if (ljpme()) next[1] = pme_next_order(pme_lj_, nl_);
         }
-        launch_pairs(mixed_, energy, nl_, pp_, part_, pos_dev, sys_dev_.p, force_fx, force_d, energy_fx, energy_d,
-                     status, nullptr, pair_grid_, s, true, next[0], next[1]);
-        if (exceptions)
-            launch_exceptions(mixed_, exc_, part_, pos_dev, sys_dev_.p, c.exceptions_pbc ? 1 : 0,
-                              c.screened() ? 1 : 0, alpha_[0], ljpme() ? lj_alpha_[0] : 0.0, force_fx, force_d,
-                              energy_fx, energy_d, status, s);
+        launch_pairs(mixed_, energy, nl_, pp_, part_, pos_dev, sys_dev_.p, energy_fx, energy_d, status, nullptr,
+                     pair_grid_, s);
     }
+    launch_fold(mixed_, nl_, direct, terms, term_params(), part_.charge.p, pos_dev, sys_dev_.p, force_fx, force_d,
+                energy ? energy_fx : nullptr, energy ? energy_d : nullptr, status, s, next[0], next[1]);
     if (join_now) join(s);
+}
+
+TermParams NbOperator::term_params() const {
+    return {cfg_[0].exceptions_pbc ? 1 : 0, cfg_[0].screened() ? 1 : 0, alpha_[0], ljpme() ? lj_alpha_[0] : 0.0};
 }
 
 void NbOperator::join(hipStream_t s) {
@@ -1482,19 +1480,18 @@ void NbOperator::profile(const double* pos_dev, int reps, long long* force_fx, d
     };
     const NbSettings& c = cfg_[0];
     const bool pme = c.pme_mesh();
-    const bool screened = c.screened();
-    const double lj_a = ljpme() ? lj_alpha_[0] : 0.0;
     ms[0] = timed([&] { nlist_build(nl_, pos_dev, sys_dev_.p, status, s, true); });
     // The pair kernel alone; its slot-ordered sums are folded in once after.
     ms[1] = timed([&] {
-        launch_pairs(mixed_, false, nl_, pp_, part_, pos_dev, sys_dev_.p, force_fx, force_d, energy_fx, energy_d,
-                     status, nullptr, pair_grid_, s, false);
+        launch_pairs(mixed_, false, nl_, pp_, part_, pos_dev, sys_dev_.p, energy_fx, energy_d,
+                     status, nullptr, pair_grid_, s);
     });
-    launch_slot_forces(mixed_, nl_, force_fx, force_d, s);
-    ms[2] = timed([&] {
-        launch_exceptions(mixed_, exc_, part_, pos_dev, sys_dev_.p, c.exceptions_pbc ? 1 : 0, screened ? 1 : 0,
-                          alpha_[0], lj_a, force_fx, force_d, energy_fx, energy_d, status, s);
-    });
+    auto fold = [&](bool slots, const TermTiles* terms) {
+        launch_fold(mixed_, nl_, slots, terms, term_params(), part_.charge.p, pos_dev, sys_dev_.p, force_fx, force_d,
+                    energy_fx, energy_d, status, s);
+    };
+    fold(true, nullptr);
+    ms[2] = timed([&] { fold(false, &exc_); });
     const int phases[3] = {PME_SPREAD, PME_FFT, PME_GATHER};
     for (int k = 0; k < 3; ++k)
         ms[3 + k] = pme ? timed([&] {
@@ -1512,8 +1509,9 @@ void NbOperator::profile(const double* pos_dev, int reps, long long* force_fx, d
         DevBuf<unsigned long long> st_dev;
         st_dev.alloc(2 * sys_h_.size());
         fill_async<unsigned long long>(st_dev.p, 2 * sys_h_.size(), 0ull, s);
-        launch_pairs(mixed_, false, nl_, pp_, part_, pos_dev, sys_dev_.p, force_fx, force_d, energy_fx, energy_d,
+        launch_pairs(mixed_, false, nl_, pp_, part_, pos_dev, sys_dev_.p, energy_fx, energy_d,
                      status, st_dev.p, pair_grid_, s);
+        fold(true, nullptr);
         std::vector<unsigned long long> st(2 * sys_h_.size());
         st_dev.download(st.data(), st.size(), s);
         OMM_HIP(hipStreamSynchronize(s));
@@ -1618,11 +1616,10 @@ void NbOperator::compute(const double* pos, const double* box, bool direct, bool
                       energy_fx_.p, energy_d_.p, status_.p, mixed_, rs);
         if (beside) OMM_HIP(hipEventRecord(ev_join_, side_));
         if (direct) {
-            launch_pairs(mixed_, want_energy, nl_, pp_, part_, pos_dev_.p, sys_dev_.p, force_fx_.p, force_d_.p,
+            launch_pairs(mixed_, want_energy, nl_, pp_, part_, pos_dev_.p, sys_dev_.p,
                          energy_fx_.p, energy_d_.p, status_.p, want_stats ? stats_.p : nullptr, pair_grid_, s);
-            launch_exceptions(mixed_, exc_, part_, pos_dev_.p, sys_dev_.p, c.exceptions_pbc ? 1 : 0,
-                              c.screened() ? 1 : 0, alpha_[0], ljpme() ? lj_alpha_[0] : 0.0, force_fx_.p,
-                              force_d_.p, energy_fx_.p, energy_d_.p, status_.p, s);
+            launch_fold(mixed_, nl_, true, &exc_, term_params(), part_.charge.p, pos_dev_.p, sys_dev_.p, force_fx_.p,
+                        force_d_.p, energy_fx_.p, energy_d_.p, status_.p, s);
         }
         if (beside) OMM_HIP(hipStreamWaitEvent(s, ev_join_, 0));
         const size_t nout = out ? n3 : 0;

@@ -1,4 +1,4 @@
-// Direct-space pair kernel and exception kernel.
+// Direct-space pair kernel.
 #pragma once
 
 #include "nlist.h"
@@ -37,38 +37,16 @@ struct ParticleDev {
     DevBuf<double> c6amp;             // LJPME mesh amplitude 2 sqrt(epsilon) sigma^3 (pme.rs:50-51)
 };
 
-struct ExceptionDev {
-    int count = 0;
-    DevBuf<int> p1, p2;
-    DevBuf<double> qq, sig, eps;
-    DevBuf<double> c6;  // LJPME: the particles' C6 (the dispersion correction), else empty
-};
-
 // Direct-space pairs over the tile list.  mixed: FP32 math with int64
 // fixed-point force/energy accumulation; otherwise FP64 math with FP64 atomics
 // into force_d/energy_d.  The pair kernel accumulates into the list's
-// slot-ordered buffer; a second kernel adds that into the caller's forces
-// (atom order) and clears it.  energy_on: also accumulate the energy (in the mixed
+// slot-ordered buffer; launch_fold adds that into the caller's forces (atom
+// order) and clears it.  energy_on: also accumulate the energy (in the mixed
 // form each pair energy is evaluated in FP64).  stats (nullable): [0] pair
 // count, [1] pair hash per system (no energy is accumulated then).  Energies
-// go to slot E_DIRECT of each system's E_SLOTS block.  order_a/order_b
-// (nullable, nl.nslots ints each): the second kernel also copies the list's
-// slot order there.
+// go to slot E_DIRECT of each system's E_SLOTS block.
 void launch_pairs(bool mixed, bool energy_on, const NlistDev& nl, const PairParams& p, const ParticleDev& part,
-                  const double* pos, const SysInfo* sys_dev, long long* force_fx, double* force_d,
-                  long long* energy_fx, double* energy_d, unsigned* status, unsigned long long* stats,
-                  int grid, hipStream_t s, bool combine = true, int* order_a = nullptr, int* order_b = nullptr);
-
-// The second kernel alone: adds the slot-ordered pair forces into force_fx
-// (mixed) or force_d and clears them (after launch_pairs with combine = false).
-void launch_slot_forces(bool mixed, const NlistDev& nl, long long* force_fx, double* force_d, hipStream_t s);
-
-// Exceptions (nonbonded.rs:995-1036), FP64 math.  has_pme selects the erf
-// reciprocal correction with particle charges.
-// lj_alpha > 0 adds the LJPME dispersion correction with ex.c6.
-void launch_exceptions(bool mixed, const ExceptionDev& ex, const ParticleDev& part, const double* pos,
-                       const SysInfo* sys_dev, int use_pbc, int has_pme, double alpha, double lj_alpha,
-                       long long* force_fx, double* force_d, long long* energy_fx, double* energy_d, unsigned* status,
-                       hipStream_t s);
+                  const double* pos, const SysInfo* sys_dev, long long* energy_fx, double* energy_d, unsigned* status, unsigned long long* stats,
+                  int grid, hipStream_t s);
 
 }  // namespace ommhip

@@ -1,5 +1,5 @@
-// Direct-space LJ + Ewald-screened Coulomb over the tile list, and the
-// exception kernel (nonbonded.rs:842-924, 995-1036).
+// Direct-space LJ + Ewald-screened Coulomb over the tile list
+// (nonbonded.rs:842-924).
 //
 // One wave64 per task = (cluster of 8 i-atoms, up to tpt consecutive tiles
 // of 64 entries of the cluster's list); the loads of the next tiles are in
@@ -697,25 +697,6 @@ __global__ __launch_bounds__(64 * ENERGY_WAVES) void k_pair_energy(
 }
 
 template <class A>
-__global__ void k_exceptions(int count, const int* __restrict__ p1, const int* __restrict__ p2,
-                             const double* __restrict__ eqq, const double* __restrict__ esig,
-                             const double* __restrict__ eeps, const double* __restrict__ charge,
-                             const double* __restrict__ pos, const int* __restrict__ atom_sys,
-                             const SysInfo* __restrict__ sys, int use_pbc, int has_pme, double alpha,
-                             const double* __restrict__ c6, double lj_alpha, A* force, A* energy, unsigned* status) {
-    int k = blockIdx.x * blockDim.x + threadIdx.x;
-    double e = 0.0;
-    int si = -1;
-    if (k < count) {
-        int i = p1[k], j = p2[k];
-        si = atom_sys[i];
-        e = exception_term(i, j, eqq[k], esig[k], eeps[k], charge[i], charge[j], pos, sys[si].box, use_pbc, has_pme,
-                           alpha, c6 ? c6[k] : 0.0, lj_alpha, force, status);
-    }
-    wave_energy_add(energy, si, E_EXCEPT, e, status);
-}
-
-template <class A>
 A* slot_buffer(const NlistDev& nl);
 template <>
 long long* slot_buffer<long long>(const NlistDev& nl) {
@@ -726,36 +707,10 @@ double* slot_buffer<double>(const NlistDev& nl) {
     return nl.fslot_d.p;
 }
 
-// Adds the slot-ordered pair forces into the atom-ordered accumulator and
-// clears them.  Atomic, because the mesh may add into the same accumulator
-// from another stream meanwhile.  order_a/order_b (nullable): copies of the
-// slot order it reads, for the meshes' next run.
-__device__ __forceinline__ void add_raw(long long* p, long long v) {
-    atomicAdd(reinterpret_cast<unsigned long long*>(p), (unsigned long long)v);
-}
-__device__ __forceinline__ void add_raw(double* p, double v) { unsafeAtomicAdd(p, v); }
-
-template <class A>
-__global__ void k_slot_forces(const int* __restrict__ sorted_atom, int nslots, A* fslot, A* force, int* order_a,
-                              int* order_b) {
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= nslots) return;
-    const int a = sorted_atom[s];
-    if (order_a) order_a[s] = a;
-    if (order_b) order_b[s] = a;
-    for (int c = 0; c < 3; ++c) {
-        const A v = fslot[(size_t)c * nslots + s];
-        if (v != (A)0) {
-            if (a >= 0) add_raw(force + 3 * a + c, v);
-            fslot[(size_t)c * nslots + s] = (A)0;
-        }
-    }
-}
-
 template <class R, class A, int ELEC, bool STATS, bool ENERGY>
 void launch_one(const NlistDev& nl, const PairParams& p, const R* qk, const R* sh, const R* e2,
-                const ParticleDev& part, const double* pos, const SysInfo* sys_dev, A* force, A* energy,
-                unsigned* status, unsigned long long* stats, int grid, bool combine, int* const* order_out,
+                const ParticleDev& part, const double* pos, const SysInfo* sys_dev, A* energy,
+                unsigned* status, unsigned long long* stats, int grid,
                 hipStream_t s) {
     constexpr bool MIXED = sizeof(R) == 4;
     hipLaunchKernelGGL((k_pairs<R, A, ELEC, STATS, ENERGY && !MIXED>), dim3(grid), dim3(64), 0, s, pos, qk, sh, e2,
@@ -768,25 +723,19 @@ void launch_one(const NlistDev& nl, const PairParams& p, const R* qk, const R* s
                            part.sh_d.p, part.e2_d.p, nl.sorted_atom.p, nl.clist_ex.p, nl.block_center.p,
                            nl.block_minimg.p, nl.clist.p, nl.ccount.p, nl.tasks.p, nl.ntasks.p, nl.block_sys.p,
                            sys_dev, p, nl.tpt, energy, status);
-    if (combine)
-        hipLaunchKernelGGL(k_slot_forces<A>, dim3((nl.nslots + 255) / 256), dim3(256), 0, s, nl.sorted_atom.p,
-                           nl.nslots, slot_buffer<A>(nl), force, order_out[0], order_out[1]);
 }
 
 template <class R, class A, int ELEC>
 void launch_pairs_t(bool stats_on, bool energy_on, const NlistDev& nl, const PairParams& p, const R* qk, const R* sh,
-                    const R* e2, const ParticleDev& part, const double* pos, const SysInfo* sys_dev, A* force, A* energy,
-                    unsigned* status, unsigned long long* stats, int grid, bool combine, int* const* order_out,
+                    const R* e2, const ParticleDev& part, const double* pos, const SysInfo* sys_dev, A* energy,
+                    unsigned* status, unsigned long long* stats, int grid,
                     hipStream_t s) {
     if (stats_on)
-        launch_one<R, A, ELEC, true, false>(nl, p, qk, sh, e2, part, pos, sys_dev, force, energy, status, stats, grid,
-                                            combine, order_out, s);
+        launch_one<R, A, ELEC, true, false>(nl, p, qk, sh, e2, part, pos, sys_dev, energy, status, stats, grid, s);
     else if (energy_on)
-        launch_one<R, A, ELEC, false, true>(nl, p, qk, sh, e2, part, pos, sys_dev, force, energy, status, stats, grid,
-                                            combine, order_out, s);
+        launch_one<R, A, ELEC, false, true>(nl, p, qk, sh, e2, part, pos, sys_dev, energy, status, stats, grid, s);
     else
-        launch_one<R, A, ELEC, false, false>(nl, p, qk, sh, e2, part, pos, sys_dev, force, energy, status, stats, grid,
-                                             combine, order_out, s);
+        launch_one<R, A, ELEC, false, false>(nl, p, qk, sh, e2, part, pos, sys_dev, energy, status, stats, grid, s);
 }
 
 }  // namespace
@@ -798,33 +747,28 @@ namespace {
 template <class R, class A>
 void dispatch_kind(int kind, bool st, bool energy_on, const NlistDev& nl, const PairParams& p, const R* qk,
                    const R* sh, const R* e2, const ParticleDev& part, const double* pos, const SysInfo* sys_dev,
-                   A* force, A* energy, unsigned* status, unsigned long long* stats, int grid, bool combine,
-                   int* const* order_out, hipStream_t s) {
+                   A* energy, unsigned* status, unsigned long long* stats, int grid, hipStream_t s) {
     switch (kind) {
         case ELEC_EWALD:
-            launch_pairs_t<R, A, ELEC_EWALD>(st, energy_on, nl, p, qk, sh, e2, part, pos, sys_dev, force, energy, status,
-                                             stats, grid, combine, order_out, s);
+            launch_pairs_t<R, A, ELEC_EWALD>(st, energy_on, nl, p, qk, sh, e2, part, pos, sys_dev, energy, status,
+                                             stats, grid, s);
             break;
         case ELEC_REACTION_FIELD:
-            launch_pairs_t<R, A, ELEC_REACTION_FIELD>(st, energy_on, nl, p, qk, sh, e2, part, pos, sys_dev, force,
-                                                      energy, status, stats, grid, combine, order_out, s);
+            launch_pairs_t<R, A, ELEC_REACTION_FIELD>(st, energy_on, nl, p, qk, sh, e2, part, pos, sys_dev, energy, status, stats, grid, s);
             break;
         case ELEC_COULOMB:
-            launch_pairs_t<R, A, ELEC_COULOMB>(st, energy_on, nl, p, qk, sh, e2, part, pos, sys_dev, force, energy,
-                                               status, stats, grid, combine, order_out, s);
+            launch_pairs_t<R, A, ELEC_COULOMB>(st, energy_on, nl, p, qk, sh, e2, part, pos, sys_dev, energy,
+                                               status, stats, grid, s);
             break;
         case ELEC_EWALD | PAIR_SWITCH:
-            launch_pairs_t<R, A, ELEC_EWALD | PAIR_SWITCH>(st, energy_on, nl, p, qk, sh, e2, part, pos, sys_dev, force,
-                                                           energy, status, stats, grid, combine, order_out, s);
+            launch_pairs_t<R, A, ELEC_EWALD | PAIR_SWITCH>(st, energy_on, nl, p, qk, sh, e2, part, pos, sys_dev, energy, status, stats, grid, s);
             break;
         case ELEC_REACTION_FIELD | PAIR_SWITCH:
             launch_pairs_t<R, A, ELEC_REACTION_FIELD | PAIR_SWITCH>(st, energy_on, nl, p, qk, sh, e2, part, pos,
-                                                                    sys_dev, force, energy, status, stats, grid,
-                                                                    combine, order_out, s);
+                                                                    sys_dev, energy, status, stats, grid, s);
             break;
         case ELEC_EWALD | PAIR_LJPME:
-            launch_pairs_t<R, A, ELEC_EWALD | PAIR_LJPME>(st, energy_on, nl, p, qk, sh, e2, part, pos, sys_dev, force,
-                                                          energy, status, stats, grid, combine, order_out, s);
+            launch_pairs_t<R, A, ELEC_EWALD | PAIR_LJPME>(st, energy_on, nl, p, qk, sh, e2, part, pos, sys_dev, energy, status, stats, grid, s);
             break;
         default:
             throw Error(OMM_ERR_INVALID, "no pair kernel for this electrostatics / switching combination");
@@ -833,46 +777,15 @@ void dispatch_kind(int kind, bool st, bool energy_on, const NlistDev& nl, const 
 }  // namespace
 
 void launch_pairs(bool mixed, bool energy_on, const NlistDev& nl, const PairParams& p, const ParticleDev& part,
-                  const double* pos, const SysInfo* sys_dev, long long* force_fx, double* force_d, long long* energy_fx,
-                  double* energy_d, unsigned* status, unsigned long long* stats, int grid, hipStream_t s,
-                  bool combine, int* order_a, int* order_b) {
+                  const double* pos, const SysInfo* sys_dev, long long* energy_fx, double* energy_d, unsigned* status, unsigned long long* stats, int grid, hipStream_t s) {
     const bool st = stats != nullptr;
-    int* const order_out[2] = {order_a, order_b};
     const int kind = p.elec | (p.switching ? PAIR_SWITCH : 0) | (p.ljpme ? PAIR_LJPME : 0);
     if (mixed)
         dispatch_kind<float, long long>(kind, st, energy_on, nl, p, part.qk.p, part.sh.p, part.e2.p, part, pos,
-                                        sys_dev, force_fx, energy_fx, status, stats, grid, combine, order_out, s);
+                                        sys_dev, energy_fx, status, stats, grid, s);
     else
         dispatch_kind<double, double>(kind, st, energy_on, nl, p, part.qk_d.p, part.sh_d.p, part.e2_d.p, part, pos,
-                                      sys_dev, force_d, energy_d, status, stats, grid, combine, order_out, s);
-    OMM_HIP(hipGetLastError());
-}
-
-void launch_slot_forces(bool mixed, const NlistDev& nl, long long* force_fx, double* force_d, hipStream_t s) {
-    if (mixed)
-        hipLaunchKernelGGL(k_slot_forces<long long>, dim3((nl.nslots + 255) / 256), dim3(256), 0, s, nl.sorted_atom.p,
-                           nl.nslots, nl.fslot_fx.p, force_fx, nullptr, nullptr);
-    else
-        hipLaunchKernelGGL(k_slot_forces<double>, dim3((nl.nslots + 255) / 256), dim3(256), 0, s, nl.sorted_atom.p,
-                           nl.nslots, nl.fslot_d.p, force_d, nullptr, nullptr);
-    OMM_HIP(hipGetLastError());
-}
-
-void launch_exceptions(bool mixed, const ExceptionDev& ex, const ParticleDev& part, const double* pos,
-                       const SysInfo* sys_dev, int use_pbc, int has_pme, double alpha, double lj_alpha,
-                       long long* force_fx, double* force_d, long long* energy_fx, double* energy_d, unsigned* status,
-                       hipStream_t s) {
-    if (ex.count == 0) return;
-    int blocks = (ex.count + 255) / 256;
-    const double* c6 = lj_alpha > 0.0 ? ex.c6.p : nullptr;
-    if (mixed)
-        hipLaunchKernelGGL(k_exceptions<long long>, dim3(blocks), dim3(256), 0, s, ex.count, ex.p1.p, ex.p2.p, ex.qq.p,
-                           ex.sig.p, ex.eps.p, part.charge.p, pos, part.atom_sys.p, sys_dev, use_pbc, has_pme, alpha,
-                           c6, lj_alpha, force_fx, energy_fx, status);
-    else
-        hipLaunchKernelGGL(k_exceptions<double>, dim3(blocks), dim3(256), 0, s, ex.count, ex.p1.p, ex.p2.p, ex.qq.p,
-                           ex.sig.p, ex.eps.p, part.charge.p, pos, part.atom_sys.p, sys_dev, use_pbc, has_pme, alpha,
-                           c6, lj_alpha, force_d, energy_d, status);
+                                      sys_dev, energy_d, status, stats, grid, s);
     OMM_HIP(hipGetLastError());
 }
 

@@ -1,5 +1,4 @@
-// FP64 per-term device functions shared by the exception kernel and the MD
-// step's fused bonded kernel.  Each returns the term's energy and writes the
+// FP64 per-term device functions.  Each returns the term's energy and writes the
 // forces on its particles; the caller accumulates them.
 #pragma once
 
@@ -83,15 +82,6 @@ __device__ __forceinline__ double exception_xyz(const double pi[3], const double
     return e;
 }
 
-__device__ __forceinline__ double exception_pair(int i, int j, double qq, double sig, double eps, double qi, double qj,
-                                                 const double* __restrict__ pos, const Box& box, int use_pbc,
-                                                 int has_pme, double alpha, double c6, double lj_alpha,
-                                                 double fi[3]) {
-    const double pi[3] = {pos[3 * i], pos[3 * i + 1], pos[3 * i + 2]};
-    const double pj[3] = {pos[3 * j], pos[3 * j + 1], pos[3 * j + 2]};
-    return exception_xyz(pi, pj, qq, sig, eps, qi, qj, box, use_pbc, has_pme, alpha, c6, lj_alpha, fi);
-}
-
 // HarmonicBondForce term without PBC (harmonic_bond.rs:113-140).  Force on i
 // is fi, on j is -fi.
 __device__ __forceinline__ double bond_xyz(const double pi[3], const double pj[3], double length, double k,
@@ -102,13 +92,6 @@ __device__ __forceinline__ double bond_xyz(const double pi[3], const double pj[3
     double f = k * dr / r;
     for (int a = 0; a < 3; ++a) fi[a] = f * d[a];
     return 0.5 * k * dr * dr;
-}
-
-__device__ __forceinline__ double bond_pair(int i, int j, double length, double k, const double* __restrict__ pos,
-                                            double fi[3]) {
-    const double pi[3] = {pos[3 * i], pos[3 * i + 1], pos[3 * i + 2]};
-    const double pj[3] = {pos[3 * j], pos[3 * j + 1], pos[3 * j + 2]};
-    return bond_xyz(pi, pj, length, k, fi);
 }
 
 // HarmonicAngleForce term without PBC (harmonic_angle.rs:118-167); j is the
@@ -132,54 +115,6 @@ __device__ __forceinline__ double angle_xyz(const double pi[3], const double pj[
         fk[a] = -de * (c * rjk[a] / ljk - rji[a] / lji) / (ljk * s);
     }
     return 0.5 * ka * dth * dth;
-}
-
-__device__ __forceinline__ double angle_triple(int i, int j, int k, double theta0, double ka,
-                                               const double* __restrict__ pos, double fi[3], double fk[3]) {
-    const double pi[3] = {pos[3 * i], pos[3 * i + 1], pos[3 * i + 2]};
-    const double pj[3] = {pos[3 * j], pos[3 * j + 1], pos[3 * j + 2]};
-    const double pk[3] = {pos[3 * k], pos[3 * k + 1], pos[3 * k + 2]};
-    return angle_xyz(pi, pj, pk, theta0, ka, fi, fk);
-}
-
-// Accumulating forms: add the forces to the force accumulator.
-template <class A>
-__device__ __forceinline__ double exception_term(int i, int j, double qq, double sig, double eps, double qi, double qj,
-                                                 const double* __restrict__ pos, const Box& box, int use_pbc,
-                                                 int has_pme, double alpha, double c6, double lj_alpha, A* force,
-                                                 unsigned* status) {
-    double fi[3];
-    const double e = exception_pair(i, j, qq, sig, eps, qi, qj, pos, box, use_pbc, has_pme, alpha, c6, lj_alpha, fi);
-    for (int a = 0; a < 3; ++a) {
-        acc_add(force + 3 * i + a, fi[a], FORCE_SCALE, status);
-        acc_add(force + 3 * j + a, -fi[a], FORCE_SCALE, status);
-    }
-    return e;
-}
-
-template <class A>
-__device__ __forceinline__ double bond_term(int i, int j, double length, double k, const double* __restrict__ pos,
-                                            A* force, unsigned* status) {
-    double fi[3];
-    const double e = bond_pair(i, j, length, k, pos, fi);
-    for (int a = 0; a < 3; ++a) {
-        acc_add(force + 3 * i + a, fi[a], FORCE_SCALE, status);
-        acc_add(force + 3 * j + a, -fi[a], FORCE_SCALE, status);
-    }
-    return e;
-}
-
-template <class A>
-__device__ __forceinline__ double angle_term(int i, int j, int k, double theta0, double ka,
-                                             const double* __restrict__ pos, A* force, unsigned* status) {
-    double fi[3], fk[3];
-    const double e = angle_triple(i, j, k, theta0, ka, pos, fi, fk);
-    for (int a = 0; a < 3; ++a) {
-        acc_add(force + 3 * i + a, fi[a], FORCE_SCALE, status);
-        acc_add(force + 3 * k + a, fk[a], FORCE_SCALE, status);
-        acc_add(force + 3 * j + a, -(fi[a] + fk[a]), FORCE_SCALE, status);
-    }
-    return e;
 }
 
 }  // namespace ommhip
