@@ -63,18 +63,9 @@ __global__ void k_check(const double* __restrict__ pos, const double* __restrict
     }
 }
 
-__device__ __forceinline__ void unit_key_of(int u, const double* __restrict__ pos, const int* __restrict__ unit_ptr,
-                                            const int* __restrict__ unit_atoms, const int* __restrict__ unit_sys,
-                                            const SysInfo* __restrict__ sys, const int* __restrict__ cell_rank,
-                                            int* unit_key, int* cell_count, const int* __restrict__ flag) {
-    const int si = unit_sys[u];
-    if (!flag[1 + si]) {
-        // Not rebuilt: the previous key reproduces the previous order.
-        atomicAdd(&cell_count[unit_key[u]], 1);
-        return;
-    }
-    int a = unit_atoms[unit_ptr[u]];
-    const SysInfo& S = sys[si];
+// Key of the cell that holds atom a (in the order of the cells' ranks).
+__device__ __forceinline__ int cell_key(int a, const double* __restrict__ pos, const SysInfo& S,
+                                        const int* __restrict__ cell_rank) {
     const Box& b = S.box;
     int c[3];
     for (int ax = 0; ax < 3; ++ax) {
@@ -85,9 +76,17 @@ __device__ __forceinline__ void unit_key_of(int u, const double* __restrict__ po
         int v = (int)(f * nc);
         c[ax] = v < 0 ? 0 : (v >= nc ? nc - 1 : v);
     }
-    int key = S.cell_off + cell_rank[S.cell_off + (c[0] * S.ncell[1] + c[1]) * S.ncell[2] + c[2]];
-    unit_key[u] = key;
-    atomicAdd(&cell_count[key], 1);
+    return S.cell_off + cell_rank[S.cell_off + (c[0] * S.ncell[1] + c[1]) * S.ncell[2] + c[2]];
+}
+
+__device__ __forceinline__ void unit_key_of(int u, const double* __restrict__ pos, const int* __restrict__ unit_ptr,
+                                            const int* __restrict__ unit_atoms, const int* __restrict__ unit_sys,
+                                            const SysInfo* __restrict__ sys, const int* __restrict__ cell_rank,
+                                            int* unit_key, int* cell_count, const int* __restrict__ flag) {
+    const int si = unit_sys[u];
+    // Not rebuilt: the previous key reproduces the previous order.
+    if (flag[1 + si]) unit_key[u] = cell_key(unit_atoms[unit_ptr[u]], pos, sys[si], cell_rank);
+    atomicAdd(&cell_count[unit_key[u]], 1);
 }
 
 __global__ void k_unit_keys(const double* __restrict__ pos, const int* __restrict__ unit_ptr,
@@ -415,25 +414,12 @@ __device__ void super_bounds_of(int sb, int si, const SysInfo& S, const int* __r
         }
 }
 
-// Two blocks per wave64: lanes 0-31 block 2*blockIdx.x, lanes 32-63 the next.
-// The first slot of a block always holds an atom (padding only ends a
-// system's last block).
-__global__ __launch_bounds__(64) void k_block_bounds(const double* __restrict__ pos,
-                                                     const int* __restrict__ sorted_atom, int nblocks,
-                                                     const int* __restrict__ block_sys,
-                                                     const SysInfo* __restrict__ sys, double reach,
-                                                     double* center, float* half, int* minimg,
-                                                     double* pos_build, float4* slot_pos, int* ntasks,
-                                                     const int* flag) {
-    if (!flag[0]) return;
-    if (blockIdx.x == 0 && threadIdx.x == 0) ntasks[0] = 0;  // k_clist appends the tasks anew
-    int lane = threadIdx.x;
-    int blk = blockIdx.x * 2 + (lane >> 5);
-    const int si = blk < nblocks ? block_sys[blk] : 0;
-    bool valid = blk < nblocks && flag[1 + si];  // unflagged systems keep their bounds
-    int a = valid ? sorted_atom[blk * IBLOCK + (lane & 31)] : -1;
-    int ref = valid ? sorted_atom[blk * IBLOCK] : 0;
-    const Box& b = sys[si].box;
+// Bounds of block blk from its 32 slots, one per lane of half a wave: a is the
+// lane's atom (-1: padding), ref the first slot's.
+__device__ __forceinline__ void block_bounds_of(int blk, bool valid, int a, int ref, const Box& b,
+                                                const double* __restrict__ pos, double reach, double* center,
+                                                float* half, int* minimg, double* pos_build, float4* slot_pos) {
+    const int lane = threadIdx.x & 63;
     double mn[3], mx[3];
     for (int k = 0; k < 3; ++k) {
         mn[k] = 1e300;
@@ -468,6 +454,109 @@ __global__ __launch_bounds__(64) void k_block_bounds(const double* __restrict__ 
             if (h + reach >= 0.5 * b.v[k * 4] - 1e-6) need = 1;
         }
         minimg[blk] = need;
+    }
+}
+
+// Two blocks per wave64: lanes 0-31 block 2*blockIdx.x, lanes 32-63 the next.
+// The first slot of a block always holds an atom (padding only ends a
+// system's last block).
+__global__ __launch_bounds__(64) void k_block_bounds(const double* __restrict__ pos,
+                                                     const int* __restrict__ sorted_atom, int nblocks,
+                                                     const int* __restrict__ block_sys,
+                                                     const SysInfo* __restrict__ sys, double reach,
+                                                     double* center, float* half, int* minimg,
+                                                     double* pos_build, float4* slot_pos, int* ntasks,
+                                                     const int* flag) {
+    if (!flag[0]) return;
+    if (blockIdx.x == 0 && threadIdx.x == 0) ntasks[0] = 0;  // k_clist appends the tasks anew
+    int lane = threadIdx.x;
+    int blk = blockIdx.x * 2 + (lane >> 5);
+    const int si = blk < nblocks ? block_sys[blk] : 0;
+    bool valid = blk < nblocks && flag[1 + si];  // unflagged systems keep their bounds
+    int a = valid ? sorted_atom[blk * IBLOCK + (lane & 31)] : -1;
+    int ref = valid ? sorted_atom[blk * IBLOCK] : 0;
+    block_bounds_of(blk, valid, a, ref, sys[si].box, pos, reach, center, half, minimg, pos_build, slot_pos);
+}
+
+// The whole chain up to the block bounds in one workgroup, for one system of
+// uniform units of at most SMALL_UNITS units, SMALL_CELLS cells and SMALL_SLOTS
+// slots: keys, cell counts, their scan, the scatter, the rank within the cell
+// and the placement with the same results as the launches above, from LDS.  One
+// launch instead of four, also on the many steps without a build: an evaluation
+// of 900 atoms 250 us -> 235, MD 51 us per step -> 49.
+constexpr int SMALL_WG = 1024, SMALL_UNITS = 2048, SMALL_CELLS = 4096, SMALL_SLOTS = 8192;
+
+__global__ __launch_bounds__(SMALL_WG) void k_list_small(
+    const double* __restrict__ pos, const int* __restrict__ unit_ptr, const int* __restrict__ unit_atoms,
+    const int* __restrict__ unit_pos, const int* __restrict__ unit_sys, int nunits, int uniform,
+    const SysInfo* __restrict__ sys, const int* __restrict__ cell_rank, int ncells, const int* __restrict__ excl_ptr,
+    const int* __restrict__ excl_idx, int closed, int* sorted_atom, int* atom_slot, int2* excl_range, int nblocks,
+    double reach, double* center, float* half, int* minimg, double* pos_build, float4* slot_pos, int* ntasks,
+    const int* __restrict__ flag) {
+    if (!flag[0]) return;
+    __shared__ int s_start[SMALL_CELLS + 1], s_atom[SMALL_SLOTS], s_wave[SMALL_WG / 64];
+    __shared__ unsigned short s_list[SMALL_UNITS];
+    const int t = threadIdx.x, lane = t & 63;
+    if (t == 0) ntasks[0] = 0;  // k_clist appends the tasks anew
+    if (!flag[1]) return;
+    for (int i = t; i <= SMALL_CELLS; i += SMALL_WG) s_start[i] = 0;
+    for (int i = t; i < nblocks * IBLOCK; i += SMALL_WG) s_atom[i] = -1;
+    __syncthreads();
+    constexpr int PER = SMALL_UNITS / SMALL_WG, CPT = SMALL_CELLS / SMALL_WG;
+    int key[PER], number[PER];
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+        const int u = t + k * SMALL_WG;
+        key[k] = -1;
+        if (u < nunits) {
+            key[k] = cell_key(unit_atoms[unit_ptr[u]], pos, sys[0], cell_rank) - sys[0].cell_off;
+            number[k] = atomicAdd(&s_start[key[k]], 1);
+        }
+    }
+    __syncthreads();
+    int count[CPT], sum = 0;
+#pragma unroll
+    for (int k = 0; k < CPT; ++k) {
+        count[k] = s_start[CPT * t + k];
+        sum += count[k];
+    }
+    int before = sum;
+    for (int off = 1; off < 64; off <<= 1) {
+        const int v = __shfl_up(before, off, 64);
+        if (lane >= off) before += v;
+    }
+    if (lane == 63) s_wave[t >> 6] = before;
+    __syncthreads();
+    before -= sum;
+    for (int w = 0; w < (t >> 6); ++w) before += s_wave[w];
+#pragma unroll
+    for (int k = 0; k < CPT; ++k) {
+        s_start[CPT * t + k] = before;
+        before += count[k];
+    }
+    if (t == SMALL_WG - 1) s_start[SMALL_CELLS] = before;
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < PER; ++k)
+        if (key[k] >= 0) s_list[s_start[key[k]] + number[k]] = (unsigned short)(t + k * SMALL_WG);
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+        if (key[k] < 0) continue;
+        const int u = t + k * SMALL_WG, lo = s_start[key[k]], hi = s_start[key[k] + 1];
+        int p = lo;
+        for (int i = lo; i < hi; ++i) p += s_list[i] < u ? 1 : 0;
+        place_unit(p, u, nullptr, uniform, unit_ptr, unit_atoms, unit_pos, unit_sys, sys, excl_ptr, excl_idx, closed,
+                   sorted_atom, atom_slot, excl_range, flag);
+        const int first = unit_ptr[u];
+        for (int i = 0; i < uniform; ++i) s_atom[p * uniform + i] = unit_atoms[first + i];
+    }
+    __syncthreads();
+    for (int b = 2 * (t >> 6); b < nblocks; b += 2 * (SMALL_WG / 64)) {
+        const int blk = b + (lane >> 5);
+        const bool valid = blk < nblocks;
+        const int a = valid ? s_atom[blk * IBLOCK + (lane & 31)] : -1, ref = valid ? s_atom[blk * IBLOCK] : 0;
+        block_bounds_of(blk, valid, a, ref, sys[0].box, pos, reach, center, half, minimg, pos_build, slot_pos);
     }
 }
 
@@ -1075,18 +1164,8 @@ void nlist_check(NlistDev& nl, const double* pos, int force, hipStream_t s) {
     OMM_HIP(hipGetLastError());
 }
 
-void nlist_build(NlistDev& nl, const double* pos, const SysInfo* sys_dev, unsigned* status, hipStream_t s,
-                 bool forced) {
-    // Forced builds (the first step of every captured graph) run
-    // unconditionally; otherwise every kernel exits early unless the
-    // displacement check asked for a rebuild.
-    const int* flag = forced ? nl.one.p : nl.flag.p;
-    // Each kernel of the chain is a graph node that costs a few microseconds
-    // even when it exits at once, so steps without a rebuild pay for the
-    // chain's length: the cell-count scan rides on the key kernel and, for a
-    // single system, the sort of uniform units on their placement.  (Batches
-    // rebuild some replica on most steps, and there one thread per unit
-    // places faster than one thread per cell.)
+// The units in order of their cells, placed at their slots.
+static void build_order(NlistDev& nl, const double* pos, const SysInfo* sys_dev, const int* flag, hipStream_t s) {
     if (nl.ncells <= SCAN_SINGLE_MAX) {
         hipLaunchKernelGGL(k_unit_keys_scan, dim3(blocks_for(nl.nunits, SCAN_WG)), dim3(SCAN_WG), 0, s, pos,
                            nl.unit_ptr.p, nl.unit_atoms.p, nl.unit_sys.p, nl.nunits, sys_dev, nl.cell_rank.p,
@@ -1116,14 +1195,40 @@ void nlist_build(NlistDev& nl, const double* pos, const SysInfo* sys_dev, unsign
                            nl.unit_sys.p, sys_dev, nl.excl_ptr.p, nl.excl_idx.p, nl.closed, nl.nunits,
                            nl.sorted_atom.p, nl.atom_slot.p, nl.excl_range.p, flag);
     }
+}
+
+void nlist_build(NlistDev& nl, const double* pos, const SysInfo* sys_dev, unsigned* status, hipStream_t s,
+                 bool forced) {
+    // Forced builds (the first step of every captured graph) run
+    // unconditionally; otherwise every kernel exits early unless the
+    // displacement check asked for a rebuild.
+    const int* flag = forced ? nl.one.p : nl.flag.p;
+    // Each kernel of the chain is a graph node that costs a few microseconds
+    // even when it exits at once, so steps without a rebuild pay for the
+    // chain's length: the cell-count scan rides on the key kernel and, for a
+    // single system, the sort of uniform units on their placement.  (Batches
+    // rebuild some replica on most steps, and there one thread per unit
+    // places faster than one thread per cell.)
+    const double reach = nl.cutoff + nl.skin;
+    const bool small = nl.uniform > 0 && nl.nsys == 1 && nl.nunits <= SMALL_UNITS && nl.ncells <= SMALL_CELLS &&
+                       nl.nslots <= SMALL_SLOTS;
+    if (small) {
+        hipLaunchKernelGGL(k_list_small, dim3(1), dim3(SMALL_WG), 0, s, pos, nl.unit_ptr.p, nl.unit_atoms.p,
+                           nl.unit_pos.p, nl.unit_sys.p, nl.nunits, nl.uniform, sys_dev, nl.cell_rank.p, nl.ncells,
+                           nl.excl_ptr.p, nl.excl_idx.p, nl.closed, nl.sorted_atom.p, nl.atom_slot.p, nl.excl_range.p,
+                           nl.nblocks, reach, nl.block_center.p, nl.block_half.p, nl.block_minimg.p, nl.pos_build.p,
+                           nl.slot_pos.p, nl.ntasks.p, flag);
+    } else {
+        build_order(nl, pos, sys_dev, flag, s);
+    }
     if (!nl.closed)
         hipLaunchKernelGGL(k_excl_range, dim3(blocks_for(nl.nslots, 256)), dim3(256), 0, s, nl.sorted_atom.p,
                            nl.atom_slot.p, nl.excl_ptr.p, nl.excl_idx.p, nl.block_sys.p, nl.nslots,
                            nl.excl_range.p, flag);
-    double reach = nl.cutoff + nl.skin;
-    hipLaunchKernelGGL(k_block_bounds, dim3(blocks_for(nl.nblocks, 2)), dim3(64), 0, s, pos, nl.sorted_atom.p,
-                       nl.nblocks, nl.block_sys.p, sys_dev, reach, nl.block_center.p, nl.block_half.p,
-                       nl.block_minimg.p, nl.pos_build.p, nl.slot_pos.p, nl.ntasks.p, flag);
+    if (!small)
+        hipLaunchKernelGGL(k_block_bounds, dim3(blocks_for(nl.nblocks, 2)), dim3(64), 0, s, pos, nl.sorted_atom.p,
+                           nl.nblocks, nl.block_sys.p, sys_dev, reach, nl.block_center.p, nl.block_half.p,
+                           nl.block_minimg.p, nl.pos_build.p, nl.slot_pos.p, nl.ntasks.p, flag);
     if (nl.use_super)
         hipLaunchKernelGGL(k_super_bounds, dim3(nl.nsuper), dim3(64), 0, s, nl.nsuper, nl.super_off.p, nl.nsys,
                            sys_dev, nl.block_center.p, nl.block_half.p, nl.super_center.p, nl.super_half.p, flag);
