@@ -51,6 +51,7 @@ struct NlistDev {
     int generation = 0;  // advanced by every nlist_setup (slot layout changes)
     int natoms = 0, nslots = 0, nblocks = 0, nclusters = 0, nchunks = 0, cap = 0, nunits = 0, ncells = 0;
     int uniform = 0;  // atoms per unit when all units are the same size, else 0
+    int max_units = 0, max_cells = 0;  // of a system (max_units: uniform units only)
     int closed = 0;   // every exception pair lies inside one unit
     int tpt = 4;  // tiles of one cluster per pair-kernel task (see tiles_per_task)
     double cutoff = 0, skin = 0;

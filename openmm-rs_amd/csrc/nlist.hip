@@ -478,42 +478,32 @@ __global__ __launch_bounds__(64) void k_block_bounds(const double* __restrict__ 
     block_bounds_of(blk, valid, a, ref, sys[si].box, pos, reach, center, half, minimg, pos_build, slot_pos);
 }
 
-// The whole chain up to the block bounds in one workgroup, for one system of
-// uniform units of at most SMALL_UNITS units, SMALL_CELLS cells and SMALL_SLOTS
-// slots: keys, cell counts, their scan, the scatter, the rank within the cell
-// and the placement with the same results as the launches above, from LDS.  One
-// launch instead of four, also on the many steps without a build: an evaluation
-// of 900 atoms 250 us -> 235, MD 51 us per step -> 49.
-constexpr int SMALL_WG = 1024, SMALL_UNITS = 2048, SMALL_CELLS = 4096, SMALL_SLOTS = 8192;
+// Order of a system's units by one workgroup, from LDS: keys, cell counts, their
+// scan, the scatter and the rank within the cell (by index), for at most
+// PER * WG units and ORDER_CELLS cells.  place(u, p): unit u (from the
+// system's first) has place p.
+constexpr int ORDER_CELLS = 4096;
 
-__global__ __launch_bounds__(SMALL_WG) void k_list_small(
-    const double* __restrict__ pos, const int* __restrict__ unit_ptr, const int* __restrict__ unit_atoms,
-    const int* __restrict__ unit_pos, const int* __restrict__ unit_sys, int nunits, int uniform,
-    const SysInfo* __restrict__ sys, const int* __restrict__ cell_rank, int ncells, const int* __restrict__ excl_ptr,
-    const int* __restrict__ excl_idx, int closed, int* sorted_atom, int* atom_slot, int2* excl_range, int nblocks,
-    double reach, double* center, float* half, int* minimg, double* pos_build, float4* slot_pos, int* ntasks,
-    const int* __restrict__ flag) {
-    if (!flag[0]) return;
-    __shared__ int s_start[SMALL_CELLS + 1], s_atom[SMALL_SLOTS], s_wave[SMALL_WG / 64];
-    __shared__ unsigned short s_list[SMALL_UNITS];
+template <int WG, int PER, class Place>
+__device__ __forceinline__ void order_system(const double* __restrict__ pos, const int* __restrict__ unit_ptr,
+                                             const int* __restrict__ unit_atoms, int first_unit, int nunits,
+                                             const SysInfo& S, const int* __restrict__ cell_rank, Place place) {
+    __shared__ int s_start[ORDER_CELLS + 1], s_wave[WG / 64];
+    __shared__ unsigned short s_list[PER * WG];
     const int t = threadIdx.x, lane = t & 63;
-    if (t == 0) ntasks[0] = 0;  // k_clist appends the tasks anew
-    if (!flag[1]) return;
-    for (int i = t; i <= SMALL_CELLS; i += SMALL_WG) s_start[i] = 0;
-    for (int i = t; i < nblocks * IBLOCK; i += SMALL_WG) s_atom[i] = -1;
-    __syncthreads();
-    constexpr int PER = SMALL_UNITS / SMALL_WG, CPT = SMALL_CELLS / SMALL_WG;
+    for (int i = t; i <= ORDER_CELLS; i += WG) s_start[i] = 0;
     int key[PER], number[PER];
 #pragma unroll
     for (int k = 0; k < PER; ++k) {
-        const int u = t + k * SMALL_WG;
-        key[k] = -1;
-        if (u < nunits) {
-            key[k] = cell_key(unit_atoms[unit_ptr[u]], pos, sys[0], cell_rank) - sys[0].cell_off;
-            number[k] = atomicAdd(&s_start[key[k]], 1);
-        }
+        const int u = min(t + k * WG, nunits - 1);
+        key[k] = cell_key(unit_atoms[unit_ptr[first_unit + u]], pos, S, cell_rank) - S.cell_off;
     }
     __syncthreads();
+#pragma unroll
+    for (int k = 0; k < PER; ++k)
+        if (t + k * WG < nunits) number[k] = atomicAdd(&s_start[key[k]], 1);
+    __syncthreads();
+    constexpr int CPT = ORDER_CELLS / WG;
     int count[CPT], sum = 0;
 #pragma unroll
     for (int k = 0; k < CPT; ++k) {
@@ -534,23 +524,49 @@ __global__ __launch_bounds__(SMALL_WG) void k_list_small(
         s_start[CPT * t + k] = before;
         before += count[k];
     }
-    if (t == SMALL_WG - 1) s_start[SMALL_CELLS] = before;
+    if (t == WG - 1) s_start[ORDER_CELLS] = before;
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < PER; ++k)
-        if (key[k] >= 0) s_list[s_start[key[k]] + number[k]] = (unsigned short)(t + k * SMALL_WG);
+        if (t + k * WG < nunits) s_list[s_start[key[k]] + number[k]] = (unsigned short)(t + k * WG);
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < PER; ++k) {
-        if (key[k] < 0) continue;
-        const int u = t + k * SMALL_WG, lo = s_start[key[k]], hi = s_start[key[k] + 1];
+        const int u = t + k * WG;
+        if (u >= nunits) continue;
+        const int lo = s_start[key[k]], hi = s_start[key[k] + 1];
         int p = lo;
         for (int i = lo; i < hi; ++i) p += s_list[i] < u ? 1 : 0;
+        place(u, p);
+    }
+}
+
+// One system of uniform units of at most SMALL_UNITS units and SMALL_SLOTS
+// slots: its order, its placement and its bounds by one workgroup.  One launch
+// instead of four, also on the many steps without a build: an evaluation of 900
+// atoms 250 us -> 235, MD 51 us per step -> 49.
+constexpr int SMALL_WG = 1024, SMALL_UNITS = 2048, SMALL_SLOTS = 8192;
+
+__global__ __launch_bounds__(SMALL_WG) void k_list_small(
+    const double* __restrict__ pos, const int* __restrict__ unit_ptr, const int* __restrict__ unit_atoms,
+    const int* __restrict__ unit_pos, const int* __restrict__ unit_sys, int nunits, int uniform,
+    const SysInfo* __restrict__ sys, const int* __restrict__ cell_rank, const int* __restrict__ excl_ptr,
+    const int* __restrict__ excl_idx, int closed, int* sorted_atom, int* atom_slot, int2* excl_range, int nblocks,
+    double reach, double* center, float* half, int* minimg, double* pos_build, float4* slot_pos, int* ntasks,
+    const int* __restrict__ flag) {
+    if (!flag[0]) return;
+    __shared__ int s_atom[SMALL_SLOTS];
+    const int t = threadIdx.x, lane = t & 63;
+    if (t == 0) ntasks[0] = 0;  // k_clist appends the tasks anew
+    if (!flag[1]) return;
+    for (int i = t; i < nblocks * IBLOCK; i += SMALL_WG) s_atom[i] = -1;
+    constexpr int PER = SMALL_UNITS / SMALL_WG;
+    order_system<SMALL_WG, PER>(pos, unit_ptr, unit_atoms, 0, nunits, sys[0], cell_rank, [&](int u, int p) {
         place_unit(p, u, nullptr, uniform, unit_ptr, unit_atoms, unit_pos, unit_sys, sys, excl_ptr, excl_idx, closed,
                    sorted_atom, atom_slot, excl_range, flag);
         const int first = unit_ptr[u];
         for (int i = 0; i < uniform; ++i) s_atom[p * uniform + i] = unit_atoms[first + i];
-    }
+    });
     __syncthreads();
     for (int b = 2 * (t >> 6); b < nblocks; b += 2 * (SMALL_WG / 64)) {
         const int blk = b + (lane >> 5);
@@ -558,6 +574,65 @@ __global__ __launch_bounds__(SMALL_WG) void k_list_small(
         const int a = valid ? s_atom[blk * IBLOCK + (lane & 31)] : -1, ref = valid ? s_atom[blk * IBLOCK] : 0;
         block_bounds_of(blk, valid, a, ref, sys[0].box, pos, reach, center, half, minimg, pos_build, slot_pos);
     }
+}
+
+// Systems of uniform units of at most ORDER_UNITS units and ORDER_CELLS cells
+// each: a workgroup orders each flagged system, and k_place_bounds places its
+// atoms, a slot per lane, and takes the blocks' bounds.  An unflagged system
+// keeps its order and costs nothing.  Two launches instead of four to nine, and
+// no scan over every system's cells: with k_clist's share of the unflagged
+// systems' tasks, MD of 24 replicas (66,000 atoms) 263 us per step -> 241, of 64
+// (476,000 atoms) 1,306 -> 1,225.  Workgroups of 1,024 wait longer for a free
+// compute unit beside the mesh (64 replicas 1,245), 256 are no faster.
+constexpr int ORDER_WG = 512, ORDER_UNITS = 8192;
+
+__global__ __launch_bounds__(ORDER_WG) void k_order_units(const double* __restrict__ pos,
+                                                          const int* __restrict__ unit_ptr,
+                                                          const int* __restrict__ unit_atoms, int uniform,
+                                                          const SysInfo* __restrict__ sys,
+                                                          const int* __restrict__ cell_rank, int* sorted_units,
+                                                          const int* __restrict__ flag) {
+    if (!flag[0] || !flag[1 + blockIdx.x]) return;
+    const SysInfo& S = sys[blockIdx.x];
+    const int first = S.atom_off / uniform;
+    order_system<ORDER_WG, ORDER_UNITS / ORDER_WG>(pos, unit_ptr, unit_atoms, first, S.n / uniform, S, cell_rank,
+                                                   [&](int u, int p) { sorted_units[first + p] = first + u; });
+}
+
+// Two blocks per wave, as k_block_bounds.
+__global__ __launch_bounds__(64) void k_place_bounds(
+    const double* __restrict__ pos, const int* __restrict__ sorted_units, int uniform,
+    const int* __restrict__ unit_ptr, const int* __restrict__ unit_atoms, const int* __restrict__ unit_pos,
+    const int* __restrict__ excl_ptr, const int* __restrict__ excl_idx, int closed, int* sorted_atom, int* atom_slot,
+    int2* excl_range, int nblocks, const int* __restrict__ block_sys, const SysInfo* __restrict__ sys, double reach,
+    double* center, float* half, int* minimg, double* pos_build, float4* slot_pos, int* ntasks,
+    const int* __restrict__ flag) {
+    if (!flag[0]) return;
+    if (blockIdx.x == 0 && threadIdx.x == 0) ntasks[0] = 0;  // k_clist appends the tasks anew
+    const int lane = threadIdx.x, blk = blockIdx.x * 2 + (lane >> 5);
+    const int si = blk < nblocks ? block_sys[blk] : 0;
+    const bool valid = blk < nblocks && flag[1 + si];  // unflagged systems keep their slots and bounds
+    const SysInfo& S = sys[si];
+    const int slot = blk * IBLOCK + (lane & 31), local = slot - S.slot_off;
+    int a = -1;
+    if (valid && local < S.n) {
+        const int p = local / uniform, k = local - p * uniform;
+        const int first = unit_ptr[sorted_units[S.atom_off / uniform + p]];
+        a = unit_atoms[first + k];
+        sorted_atom[slot] = a;
+        atom_slot[a] = slot;
+        if (closed) {
+            int lo = INT_MAX, hi = -1;
+            for (int e = excl_ptr[a]; e < excl_ptr[a + 1]; ++e) {
+                const int x = slot - k + unit_pos[excl_idx[e]];
+                lo = min(lo, x);
+                hi = max(hi, x);
+            }
+            excl_range[slot] = make_int2(lo, hi);
+        }
+    }
+    const int ref = __shfl(a, lane & 32, 64);  // the first slot of a block holds an atom
+    block_bounds_of(blk, valid, a, valid ? ref : 0, S.box, pos, reach, center, half, minimg, pos_build, slot_pos);
 }
 
 // Superblock bounds of flagged systems, one wave per superblock.
@@ -590,7 +665,6 @@ __global__ __launch_bounds__(64) void k_super_bounds(int nsuper, const int* __re
 // tile (their order in the table does not matter, as forces are fixed-point
 // sums; one atomic per workgroup reserves the runs of its clusters).  The
 // atoms of four passing blocks are loaded together, so their loads overlap.
-// Unflagged systems keep their lists and only append their tasks.
 // Exclusion data the list build reads to mark excluded pairs per entry.
 struct ExclLookup {
     const int* atom_slot;
@@ -697,10 +771,13 @@ __device__ __forceinline__ int nth_set_bit(unsigned long long m, int k) {
 }
 
 // Clusters (one per wave) per workgroup of k_clist: two for a single system
-// (small workgroups spread over every compute unit), sixteen for batches,
-// where the workgroups of unflagged systems only append their tasks and one
-// task reservation per workgroup keeps the atomics on the counter few.
-constexpr int CLIST_WAVES_SINGLE = 2, CLIST_WAVES_BATCH = 16;
+// (small workgroups spread over every compute unit), CLIST_WAVES_BATCH for
+// batches, whose first nkept workgroups append the tasks of the unflagged
+// systems, a cluster per thread (one reservation on the counter, 12 ns each, for
+// 64 CLIST_WAVES_BATCH clusters), while the others leave those at once.
+// Workgroups of four: 64 replicas 1,245 us per step, of eight 1,285, of sixteen
+// that append as well 1,306.
+constexpr int CLIST_WAVES_SINGLE = 2, CLIST_WAVES_BATCH = 4;
 
 template <int W>
 __global__ __launch_bounds__(64 * W) void k_clist(
@@ -710,19 +787,42 @@ __global__ __launch_bounds__(64 * W) void k_clist(
     const float* __restrict__ super_half, const int* __restrict__ atom_slot, const int* __restrict__ excl_ptr,
     const int* __restrict__ excl_idx, const int2* __restrict__ excl_range, const int* __restrict__ minimg,
     const float4* __restrict__ slot_pos, double reach, int cap, int nclusters, int tpt, int2* clist,
-    unsigned char* clist_ex, int* ccount, int* tasks, int* ntasks, unsigned* status, const int* flag) {
+    unsigned char* clist_ex, int* ccount, int* tasks, int* ntasks, unsigned* status, const int* flag, int nkept) {
     __shared__ int s_runs[W];
     __shared__ int s_base;
     if (!flag[0]) return;
     const int wave = threadIdx.x / 64;
     const int lane = threadIdx.x % 64;
-    const int C = blockIdx.x * W + wave;
+    auto runs_of = [&](int entries) { return ((entries + JTILE - 1) / JTILE + tpt - 1) / tpt; };
+    if ((int)blockIdx.x < nkept) {
+        const int C = blockIdx.x * (64 * W) + threadIdx.x;
+        int runs = 0;
+        if (C < nclusters && !flag[1 + block_sys[C / CPB]]) runs = runs_of(ccount[C]);
+        int upto = runs;
+        for (int off = 1; off < 64; off <<= 1) {
+            const int v = __shfl_up(upto, off, 64);
+            if (lane >= off) upto += v;
+        }
+        if (lane == 63) s_runs[wave] = upto;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            int all = 0;
+            for (int w = 0; w < W; ++w) all += s_runs[w];
+            s_base = all > 0 ? atomicAdd(ntasks, all) : 0;
+        }
+        __syncthreads();
+        int at = s_base + upto - runs;
+        for (int w = 0; w < wave; ++w) at += s_runs[w];
+        for (int k = 0; k < runs; ++k) tasks[at + k] = (C << 8) | (k * tpt);
+        return;
+    }
+    const int C = ((int)blockIdx.x - nkept) * W + wave;
     const int I = C / CPB;
     const int si = C < nclusters ? block_sys[I] : 0;
     const int first = C * CLUSTER;  // the cluster's first slot
     int count = 0;
     if (C < nclusters && !flag[1 + si]) {
-        count = ccount[C];  // unflagged systems keep their lists
+        // Unflagged systems keep their lists.
     } else if (C < nclusters && sorted_atom[first] >= 0) {
         const SysInfo& S = sys[si];
         const Box& b = S.box;
@@ -890,7 +990,7 @@ __global__ __launch_bounds__(64 * W) void k_clist(
     } else if (C < nclusters) {
         if (lane == 0) ccount[C] = 0;  // a cluster of padding only
     }
-    const int runs = ((count + JTILE - 1) / JTILE + tpt - 1) / tpt;
+    const int runs = runs_of(count);
     if (lane == 0) s_runs[wave] = runs;
     __syncthreads();
     if (threadIdx.x == 0) {
@@ -971,6 +1071,7 @@ void nlist_setup(NlistDev& nl, const std::vector<NlistSystem>& systems, std::vec
     int natoms = 0, nblocks = 0, nchunks = 0, ncells = 0, max_npad = 0;
     nl.uniform = -1;
     nl.closed = 1;
+    nl.max_units = nl.max_cells = 0;
     for (int si = 0; si < nsys; ++si) {
         const NlistSystem& sy = systems[si];
         const int n = sy.n;
@@ -1053,6 +1154,7 @@ void nlist_setup(NlistDev& nl, const std::vector<NlistSystem>& systems, std::vec
         rank_all.insert(rank_all.end(), rank.begin(), rank.end());
         S.cell_off = ncells;
         ncells += nc;
+        nl.max_cells = std::max(nl.max_cells, nc);
         // Slots, blocks and PME chunks; the identity layout until the first build.
         const int nb = (n + IBLOCK - 1) / IBLOCK;
         S.atom_off = natoms;
@@ -1078,6 +1180,7 @@ void nlist_setup(NlistDev& nl, const std::vector<NlistSystem>& systems, std::vec
         max_npad = std::max(max_npad, nb * IBLOCK);
     }
     if (nl.uniform < 0) nl.uniform = 0;
+    for (int si = 0; si < nsys && nl.uniform > 0; ++si) nl.max_units = std::max(nl.max_units, sys[si].n / nl.uniform);
     nl.natoms = natoms;
     nl.nblocks = nblocks;
     nl.nclusters = nblocks * CPB;
@@ -1210,34 +1313,42 @@ void nlist_build(NlistDev& nl, const double* pos, const SysInfo* sys_dev, unsign
     // rebuild some replica on most steps, and there one thread per unit
     // places faster than one thread per cell.)
     const double reach = nl.cutoff + nl.skin;
-    const bool small = nl.uniform > 0 && nl.nsys == 1 && nl.nunits <= SMALL_UNITS && nl.ncells <= SMALL_CELLS &&
-                       nl.nslots <= SMALL_SLOTS;
-    if (small) {
+    const bool by_system = nl.uniform > 0 && nl.max_units <= ORDER_UNITS && nl.max_cells <= ORDER_CELLS;
+    if (by_system && nl.nsys == 1 && nl.nunits <= SMALL_UNITS && nl.nslots <= SMALL_SLOTS) {
         hipLaunchKernelGGL(k_list_small, dim3(1), dim3(SMALL_WG), 0, s, pos, nl.unit_ptr.p, nl.unit_atoms.p,
-                           nl.unit_pos.p, nl.unit_sys.p, nl.nunits, nl.uniform, sys_dev, nl.cell_rank.p, nl.ncells,
+                           nl.unit_pos.p, nl.unit_sys.p, nl.nunits, nl.uniform, sys_dev, nl.cell_rank.p,
                            nl.excl_ptr.p, nl.excl_idx.p, nl.closed, nl.sorted_atom.p, nl.atom_slot.p, nl.excl_range.p,
                            nl.nblocks, reach, nl.block_center.p, nl.block_half.p, nl.block_minimg.p, nl.pos_build.p,
                            nl.slot_pos.p, nl.ntasks.p, flag);
+    } else if (by_system) {
+        hipLaunchKernelGGL(k_order_units, dim3(nl.nsys), dim3(ORDER_WG), 0, s, pos, nl.unit_ptr.p, nl.unit_atoms.p,
+                           nl.uniform, sys_dev, nl.cell_rank.p, nl.sorted_units.p, flag);
+        hipLaunchKernelGGL(k_place_bounds, dim3(blocks_for(nl.nblocks, 2)), dim3(64), 0, s, pos, nl.sorted_units.p,
+                           nl.uniform, nl.unit_ptr.p, nl.unit_atoms.p, nl.unit_pos.p, nl.excl_ptr.p, nl.excl_idx.p,
+                           nl.closed, nl.sorted_atom.p, nl.atom_slot.p, nl.excl_range.p, nl.nblocks, nl.block_sys.p,
+                           sys_dev, reach, nl.block_center.p, nl.block_half.p, nl.block_minimg.p, nl.pos_build.p,
+                           nl.slot_pos.p, nl.ntasks.p, flag);
     } else {
         build_order(nl, pos, sys_dev, flag, s);
+        hipLaunchKernelGGL(k_block_bounds, dim3(blocks_for(nl.nblocks, 2)), dim3(64), 0, s, pos, nl.sorted_atom.p,
+                           nl.nblocks, nl.block_sys.p, sys_dev, reach, nl.block_center.p, nl.block_half.p,
+                           nl.block_minimg.p, nl.pos_build.p, nl.slot_pos.p, nl.ntasks.p, flag);
     }
     if (!nl.closed)
         hipLaunchKernelGGL(k_excl_range, dim3(blocks_for(nl.nslots, 256)), dim3(256), 0, s, nl.sorted_atom.p,
                            nl.atom_slot.p, nl.excl_ptr.p, nl.excl_idx.p, nl.block_sys.p, nl.nslots,
                            nl.excl_range.p, flag);
-    if (!small)
-        hipLaunchKernelGGL(k_block_bounds, dim3(blocks_for(nl.nblocks, 2)), dim3(64), 0, s, pos, nl.sorted_atom.p,
-                           nl.nblocks, nl.block_sys.p, sys_dev, reach, nl.block_center.p, nl.block_half.p,
-                           nl.block_minimg.p, nl.pos_build.p, nl.slot_pos.p, nl.ntasks.p, flag);
     if (nl.use_super)
         hipLaunchKernelGGL(k_super_bounds, dim3(nl.nsuper), dim3(64), 0, s, nl.nsuper, nl.super_off.p, nl.nsys,
                            sys_dev, nl.block_center.p, nl.block_half.p, nl.super_center.p, nl.super_half.p, flag);
     auto clist = [&](auto kernel, int w) {
-        hipLaunchKernelGGL(kernel, dim3(blocks_for(nl.nclusters, w)), dim3(64 * w), 0, s, pos, nl.sorted_atom.p,
+        const int kept = nl.nsys == 1 ? 0 : blocks_for(nl.nclusters, 64 * w);
+        hipLaunchKernelGGL(kernel, dim3(kept + blocks_for(nl.nclusters, w)), dim3(64 * w), 0, s, pos, nl.sorted_atom.p,
                            nl.block_sys.p, sys_dev, nl.block_center.p, nl.block_half.p, nl.super_off.p,
                            nl.super_center.p, nl.super_half.p, nl.atom_slot.p, nl.excl_ptr.p, nl.excl_idx.p,
                            nl.excl_range.p, nl.block_minimg.p, nl.slot_pos.p, reach, nl.cap, nl.nclusters, nl.tpt, nl.clist.p,
-                           nl.clist_ex.p, nl.ccount.p, nl.tasks.p, nl.ntasks.p, status, flag);
+                           nl.clist_ex.p, nl.ccount.p, nl.tasks.p, nl.ntasks.p, status, flag,
+                           kept);
     };
     if (nl.nsys == 1)
         clist(k_clist<CLIST_WAVES_SINGLE>, CLIST_WAVES_SINGLE);
