@@ -251,8 +251,9 @@ __global__ __launch_bounds__(SPREAD_THREADS) void k_spread_tiles(const int* __re
 // sum in a varying order either way).  The grid is zero at the launch (the
 // transform after the previous spread cleared every point).
 //
-// One workgroup per chunk; its four waves hold the same 64 atoms, one per lane,
-// with their weights in registers, and share the stencil's 25 rows.  Bound:
+// One workgroup per chunk; three waves take the splines and the box along one
+// axis each, then its four waves hold the same atoms, one per lane, with their
+// weights in registers, and share the stencil's 25 rows.  Bound:
 // latency at small systems, the device atomics of the box (27 points per atom at
 // 100 atoms/nm^3) at large ones.  Kept in LDS with a thread per row of an atom's
 // stencil, and with tiles for FP64 grids, it took (here): 3,000 unsorted atoms on
@@ -352,6 +353,8 @@ __global__ __launch_bounds__(ATOM_SPREAD_THREADS) void k_spread_atoms(const int*
     // The box (int32 sums at 2^-24: at most PME_CHUNK contributions of
     // |q| w <= 2 x 0.2153 per point stay below 2^31).
     __shared__ Box box[SPREAD_BOX_BYTES / sizeof(Box)];
+    __shared__ R s_w[3][5][ATOMS];
+    __shared__ int s_idx[3][ATOMS], s_at[3][ATOMS], s_org[3], s_ext[3];
     const int t = threadIdx.x, k = t & (ATOMS - 1), group = t / ATOMS;
     const int chunk = blockIdx.x / PARTS;
     int si = 0, local = chunk;
@@ -367,23 +370,41 @@ __global__ __launch_bounds__(ATOM_SPREAD_THREADS) void k_spread_atoms(const int*
     const double charge_a = charge[a0];
     const double p[3] = {pos[3 * (size_t)a0], pos[3 * (size_t)a0 + 1], pos[3 * (size_t)a0 + 2]};
     const int n[3] = {S.grid[0], S.grid[1], S.grid[2]};
-    int idx[3];
-    R w[3][5], dw[3][5];
-    stencil<R>(p, S.box, n, idx, w, dw);
     const double q = a >= 0 ? charge_a : 0.0;
     const bool on = q != 0.0;  // uncharged atoms do not spread (pme.rs:315-330)
     const unsigned long long live = __ballot(on);
     if (!live) return;  // the same in all four waves
-    // The box: offsets from the first charged atom, nearest images.
-    const int lead = __ffsll((long long)live) - 1;
-    int org[3], ext[3], at[3];
-    for (int d = 0; d < 3; ++d) {
-        const int first = __shfl(idx[d], lead, 64);
-        const int r = nearest_offset(idx[d] - first, n[d]);
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6), lead = __ffsll((long long)live) - 1;
+    if (wave < 3) {
+        // One axis per wave: the splines, and the box's origin and extent from
+        // the offsets from the first charged atom, nearest images.
+        R wd[5], dw[5];
+        const int i = stencil_axis<R>(p, S.box, wave, n[wave], wd, dw);
+        const int first = __shfl(i, lead, 64);
+        const int r = nearest_offset(i - first, n[wave]);
         const int lo = group_min<ATOMS>(on ? r : INT_MAX), hi = group_max<ATOMS>(on ? r : INT_MIN);
-        org[d] = wrap_near(first + lo, n[d]);
-        ext[d] = hi - lo + 5;
-        at[d] = r - lo;
+        if (t % 64 < ATOMS) {
+            s_at[wave][k] = r - lo;
+            s_idx[wave][k] = i;
+#pragma unroll
+            for (int j = 0; j < 5; ++j) s_w[wave][j][k] = wd[j];
+        }
+        if (t % 64 == 0) {
+            s_org[wave] = wrap_near(first + lo, n[wave]);
+            s_ext[wave] = hi - lo + 5;
+        }
+    }
+    __syncthreads();
+    int idx[3], org[3], ext[3], at[3];
+    R w[3][5];
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        idx[d] = s_idx[d][k];
+        at[d] = s_at[d][k];
+        org[d] = s_org[d];
+        ext[d] = s_ext[d];
+#pragma unroll
+        for (int j = 0; j < 5; ++j) w[d][j] = s_w[d][j][k];
     }
     G* g = grid + S.qgrid_off;
     const int e1 = ext[1], e2 = ext[2], vol = ext[0] * e1 * e2;
@@ -456,9 +477,12 @@ __global__ __launch_bounds__(256) void k_spread_direct(int natoms, const double*
     }
 }
 
-// Gather with five threads per atom (one per x plane of the stencil), atoms
-// in the spatially sorted order; the five partial gradients are combined in
-// LDS.
+// Gather with five threads per atom, one per z of the stencil, so that five
+// lanes read a row's consecutive points together (one per x plane touches five
+// times as many cache lines, which bounds the kernel); atoms in the spatially
+// sorted order.  The first three waves take the splines of one axis each, the
+// five partial gradients are combined in LDS.  300,000 atoms 45 -> 38 us, 900
+// atoms 5.0 -> 4.0 (with a plane and the whole stencil per thread before).
 constexpr int GATHER_ATOMS = PME_CHUNK;
 
 template <class R, class A>
@@ -468,62 +492,88 @@ __global__ __launch_bounds__(GATHER_ATOMS * 5) void k_gather5(const int* __restr
                                                               const double* __restrict__ charge,
                                                               const SysInfo* __restrict__ sys,
                                                               const R* __restrict__ phi, A* force, unsigned* status) {
-    __shared__ R s_g[GATHER_ATOMS][5][3];
-    const int si = find_sys(chunk_off, nsys, blockIdx.x);
+    __shared__ R s_w[3][5][GATHER_ATOMS], s_dw[3][5][GATHER_ATOMS], s_g[3][5][GATHER_ATOMS];
+    __shared__ int s_idx[3][GATHER_ATOMS], s_atom[GATHER_ATOMS];
+    __shared__ double s_q[GATHER_ATOMS];
+    int si = 0, local = blockIdx.x;
+    if (nsys > 1) {
+        si = find_sys(chunk_off, nsys, blockIdx.x);
+        local -= chunk_off[si];
+    }
     const SysInfo& S = sys[si];
+    const Box& b = S.box;
     const int nx = S.grid[0], ny = S.grid[1], nz = S.grid[2];
     phi += S.qgrid_off;
     const int t = threadIdx.x;
-    const int k = t / 5, ix = t - k * 5;
-    const int slot = S.slot_off + (blockIdx.x - S.chunk_off) * GATHER_ATOMS + k;
-    const int a = slot < S.slot_off + S.nblocks * IBLOCK ? order[slot] : -1;
-    const double q = a >= 0 ? charge[a] : 0.0;
-    const Box& b = S.box;
-    R g0 = 0, g1 = 0, g2 = 0;
-    if (q != 0.0) {
-        const int dims[3] = {nx, ny, nz};
-        int idx[3];
-        R w[3][5], dw[3][5];
-        stencil<R>(pos + 3 * a, b, dims, idx, w, dw);
-        int gx = idx[0] + ix;
-        if (gx >= nx) gx -= nx;
-        int zz[5];
-        for (int iz = 0; iz < 5; ++iz) {
-            zz[iz] = idx[2] + iz;
-            if (zz[iz] >= nz) zz[iz] -= nz;
+    if (t < 3 * GATHER_ATOMS) {
+        const int k = t & (GATHER_ATOMS - 1), d = __builtin_amdgcn_readfirstlane(t / GATHER_ATOMS);
+        const int slot = S.slot_off + local * GATHER_ATOMS + k, end = S.slot_off + S.nblocks * IBLOCK;
+        const int listed = order[min(slot, end - 1)];
+        const int a = slot < end ? listed : -1, a0 = max(a, 0);
+        const double p[3] = {pos[3 * (size_t)a0], pos[3 * (size_t)a0 + 1], pos[3 * (size_t)a0 + 2]};
+        if (d == 0) {
+            const double qa = charge[a0];
+            s_atom[k] = a0;
+            s_q[k] = a >= 0 ? qa : 0.0;
         }
-        for (int iy = 0; iy < 5; ++iy) {
-            int gy = idx[1] + iy;
-            if (gy >= ny) gy -= ny;
-            const R wxy = w[0][ix] * w[1][iy];
-            const R d0 = dw[0][ix] * w[1][iy];
-            const R d1 = w[0][ix] * dw[1][iy];
-            const R* row = phi + ((size_t)gx * ny + gy) * nz;
-            for (int iz = 0; iz < 5; ++iz) {
-                const R p = row[zz[iz]];
-                g0 += p * d0 * w[2][iz];
-                g1 += p * d1 * w[2][iz];
-                g2 += p * wxy * dw[2][iz];
-            }
+        R w[5], dw[5];
+        s_idx[d][k] = stencil_axis<R>(p, b, d, S.grid[d], w, dw);
+#pragma unroll
+        for (int j = 0; j < 5; ++j) {
+            s_w[d][j][k] = w[j];
+            s_dw[d][j][k] = dw[j];
         }
     }
-    s_g[k][ix][0] = g0;
-    s_g[k][ix][1] = g1;
-    s_g[k][ix][2] = g2;
     __syncthreads();
-    if (ix == 0 && q != 0.0) {
-        R G0 = 0, G1 = 0, G2 = 0;
-        for (int m = 0; m < 5; ++m) {
-            G0 += s_g[k][m][0];
-            G1 += s_g[k][m][1];
-            G2 += s_g[k][m][2];
+    const int k = t / 5, iz = t - k * 5;
+    const double q = s_q[k];
+    if (q != 0.0) {
+        R wy[5], dwy[5];
+        int row[5];
+#pragma unroll
+        for (int iy = 0; iy < 5; ++iy) {
+            wy[iy] = s_w[1][iy][k];
+            dwy[iy] = s_dw[1][iy][k];
+            int gy = s_idx[1][k] + iy;
+            if (gy >= ny) gy -= ny;
+            row[iy] = gy * nz;
         }
+        int gz = s_idx[2][k] + iz;
+        if (gz >= nz) gz -= nz;
+        const int gx0 = s_idx[0][k];
+        const R* column = phi + gz;
+        R s00 = 0, s10 = 0, s01 = 0;  // sums of phi w_x w_y, phi w'_x w_y, phi w_x w'_y
+#pragma unroll
+        for (int ix = 0; ix < 5; ++ix) {
+            int gx = gx0 + ix;
+            if (gx >= nx) gx -= nx;
+            const R* plane = column + (size_t)gx * ny * nz;
+            const R wx = s_w[0][ix][k], dwx = s_dw[0][ix][k];
+            R r0 = 0, r1 = 0;
+#pragma unroll
+            for (int iy = 0; iy < 5; ++iy) {
+                const R v = plane[row[iy]];
+                r0 += v * wy[iy];
+                r1 += v * dwy[iy];
+            }
+            s00 += wx * r0;
+            s10 += dwx * r0;
+            s01 += wx * r1;
+        }
+        const R wz = s_w[2][iz][k], dwz = s_dw[2][iz][k];
+        s_g[0][iz][k] = s10 * wz;
+        s_g[1][iz][k] = s01 * wz;
+        s_g[2][iz][k] = s00 * dwz;
+    }
+    __syncthreads();
+    if (iz < 3 && q != 0.0) {
+        R G[3] = {0, 0, 0};
+        for (int d = 0; d < 3; ++d)
+            for (int m = 0; m < 5; ++m) G[d] += s_g[d][m][k];
         // pme.rs:417-422
-        for (int c = 0; c < 3; ++c) {
-            double s = (double)G0 * nx * b.recip[0 * 3 + c] + (double)G1 * ny * b.recip[1 * 3 + c] +
-                       (double)G2 * nz * b.recip[2 * 3 + c];
-            acc_add(force + 3 * a + c, -q * s, FORCE_SCALE, status);
-        }
+        const double s = (double)G[0] * nx * b.recip[0 * 3 + iz] + (double)G[1] * ny * b.recip[1 * 3 + iz] +
+                         (double)G[2] * nz * b.recip[2 * 3 + iz];
+        acc_add(force + 3 * (size_t)s_atom[k] + iz, -q * s, FORCE_SCALE, status);
     }
 }
 
