@@ -263,7 +263,7 @@ omm_status omm_pme_destroy(omm_pme* pme);
  * memory is a static FP64 complex grid of 64^3 points (4 MiB) per device,
  * held until the process ends: grids above 64 points on an axis are rejected
  * with OMM_ERR_INVALID.  Every call on a device shares that grid (each call
- * clears it first), so calls that overlap on one device, from other streams
+ * overwrites it), so calls that overlap on one device, from other streams
  * or threads, race.  An index outside [0, n) sets its derivative to NaN. */
 omm_status omm_pme_charge_derivatives_noalloc(int32_t num_particles, const double* pos, const double* charges,
                                               const double* box, double alpha, const int32_t grid[3],

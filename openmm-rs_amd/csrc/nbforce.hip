@@ -1331,8 +1331,10 @@ double NbOperator::mesh_charges(const double* pos, const double* box, double alp
     for (int attempt = 0; attempt < 8; ++attempt) {
         hipLaunchKernelGGL(k_mesh_begin, dim3((3 * n + 255) / 256), dim3(256), 0, s, n, in, pos_dev_.p, mesh_q_.p,
                            force_d_.p, energy_d_.p, status_.p);
+        pme_.unsorted = true;  // these positions have no list
         pme_run(pme_, MESH_F64, nl_, pos_dev_.p, mesh_q_.p, sys_dev_.p, nullptr, force_d_.p, nullptr, energy_d_.p,
                 status_.p, s, phases);
+        pme_.unsorted = false;
         // The potentials or the forces go straight to page-locked memory.
         if (count > 0) pme_potential_at(pme_, sys_dev_.p, pos_dev_.p, mesh_atoms_.p, count, out, s);
         const size_t n3 = count > 0 ? 0 : 3 * (size_t)n;

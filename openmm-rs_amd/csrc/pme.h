@@ -52,6 +52,9 @@ struct PmeDev {
     // Atom-owned spread (chunks of sorted atoms summed in LDS boxes) instead
     // of the tile-owned one; both write the same bits.
     bool spread_atoms = false;
+    // One system whose atoms no list has ordered (FP64 grids): a plane per workgroup.
+    bool unsorted = false;
+    int planes = 0, plane_points = 0;
     size_t fft_shmem[2][3] = {};  // dynamic LDS per axis
     // Matrix-core passes (dft.h), for the systems of dft_system: workgroup
     // prefix tables of the three passes per precision (the staged passes'

@@ -42,6 +42,20 @@ __device__ __forceinline__ void spline5(R f, R w[5], R dw[5]) {
     w[0] *= ((R)1 - f) / (R)4;
 }
 
+// w[i] for an i known at run time, without an indexed register.
+template <class R>
+__device__ __forceinline__ R pick(const R w[5], int i) {
+    return i == 0 ? w[0] : (i == 1 ? w[1] : (i == 2 ? w[2] : (i == 3 ? w[3] : w[4])));
+}
+
+// The base index alone, as stencil_axis takes it.
+__device__ __forceinline__ int stencil_base(const double p[3], const Box& b, int d, int n) {
+#pragma clang fp contract(off)
+    const double f = fma(p[2], b.recip[d * 3 + 2], fma(p[1], b.recip[d * 3 + 1], p[0] * b.recip[d * 3]));
+    const int i = (int)floor((f - floor(f)) * (double)n);
+    return i < n ? i : 0;
+}
+
 // pme.rs:201-218: base index and spline of the fractional grid coordinate along
 // axis d of a grid of n points.
 template <class R>
