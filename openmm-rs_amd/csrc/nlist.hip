@@ -544,8 +544,9 @@ __device__ __forceinline__ void order_system(const double* __restrict__ pos, con
 // One system of uniform units of at most SMALL_UNITS units and SMALL_SLOTS
 // slots: its order, its placement and its bounds by one workgroup.  One launch
 // instead of four, also on the many steps without a build: an evaluation of 900
-// atoms 250 us -> 235, MD 51 us per step -> 49.
-constexpr int SMALL_WG = 1024, SMALL_UNITS = 2048, SMALL_SLOTS = 8192;
+// atoms 250 us -> 235, MD 51 us per step -> 49.  At 2,000 units its build takes 14
+// us longer than the two launches below.
+constexpr int SMALL_WG = 1024, SMALL_UNITS = 1024, SMALL_SLOTS = 4096;
 
 __global__ __launch_bounds__(SMALL_WG) void k_list_small(
     const double* __restrict__ pos, const int* __restrict__ unit_ptr, const int* __restrict__ unit_atoms,
@@ -648,7 +649,7 @@ __global__ __launch_bounds__(64) void k_super_bounds(int nsuper, const int* __re
 }
 
 
-// Cluster lists, one wave per cluster C of block I = C / CPB (W clusters per
+// Cluster lists, one wave per cluster C of block I = C / CPB (CLIST_WAVES per
 // workgroup).  Each pair of blocks of a system is taken by one
 // of the two: in a system of nb blocks scanned flat, block I takes the nb/2
 // blocks after it, cyclically (J = I + d mod nb for 0 < d < nb/2, and
@@ -770,17 +771,17 @@ __device__ __forceinline__ int nth_set_bit(unsigned long long m, int k) {
     return pos;
 }
 
-// Clusters (one per wave) per workgroup of k_clist: two for a single system
-// (small workgroups spread over every compute unit), CLIST_WAVES_BATCH for
-// batches, whose first nkept workgroups append the tasks of the unflagged
-// systems, a cluster per thread (one reservation on the counter, 12 ns each, for
-// 64 CLIST_WAVES_BATCH clusters), while the others leave those at once.
-// Workgroups of four: 64 replicas 1,245 us per step, of eight 1,285, of sixteen
-// that append as well 1,306.
-constexpr int CLIST_WAVES_SINGLE = 2, CLIST_WAVES_BATCH = 4;
+// Clusters (one per wave) per workgroup of k_clist.  Each workgroup reserves its
+// tasks on one counter, 12 ns each, which two waves feel above 10,000 atoms and
+// which wide workgroups pay for in waiting for a free compute unit: with 2, 4, 8
+// and 16 waves 9,000 atoms 37.5, 35.7, 37, 48 us, 23,550 47, 36, 41, 41, 300,000
+// 349, 337, 422, 509.  In batches the first nkept workgroups append the tasks of
+// the unflagged systems, a cluster per thread, and the others leave those at
+// once (64 replicas 1,245 us per step, with 8 waves 1,285; with every workgroup
+// of sixteen appending, 1,306).
+constexpr int CLIST_WAVES = 4;
 
-template <int W>
-__global__ __launch_bounds__(64 * W) void k_clist(
+__global__ __launch_bounds__(64 * CLIST_WAVES) void k_clist(
     const double* __restrict__ pos, const int* __restrict__ sorted_atom, const int* __restrict__ block_sys,
     const SysInfo* __restrict__ sys, const double* __restrict__ center, const float* __restrict__ half,
     const int* __restrict__ super_off, const double* __restrict__ super_center,
@@ -788,14 +789,15 @@ __global__ __launch_bounds__(64 * W) void k_clist(
     const int* __restrict__ excl_idx, const int2* __restrict__ excl_range, const int* __restrict__ minimg,
     const float4* __restrict__ slot_pos, double reach, int cap, int nclusters, int tpt, int2* clist,
     unsigned char* clist_ex, int* ccount, int* tasks, int* ntasks, unsigned* status, const int* flag, int nkept) {
-    __shared__ int s_runs[W];
+    __shared__ int s_runs[CLIST_WAVES];
     __shared__ int s_base;
+    __shared__ float4 s_near[CLIST_WAVES][64];
     if (!flag[0]) return;
     const int wave = threadIdx.x / 64;
     const int lane = threadIdx.x % 64;
     auto runs_of = [&](int entries) { return ((entries + JTILE - 1) / JTILE + tpt - 1) / tpt; };
     if ((int)blockIdx.x < nkept) {
-        const int C = blockIdx.x * (64 * W) + threadIdx.x;
+        const int C = blockIdx.x * (64 * CLIST_WAVES) + threadIdx.x;
         int runs = 0;
         if (C < nclusters && !flag[1 + block_sys[C / CPB]]) runs = runs_of(ccount[C]);
         int upto = runs;
@@ -807,7 +809,7 @@ __global__ __launch_bounds__(64 * W) void k_clist(
         __syncthreads();
         if (threadIdx.x == 0) {
             int all = 0;
-            for (int w = 0; w < W; ++w) all += s_runs[w];
+            for (int w = 0; w < CLIST_WAVES; ++w) all += s_runs[w];
             s_base = all > 0 ? atomicAdd(ntasks, all) : 0;
         }
         __syncthreads();
@@ -816,7 +818,7 @@ __global__ __launch_bounds__(64 * W) void k_clist(
         for (int k = 0; k < runs; ++k) tasks[at + k] = (C << 8) | (k * tpt);
         return;
     }
-    const int C = ((int)blockIdx.x - nkept) * W + wave;
+    const int C = ((int)blockIdx.x - nkept) * CLIST_WAVES + wave;
     const int I = C / CPB;
     const int si = C < nclusters ? block_sys[I] : 0;
     const int first = C * CLUSTER;  // the cluster's first slot
@@ -910,28 +912,38 @@ __global__ __launch_bounds__(64 * W) void k_clist(
             if (m != 0 && __ballot(pass && near) == m) {
                 // Every passing block takes the slot-offset test, NEAR_ROUND
                 // per round with all their loads issued together: lanes 0-31
-                // the first of each pair, lanes 32-63 the second.
-                constexpr int NEAR_ROUND = 8;
-                const float4 none = make_float4(0.0f, 0.0f, 0.0f, __int_as_float(-1));
+                // the first of each pair, lanes 32-63 the second.  The passing
+                // blocks with their offsets are lined up in LDS.
+                constexpr int NEAR_ROUND = 4;
+                if (pass)
+                    s_near[wave][__popcll(m & below)] = make_float4(dcf[0], dcf[1], dcf[2], __int_as_float(J));
+                __builtin_amdgcn_wave_barrier();
+                struct Near {
+                    float4 dc, q;
+                    int2 range;
+                    int slot;
+                };
+                auto load = [&](int kk) {
+                    Near e;
+                    e.dc = s_near[wave][min(kk, npass - 1)];
+                    e.slot = __float_as_int(e.dc.w) * IBLOCK + (lane & 31);
+                    e.q = slot_pos[e.slot];
+                    e.range = excl_range[e.slot];
+                    if (kk >= npass) e.q.w = __int_as_float(-1);
+                    return e;
+                };
+                Near e[NEAR_ROUND / 2], next[NEAR_ROUND / 2];
+#pragma unroll
+                for (int u = 0; u < NEAR_ROUND / 2; ++u) e[u] = load(2 * u + (lane >> 5));
                 for (int r = 0; r < npass; r += NEAR_ROUND) {
-                    int src[NEAR_ROUND / 2], sl[NEAR_ROUND / 2];
-                    float4 q[NEAR_ROUND / 2];
-                    int2 rg[NEAR_ROUND / 2];
 #pragma unroll
-                    for (int u = 0; u < NEAR_ROUND / 2; ++u) {
-                        const int kk = r + 2 * u + (lane >> 5);
-                        src[u] = kk < npass ? nth_set_bit(m, kk) : 0;
-                        sl[u] = kk < npass ? (J0 + src[u]) * IBLOCK + (lane & 31) : -1;
-                    }
-#pragma unroll
-                    for (int u = 0; u < NEAR_ROUND / 2; ++u) {
-                        q[u] = sl[u] >= 0 ? slot_pos[sl[u]] : none;
-                        rg[u] = sl[u] >= 0 ? excl_range[sl[u]] : make_int2(INT_MAX, -1);
-                    }
+                    for (int u = 0; u < NEAR_ROUND / 2; ++u) next[u] = load(r + NEAR_ROUND + 2 * u + (lane >> 5));
 #pragma unroll
                     for (int u = 0; u < NEAR_ROUND / 2; ++u)
-                        append_near(sl[u], q[u], rg[u], __shfl(dcf[0], src[u], 64), __shfl(dcf[1], src[u], 64),
-                                    __shfl(dcf[2], src[u], 64), first, cap, out, out_ex, ex, count, below, ca);
+                        append_near(e[u].slot, e[u].q, e[u].range, e[u].dc.x, e[u].dc.y, e[u].dc.z, first, cap, out,
+                                    out_ex, ex, count, below, ca);
+#pragma unroll
+                    for (int u = 0; u < NEAR_ROUND / 2; ++u) e[u] = next[u];
                 }
                 return;
             }
@@ -995,7 +1007,7 @@ __global__ __launch_bounds__(64 * W) void k_clist(
     __syncthreads();
     if (threadIdx.x == 0) {
         int all = 0;
-        for (int w = 0; w < W; ++w) all += s_runs[w];
+        for (int w = 0; w < CLIST_WAVES; ++w) all += s_runs[w];
         s_base = all > 0 ? atomicAdd(ntasks, all) : 0;
     }
     __syncthreads();
@@ -1341,19 +1353,12 @@ void nlist_build(NlistDev& nl, const double* pos, const SysInfo* sys_dev, unsign
     if (nl.use_super)
         hipLaunchKernelGGL(k_super_bounds, dim3(nl.nsuper), dim3(64), 0, s, nl.nsuper, nl.super_off.p, nl.nsys,
                            sys_dev, nl.block_center.p, nl.block_half.p, nl.super_center.p, nl.super_half.p, flag);
-    auto clist = [&](auto kernel, int w) {
-        const int kept = nl.nsys == 1 ? 0 : blocks_for(nl.nclusters, 64 * w);
-        hipLaunchKernelGGL(kernel, dim3(kept + blocks_for(nl.nclusters, w)), dim3(64 * w), 0, s, pos, nl.sorted_atom.p,
-                           nl.block_sys.p, sys_dev, nl.block_center.p, nl.block_half.p, nl.super_off.p,
-                           nl.super_center.p, nl.super_half.p, nl.atom_slot.p, nl.excl_ptr.p, nl.excl_idx.p,
-                           nl.excl_range.p, nl.block_minimg.p, nl.slot_pos.p, reach, nl.cap, nl.nclusters, nl.tpt, nl.clist.p,
-                           nl.clist_ex.p, nl.ccount.p, nl.tasks.p, nl.ntasks.p, status, flag,
-                           kept);
-    };
-    if (nl.nsys == 1)
-        clist(k_clist<CLIST_WAVES_SINGLE>, CLIST_WAVES_SINGLE);
-    else
-        clist(k_clist<CLIST_WAVES_BATCH>, CLIST_WAVES_BATCH);
+    const int kept = nl.nsys == 1 ? 0 : blocks_for(nl.nclusters, 64 * CLIST_WAVES);
+    hipLaunchKernelGGL(k_clist, dim3(kept + blocks_for(nl.nclusters, CLIST_WAVES)), dim3(64 * CLIST_WAVES), 0, s, pos,
+                       nl.sorted_atom.p, nl.block_sys.p, sys_dev, nl.block_center.p, nl.block_half.p, nl.super_off.p,
+                       nl.super_center.p, nl.super_half.p, nl.atom_slot.p, nl.excl_ptr.p, nl.excl_idx.p,
+                       nl.excl_range.p, nl.block_minimg.p, nl.slot_pos.p, reach, nl.cap, nl.nclusters, nl.tpt,
+                       nl.clist.p, nl.clist_ex.p, nl.ccount.p, nl.tasks.p, nl.ntasks.p, status, flag, kept);
     OMM_HIP(hipGetLastError());
 }
 

@@ -10,9 +10,10 @@ from helpers import water
 pytestmark = pytest.mark.gpu
 
 
-# Below, at and above 2,048 units (whose last wave of blocks is partial), one
-# unit, and a tilted box with few cells.
-@pytest.mark.parametrize("molecules,edge,tilt", [(1, 1.85, 0.0), (22, 1.85, 0.3), (1025, 3.2, 0.0), (2048, 3.95, 0.2),
+# Below, at and above the 1,024 units of the one-workgroup list, one unit, a
+# tilted box with few cells.
+@pytest.mark.parametrize("molecules,edge,tilt", [(1, 1.85, 0.0), (22, 1.85, 0.3), (1024, 3.2, 0.1),
+                                                 (1025, 3.2, 0.0), (2048, 3.95, 0.2),
                                                  (2049, 3.95, 0.2)])
 def test_pairs_and_steps_at_the_size_limits(molecules, edge, tilt):
     s = water(molecules, edge, seed=molecules, cutoff=0.9)
