@@ -45,6 +45,8 @@ __global__ __launch_bounds__(TERM_THREADS) void k_fold(int ntiles, const Term* _
                                                        unsigned* status) {
     __shared__ double s_pos[3][TERM_THREADS], s_q[TERM_THREADS];
     __shared__ A s_f[3][TERM_THREADS];
+    __shared__ double s_e[TERM_THREADS / 64];
+    __shared__ int s_kind[TERM_THREADS / 64];
     const int t = threadIdx.x;
     if ((int)blockIdx.x >= ntiles) {
         const int s = ((int)blockIdx.x - ntiles) * TERM_THREADS + t;
@@ -106,10 +108,21 @@ __global__ __launch_bounds__(TERM_THREADS) void k_fold(int ntiles, const Term* _
         for (int c = 0; c < 3; ++c)
             if (s_f[c][t] != (A)0) add_raw(force + 3 * (size_t)a + c, s_f[c][t]);
     if (energy) {
-        // The first lane of a wave has a term if any lane has.
-        const int slot = kind == TERM_ANGLE ? E_ANGLE : (kind == TERM_BOND ? E_BOND : E_EXCEPT);
+        // A wave's terms are of its first lane's kind; one add per kind and
+        // workgroup (they meet on one address).
         const double sum = wave_sum(e);
-        if ((t & 63) == 0 && sum != 0.0) acc_add(energy + (size_t)si * E_SLOTS + slot, sum, ENERGY_SCALE, status);
+        if ((t & 63) == 0) {
+            s_e[t >> 6] = sum;
+            s_kind[t >> 6] = kind;
+        }
+        __syncthreads();
+        if (t < 3) {
+            const int of = t == 0 ? TERM_EXCEPTION : (t == 1 ? TERM_BOND : TERM_ANGLE);
+            double total = 0.0;
+            for (int w = 0; w < TERM_THREADS / 64; ++w) total += s_kind[w] == of ? s_e[w] : 0.0;
+            const int slot = t == 0 ? E_EXCEPT : (t == 1 ? E_BOND : E_ANGLE);
+            if (total != 0.0) acc_add(energy + (size_t)si * E_SLOTS + slot, total, ENERGY_SCALE, status);
+        }
     }
 }
 

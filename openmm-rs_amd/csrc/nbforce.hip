@@ -1490,7 +1490,7 @@ void NbOperator::profile(const double* pos_dev, int reps, long long* force_fx, d
     });
     auto fold = [&](bool slots, const TermTiles* terms) {
         launch_fold(mixed_, nl_, slots, terms, term_params(), part_.charge.p, pos_dev, sys_dev_.p, force_fx, force_d,
-                    energy_fx, energy_d, status, s);
+                    nullptr, nullptr, status, s);
     };
     fold(true, nullptr);
     ms[2] = timed([&] { fold(false, &exc_); });
@@ -1621,7 +1621,8 @@ void NbOperator::compute(const double* pos, const double* box, bool direct, bool
             launch_pairs(mixed_, want_energy, nl_, pp_, part_, pos_dev_.p, sys_dev_.p,
                          energy_fx_.p, energy_d_.p, status_.p, want_stats ? stats_.p : nullptr, pair_grid_, s);
             launch_fold(mixed_, nl_, true, &exc_, term_params(), part_.charge.p, pos_dev_.p, sys_dev_.p, force_fx_.p,
-                        force_d_.p, energy_fx_.p, energy_d_.p, status_.p, s);
+                        force_d_.p, want_energy ? energy_fx_.p : nullptr, want_energy ? energy_d_.p : nullptr,
+                        status_.p, s);
         }
         if (beside) OMM_HIP(hipStreamWaitEvent(s, ev_join_, 0));
         const size_t nout = out ? n3 : 0;
