@@ -578,9 +578,11 @@ __global__ __launch_bounds__(64) void k_pairs(const double* __restrict__ pos, co
 // the tasks' size nor their order changes the total.  Adds to one energy
 // serialise (12 ns each: one per task was 60 us at 9,000 atoms), so few waves
 // are launched and a workgroup adds once when its waves saw one system.
-// Bound: FP64 issue (about 150 instructions per step of 64 slots).  Pair forces
-// and energies together, in one kernel and now in two: 58 -> 17 us at 900 atoms,
-// 91 -> 47 at 9,000, 132 -> 104 at 23,550.
+// Bound: FP64 issue.  36% of a tile's slots are in range: they are lined up in
+// LDS first and evaluated 64 at a time (every slot evaluated: 9,000 atoms 27.7 us,
+// so 24.1; 23,550 62.6 and 55.2; 300,000 869 and 733).  Pair forces and energies
+// together, in one kernel and now in two: 58 -> 18 us at 900 atoms, 91 -> 44 at
+// 9,000, 132 -> 98 at 23,550.
 constexpr int ENERGY_WAVES = 4;           // waves per workgroup
 constexpr int ENERGY_WORKGROUPS = 768;    // at most: three waves per SIMD of the chip
 
@@ -604,12 +606,16 @@ __global__ __launch_bounds__(64 * ENERGY_WAVES) void k_pair_energy(
     __shared__ __align__(8) unsigned char s_exw[ENERGY_WAVES][JTILE];
     __shared__ long long s_sum[ENERGY_WAVES];
     __shared__ int s_of[ENERGY_WAVES];
+    constexpr int RING = 128, RING_VALUES = (KIND & PAIR_LJPME) != 0 ? 5 : 4;
+    __shared__ double s_ring[ENERGY_WAVES][RING_VALUES][RING];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    double(*ring)[RING] = s_ring[wave];
     Q4<double>* s_p = s_pw[wave];
     Q2<double>* s_se = s_sew[wave];
     int *s_js = s_jsw[wave], *s_ja = s_jaw[wave];
     unsigned char* s_ex = s_exw[wave];
     const int lane = threadIdx.x & 63, grp = lane / CLUSTER, il = lane % CLUSTER;
+    const unsigned long long below = (1ull << lane) - 1ull;
     const double cutoff2 = P.cutoff * P.cutoff;
     const double rc2_lo = cutoff2 * (1.0 - 1e-12), rc2_hi = cutoff2 * (1.0 + 1e-12);
     long long esum = 0;  // lane 0: fixed-point energy of system esys
@@ -657,21 +663,46 @@ __global__ __launch_bounds__(64 * ENERGY_WAVES) void k_pair_energy(
             const unsigned present = valid_entries(s_js + grp * CLUSTER, s_ex + grp * CLUSTER, is, il);
             const unsigned vmask = ia >= 0 ? present : 0u;
             double eacc = 0.0;
+            // The tile's pairs in range are lined up in a ring, 64 evaluated at
+            // a time; the last turn evaluates the rest.
+            int head = 0, waiting = 0;
 #pragma unroll 1
-            for (int s8 = 0; s8 < CLUSTER; ++s8) {
-                const int slot = grp * CLUSTER + s8;
-                const Q4<double> pj = s_p[slot];
-                const Q2<double> sj = s_se[slot];
-                double dd[3] = {pj.x - di[0], pj.y - di[1], pj.z - di[2]};
-                if (mi) wrap_nearest(dd, bx);
-                const double r2 = dd[0] * dd[0] + dd[1] * dd[1] + dd[2] * dd[2];
-                const bool valid = (vmask >> s8) & 1u;
-                bool in = valid && (!P.use_cutoff || r2 < rc2_lo);
-                if (valid && !in && r2 < rc2_hi)
-                    in = within_cutoff_exact(pos, ia, s_ja[slot], bx, P.periodic, cutoff2);
-                // A rejected slot is evaluated away from the singularity.
-                const double e = pair_energy_fp64<KIND>(in ? r2 : 1.0, si + sj.x, ei * sj.y, si * sj.x, qi * pj.w, P);
-                eacc += in ? e : 0.0;
+            for (int s8 = 0; s8 <= CLUSTER; ++s8) {
+                if (s8 < CLUSTER) {
+                    const int slot = grp * CLUSTER + s8;
+                    const Q4<double> pj = s_p[slot];
+                    double dd[3] = {pj.x - di[0], pj.y - di[1], pj.z - di[2]};
+                    if (mi) wrap_nearest(dd, bx);
+                    const double r2 = dd[0] * dd[0] + dd[1] * dd[1] + dd[2] * dd[2];
+                    const bool valid = (vmask >> s8) & 1u;
+                    bool in = valid && (!P.use_cutoff || r2 < rc2_lo);
+                    if (valid && !in && r2 < rc2_hi)
+                        in = within_cutoff_exact(pos, ia, s_ja[slot], bx, P.periodic, cutoff2);
+                    const unsigned long long m = __ballot(in);
+                    if (in) {
+                        const Q2<double> sj = s_se[slot];
+                        const int at = (head + waiting + __popcll(m & below)) & (RING - 1);
+                        ring[0][at] = r2;
+                        ring[1][at] = si + sj.x;
+                        ring[2][at] = ei * sj.y;
+                        ring[3][at] = qi * pj.w;
+                        if constexpr ((KIND & PAIR_LJPME) != 0) ring[4][at] = si * sj.x;
+                    }
+                    waiting += __popcll(m);
+                    wave_sync();
+                    if (waiting < 64) continue;
+                } else if (waiting == 0) {
+                    break;
+                }
+                // A lane without a pair evaluates the last one.
+                const int at = (head + min(lane, waiting - 1)) & (RING - 1);
+                const double ss = (KIND & PAIR_LJPME) != 0 ? ring[RING_VALUES - 1][at] : 0.0;
+                const double e = pair_energy_fp64<KIND>(ring[0][at], ring[1][at], ring[2][at], ss, ring[3][at], P);
+                eacc += lane < waiting ? e : 0.0;
+                const int taken = min(waiting, 64);
+                head += taken;
+                waiting -= taken;
+                wave_sync();
             }
             const double et = wave_sum(eacc);
             esum += to_fixed(et, ENERGY_SCALE, status);
