@@ -1279,7 +1279,11 @@ void nlist_check(NlistDev& nl, const double* pos, int force, hipStream_t s) {
     OMM_HIP(hipGetLastError());
 }
 
-// The units in order of their cells, placed at their slots.
+// The units in order of their cells, placed at their slots, for systems that a
+// workgroup cannot order.  The cell-count scan rides on the key kernel and, for
+// a single system, the sort of uniform units on their placement (batches rebuild
+// some replica on most steps, and there one thread per unit places faster than
+// one thread per cell).
 static void build_order(NlistDev& nl, const double* pos, const SysInfo* sys_dev, const int* flag, hipStream_t s) {
     if (nl.ncells <= SCAN_SINGLE_MAX) {
         hipLaunchKernelGGL(k_unit_keys_scan, dim3(blocks_for(nl.nunits, SCAN_WG)), dim3(SCAN_WG), 0, s, pos,
@@ -1320,10 +1324,7 @@ void nlist_build(NlistDev& nl, const double* pos, const SysInfo* sys_dev, unsign
     const int* flag = forced ? nl.one.p : nl.flag.p;
     // Each kernel of the chain is a graph node that costs a few microseconds
     // even when it exits at once, so steps without a rebuild pay for the
-    // chain's length: the cell-count scan rides on the key kernel and, for a
-    // single system, the sort of uniform units on their placement.  (Batches
-    // rebuild some replica on most steps, and there one thread per unit
-    // places faster than one thread per cell.)
+    // chain's length.
     const double reach = nl.cutoff + nl.skin;
     const bool by_system = nl.uniform > 0 && nl.max_units <= ORDER_UNITS && nl.max_cells <= ORDER_CELLS;
     if (by_system && nl.nsys == 1 && nl.nunits <= SMALL_UNITS && nl.nslots <= SMALL_SLOTS) {

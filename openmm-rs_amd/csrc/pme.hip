@@ -256,10 +256,10 @@ __global__ __launch_bounds__(SPREAD_THREADS) void k_spread_tiles(const int* __re
 // axis each, then its four waves hold the same atoms, one per lane, with their
 // weights in registers, and share the stencil's 25 rows.  Bound:
 // latency at small systems, the device atomics of the box (27 points per atom at
-// 100 atoms/nm^3) at large ones.  Kept in LDS with a thread per row of an atom's
-// stencil, and with tiles for FP64 grids, it took (here): 3,000 unsorted atoms on
-// an FP64 grid 57 us (22), 9,000 sorted ones 50 (14); FP32 stencils at 300,000
-// atoms 91 (83).  Four chunks per workgroup in one box add a third fewer points
+// 100 atoms/nm^3; a compute unit issues one in 1.5 ns) at large ones.  Before, with
+// the weights in LDS and a thread per row of an atom's stencil, and now: FP32
+// stencils 900 atoms 18 -> 9 us, 300,000 91 -> 75; 9,000 on an FP64 grid, by tiles
+// before, 50 -> 9.  Four chunks per workgroup in one box add a third fewer points
 // and take twice as long below 60,000 atoms (36 us against 16 at 23,550).
 constexpr int SPREAD_BOX_BYTES = 32768;
 constexpr int ATOM_SPREAD_WAVES = 4, ATOM_SPREAD_THREADS = 64 * ATOM_SPREAD_WAVES;
@@ -1402,8 +1402,8 @@ void pme_setup(PmeDev& pm, std::vector<SysInfo>& sys, int natoms, const int* ato
     pm.nsys = nsys;
     pm.natoms = natoms;
     pm.atom_sys = atom_sys;
-    // Until an autotuner chooses: atom-owned (9,000 atoms with FP64 stencils, 14
-    // us against 50 for the tiles).
+    // Until an autotuner chooses: atom-owned (9,000 atoms with FP64 stencils, 9 us
+    // against 50 for the tiles).
     pm.spread_atoms = true;
     pm.planes = nsys == 1 ? sys[0].grid[0] : 0;
     pm.plane_points = nsys == 1 ? sys[0].grid[1] * sys[0].grid[2] : INT_MAX;
