@@ -329,6 +329,7 @@ private:
     PinnedBuf<EvalResult> host_res_;
     Box last_box_{};
     bool have_box_ = false;
+    bool list_stale_ = true;  // compute's list has not been built since the box changed
 };
 
 

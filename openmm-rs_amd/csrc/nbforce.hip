@@ -1315,6 +1315,7 @@ double NbOperator::mesh_charges(const double* pos, const double* box, double alp
         upload_systems(s);
         last_box_ = b;
         have_box_ = true;
+        list_stale_ = true;
     }
     mesh_q_.alloc((size_t)n);
     if (count > 0) {
@@ -1563,12 +1564,12 @@ void NbOperator::compute(const double* pos, const double* box, bool direct, bool
         if (pair_hash) *pair_hash = 0;
         return;
     }
-    bool box_changed = vchanged || !have_box_ || std::memcmp(b.v, last_box_.v, sizeof(b.v)) != 0;
-    if (box_changed) {
+    if (vchanged || !have_box_ || std::memcmp(b.v, last_box_.v, sizeof(b.v)) != 0) {
         sys_h_[0].box = b;
         upload_systems(s);
         last_box_ = b;
         have_box_ = true;
+        list_stale_ = true;  // also where this call reads no list: the next one that does builds it
     }
     if (pos_dev_in) {
         // Ordered after the caller's work on its stream; the call returns
@@ -1589,7 +1590,7 @@ void NbOperator::compute(const double* pos, const double* box, bool direct, bool
     for (int attempt = 0; attempt < 6; ++attempt) {
         const double* src = attempt > 0 ? pos_dev_.p : (pos_dev_in ? pos_dev_in : host_in_.p);
         const double* built = direct ? nl_.pos_build.p : nullptr;
-        const int rebuild = direct && (box_changed || attempt > 0) ? 1 : 0;
+        const int rebuild = direct && (list_stale_ || attempt > 0) ? 1 : 0;
         const dim3 wgs((n + EVAL_WG - 1) / EVAL_WG);
         if (mixed_)
             hipLaunchKernelGGL(k_eval_begin<long long>, wgs, dim3(EVAL_WG), 0, s, n, src, pos_dev_.p, built,
@@ -1640,6 +1641,7 @@ void NbOperator::compute(const double* pos, const double* box, bool direct, bool
             grow(st);
             continue;
         }
+        if (direct) list_stale_ = false;
         if (st & ST_NONFINITE) throw Error(OMM_ERR_NONFINITE, "non-finite force or energy on the device");
         if (st & ST_OVERFLOW) throw Error(OMM_ERR_OVERFLOW, "fixed-point force/energy accumulator overflow");
         const double* e = res->energy;
