@@ -20,8 +20,14 @@
 // Bound: launch and load latency up to about 64 points per axis (three
 // launches of 4-7 us at 55^3, 0.3 of it matrix-core issue), matrix-core issue
 // and LDS reads above.  Transforms and convolution, FP32, serial launches,
-// before (staged passes) and with these passes: 19^3 25 -> 14 us, 55^3 31 ->
-// 21, 109^3 451 -> 80, 116^3 215 -> 102.
+// before (staged passes) and with these passes: 19^3 25 -> 15 us, 55^3 31 ->
+// 22, 109^3 268 -> 81, 116^3 147 -> 102.
+//
+// FP32 accuracy (StepSum), relative RMS error of the mesh forces of water boxes
+// with staged passes and with these: 37^3 8.50e-6, 8.23e-6; 55^3 1.31e-5, 1.32e-5;
+// 96^3 1.31e-5, 1.32e-5; 116^3 1.56e-5, 1.55e-5; 120^3 1.92e-5, 1.91e-5 (10 to 24
+// boxes each, 1% of scatter; the splines and the gather make up most of it).
+// On 120 x 12 x 12 points, where the transforms show: 1.65e-6 and 1.47e-6.
 #pragma once
 
 #include "fmath.h"
@@ -172,6 +178,26 @@ struct Mat<double> {
 // steps whose LDS operands are loaded while the pair before them multiplies.
 __host__ __device__ inline int round8(int n) { return (n + 7) & ~7; }
 
+// Sum of the pairs of steps.  FP32: each pair is summed by itself and then added
+// to the others, so that the rounding error of n terms grows as that of 8 + n/8
+// (in one chain had 2.5e-6 on those 120 points).  The pair added is the one
+// before the last, whose products are done.  FP64: one chain.
+template <class R>
+struct StepSum {
+    using V4 = typename Mat<R>::V4;
+    static constexpr bool BLOCKED = sizeof(R) == 4;
+    V4 sum = {0, 0, 0, 0}, last = {0, 0, 0, 0};
+    __device__ __forceinline__ V4 start() const {
+        const V4 zero = {0, 0, 0, 0};
+        return BLOCKED ? zero : last;
+    }
+    __device__ __forceinline__ void add(V4 pair) {
+        if (BLOCKED) sum += last;
+        last = pair;
+    }
+    __device__ __forceinline__ V4 total() const { return BLOCKED ? sum + last : last; }
+};
+
 // Rows row0 .. row0 + 15 of the complex DFT of one tile held in LDS as
 // b[round8(n)][16] with zeros past row n.  roots[m] = e^{-2 pi i m / n}; sgn =
 // +1 for the forward transform, -1 for the inverse.  With w = wr + i wi,
@@ -187,7 +213,7 @@ __device__ __forceinline__ typename Mat<R>::V4 dft_rows(const R* b, int n, int r
     const R* p = b + kq * DFT_W + c;
     const R* q = b + kq * DFT_W + (c ^ DFT_COLS);
     const R s = c < DFT_COLS ? -sgn : sgn;
-    typename Mat<R>::V4 acc = {0, 0, 0, 0};
+    StepSum<R> total;
     Cx<R> w[2];
     R v[2], u[2];
     auto load = [&](int k) {
@@ -206,13 +232,15 @@ __device__ __forceinline__ typename Mat<R>::V4 dft_rows(const R* b, int n, int r
         const Cx<R> w0 = w[0], w1 = w[1];
         const R v0 = v[0], v1 = v[1], u0 = s * u[0], u1 = s * u[1];
         if (k < end) load(k);
+        typename Mat<R>::V4 acc = total.start();
         acc = Mat<R>::mac(w0.x, v0, acc);
         acc = Mat<R>::mac(w0.y, u0, acc);
         acc = Mat<R>::mac(w1.x, v1, acc);
         acc = Mat<R>::mac(w1.y, u1, acc);
+        total.add(acc);
         if (k >= end) break;
     }
-    return acc;
+    return total.total();
 }
 
 // Orders a wave's LDS writes before its other lanes' reads.
@@ -293,7 +321,7 @@ __global__ __launch_bounds__(64 * W) void k_dft_zy(const int* __restrict__ off, 
         if (y0 >= nyp) break;
         // Column c < 8: sum_z q cos(2 pi z kz / nz), else its imaginary part.
         const R* w = reinterpret_cast<const R*>(rz) + (c >= DFT_COLS ? 1 : 0);
-        typename Mat<R>::V4 acc = {0, 0, 0, 0};
+        StepSum<R> total;
         int idx = mod_small(kq * kz, nz, inv_nz);
         const R* a = stage + c * zs + kq;
         R av[2], wv[2];
@@ -310,10 +338,13 @@ __global__ __launch_bounds__(64 * W) void k_dft_zy(const int* __restrict__ off, 
         for (int k = 8;; k += 8) {
             const R a0 = av[0], a1 = av[1], w0 = wv[0], w1 = wv[1];
             if (k < nzp) load(k);
+            typename Mat<R>::V4 acc = total.start();
             acc = Mat<R>::mac(a0, w0, acc);
             acc = Mat<R>::mac(a1, w1, acc);
+            total.add(acc);
             if (k >= nzp) break;
         }
+        const typename Mat<R>::V4 acc = total.total();
         for (int r = 0; r < 4; ++r) {
             const int y = y0 + Mat<R>::row(lane, r);
             if (y < nyp) z[y * DFT_W + c] = acc[r];  // rows past ny are zero
@@ -478,7 +509,7 @@ __global__ __launch_bounds__(64 * W) void k_dft_yz(const int* __restrict__ off, 
         const int z = z0 + c < nz ? z0 + c : 0;
         int idx = mod_small(z * kq, nz, inv_nz);
         const int step = mod_small(4 * z, nz, inv_nz);
-        typename Mat<R>::V4 acc = {0, 0, 0, 0};
+        StepSum<R> total;
         const R* a = v + c * vs + kq;
         Cx<R> w[2];
         R re[2], im[2];
@@ -499,12 +530,15 @@ __global__ __launch_bounds__(64 * W) void k_dft_yz(const int* __restrict__ off, 
             const Cx<R> w0 = w[0], w1 = w[1];
             const R r0 = re[0], r1 = re[1], i0 = im[0], i1 = im[1];
             if (g < ntile) load(g);
+            typename Mat<R>::V4 acc = total.start();
             acc = Mat<R>::mac(r0, w0.x, acc);
             acc = Mat<R>::mac(i0, w0.y, acc);
             acc = Mat<R>::mac(r1, w1.x, acc);
             acc = Mat<R>::mac(i1, w1.y, acc);
+            total.add(acc);
             if (g >= ntile) break;
         }
+        const typename Mat<R>::V4 acc = total.total();
         for (int r = 0; r < 4; ++r) {
             const int y = y0 + Mat<R>::row(lane, r);
             if (y < ny && z0 + c < nz) phi[S.qgrid_off + ((size_t)x * ny + y) * nz + z0 + c] = acc[r];
