@@ -180,7 +180,7 @@ __host__ __device__ inline int round8(int n) { return (n + 7) & ~7; }
 
 // Sum of the pairs of steps.  FP32: each pair is summed by itself and then added
 // to the others, so that the rounding error of n terms grows as that of 8 + n/8
-// (in one chain had 2.5e-6 on those 120 points).  The pair added is the one
+// (one chain had 2.5e-6 on the 120 points above).  The pair added is the one
 // before the last, whose products are done.  FP64: one chain.
 template <class R>
 struct StepSum {

@@ -182,41 +182,59 @@ __device__ __forceinline__ unsigned valid_entries(const int* js, const unsigned 
     return vmask & ~(lo4 | (hi4 << 4));
 }
 
-// A lane's force on its i-atom over a task.  Mixed form: each tile's FP32 sum
-// is rounded to multiples of 2^-28 (3.7e-9 kJ/mol/nm) by adding and subtracting
-// 1.5 x 2^24, where FP64 has that step, and the multiples are added in FP64,
-// exactly in any grouping while sums stay below 2^24; so the total does not
-// depend on how many tiles a task holds.  Four instructions per component and
-// tile; converting each tile's sum to the accumulators' fixed point cost 5% of
-// the kernel at 300,000 atoms.
-struct FixedForce {
-    static constexpr double STEP = 25165824.0;  // 1.5 x 2^24
-    double x = 0, y = 0, z = 0;
-    static __device__ __forceinline__ double rounded(float f) { return ((double)f + STEP) - STEP; }
-    __device__ __forceinline__ void add(float fx, float fy, float fz) {
-        x += rounded(fx);
-        y += rounded(fy);
-        z += rounded(fz);
-    }
-    static __device__ __forceinline__ long long total(double v, unsigned* status) {
-        return to_fixed(v, FORCE_SCALE, status);
-    }
-};
-struct PlainForce {
-    double x = 0, y = 0, z = 0;
-    __device__ __forceinline__ void add(double fx, double fy, double fz) {
-        x += fx;
-        y += fy;
-        z += fz;
-    }
-    static __device__ __forceinline__ double total(double v, unsigned*) { return v; }
-};
 // Sum over the eight groups (lanes l, l ^ 8, l ^ 16, ...).
 template <class T>
 __device__ __forceinline__ T group_sum(T v) {
     for (int o = CLUSTER; o < 64; o <<= 1) v += __shfl_xor(v, o, 64);
     return v;
 }
+// A lane's force on its i-atom over a task.  Mixed form: each tile's FP32 sum is
+// rounded to multiples of 2^-32, the accumulators' step, which are added as
+// integers, so the total does not depend on how many tiles a task holds.  Adding
+// 1.5 x 2^20, where FP64 has that step, leaves the multiple in the low bits.
+// Components of 2^19 kJ/mol/nm and more, which are rare, are multiples of 2^-4 and
+// are added in FP64, exactly while sums stay below 2^49.
+struct FixedForce {
+    static constexpr double STEP = 1572864.0;  // 1.5 x 2^20
+    static constexpr float LARGE = 524288.0f;  // 2^19
+    long long sum[3] = {0, 0, 0};
+    double large[3] = {0, 0, 0};
+    static __device__ __forceinline__ long long steps(float f) {
+        return __double_as_longlong((double)f + STEP) - __double_as_longlong(STEP);
+    }
+    __device__ __forceinline__ void add(float fx, float fy, float fz) {
+        const float f[3] = {fx, fy, fz};
+        // The absolute sum bounds each component and is NaN where one of them is.
+        if (__ballot(!(fabsf(fx) + fabsf(fy) + fabsf(fz) < LARGE)) == 0ull) {
+#pragma unroll
+            for (int c = 0; c < 3; ++c) sum[c] += steps(f[c]);
+            return;
+        }
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            const bool small = fabsf(f[c]) < LARGE;
+            sum[c] += steps(small ? f[c] : 0.0f);
+            large[c] += small ? 0.0 : (double)f[c];
+        }
+    }
+    __device__ __forceinline__ long long total(int c, unsigned* status) const {
+        const long long s = group_sum(sum[c]);  // below 2^56
+        if (__ballot(large[c] != 0.0) == 0ull) return s;
+        // The range is that of the whole task's force.
+        const double l = group_sum(large[c]);
+        if (!(fabs(l * FORCE_SCALE + (double)s) < 9.0e18)) return to_fixed(l + (double)s * (1.0 / FORCE_SCALE), FORCE_SCALE, status);
+        return s + (long long)(l * FORCE_SCALE);
+    }
+};
+struct PlainForce {
+    double x[3] = {0, 0, 0};
+    __device__ __forceinline__ void add(double fx, double fy, double fz) {
+        x[0] += fx;
+        x[1] += fy;
+        x[2] += fz;
+    }
+    __device__ __forceinline__ double total(int c, unsigned*) const { return group_sum(x[c]); }
+};
 __device__ __forceinline__ void add_total(long long* p, long long v) {
     if (v) atomicAdd(reinterpret_cast<unsigned long long*>(p), (unsigned long long)v);
 }
@@ -548,8 +566,7 @@ __global__ __launch_bounds__(64) void k_pairs(const double* __restrict__ pos, co
             r0 = r1;
         }
         // i-forces: the eight groups' sums, in a fixed order.
-        const A tx = group_sum(Force::total(ftot.x, status)), ty = group_sum(Force::total(ftot.y, status)),
-                tz = group_sum(Force::total(ftot.z, status));
+        const A tx = ftot.total(0, status), ty = ftot.total(1, status), tz = ftot.total(2, status);
         if (grp == 0 && ia >= 0) {
             add_total(fslot + is, tx);
             add_total(fslot + P.nslots + is, ty);
