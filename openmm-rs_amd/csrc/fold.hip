@@ -4,8 +4,7 @@
 //
 // Terms: the tile's atoms are staged in LDS once, each wave evaluates terms of
 // one kind (a wave that mixes them runs the kinds one after another), the forces
-// are summed per atom in LDS and leave with one add per atom component.  The
-// mixed form sums fixed-point values, in any order the same bits.  Bound:
+// are summed per atom in LDS and leave with one add per atom component.  Bound:
 // latency (a chain of two loads, an FP64 erf or acos, two barriers).  As two
 // launches, a molecule's terms on eight lanes that ran the kinds one after
 // another, they took 13 us and the gap between them; MD of 23,550 atoms 105 us
@@ -24,11 +23,54 @@ __device__ __forceinline__ void add_raw(long long* p, long long v) {
     atomicAdd(reinterpret_cast<unsigned long long*>(p), (unsigned long long)v);
 }
 __device__ __forceinline__ void add_raw(double* p, double v) { unsafeAtomicAdd(p, v); }
-// Adds v to an atom's sum in LDS.
-__device__ __forceinline__ void lds_force(long long* p, double v, unsigned* status) {
-    atomicAdd(reinterpret_cast<unsigned long long*>(p), (unsigned long long)to_fixed(v, FORCE_SCALE, status));
-}
-__device__ __forceinline__ void lds_force(double* p, double v, unsigned*) { atomicAdd(p, v); }
+
+// An atom's sum over a tile's terms in LDS.  Mixed form: each value is cut into
+// multiples of 2^20 kJ/mol/nm (hardly ever any), steps of the accumulator and
+// fractions at 2^-20 of a step, summed as integers (at most 3 x TERM_THREADS of
+// each: below 2^53, 2^62 and 2^31).  So the atom's force is rounded and checked once,
+// not term by term, and the order of the adds does not matter.
+template <class A>
+struct LdsForce;
+template <>
+struct LdsForce<long long> {
+    long long large[3][TERM_THREADS], steps[3][TERM_THREADS];
+    int parts[3][TERM_THREADS];
+    static __device__ __forceinline__ void add_to(long long* p, long long v) {
+        atomicAdd(reinterpret_cast<unsigned long long*>(p), (unsigned long long)v);
+    }
+    __device__ __forceinline__ void clear(int c, int i) {
+        large[c][i] = steps[c][i] = 0;
+        parts[c][i] = 0;
+    }
+    __device__ __forceinline__ void add(int c, int i, double v, unsigned* status) {
+        const double l = trunc(v * (1.0 / 1048576.0));
+        if (l != 0.0) {
+            if (!(fabs(l) < 4398046511104.0)) {  // 2^42, or not a number
+                (void)to_fixed(v, FORCE_SCALE, status);
+                return;
+            }
+            add_to(&large[c][i], (long long)l);
+            v -= l * 1048576.0;
+        }
+        const long long whole = (long long)(v * FORCE_SCALE);
+        add_to(&steps[c][i], whole);
+        atomicAdd(&parts[c][i], (int)rint((v * FORCE_SCALE - (double)whole) * 1048576.0));
+    }
+    __device__ __forceinline__ long long total(int c, int i, unsigned* status) const {
+        const long long s = steps[c][i] + ((parts[c][i] + 524288) >> 20), l = large[c][i];
+        if (l == 0) return s;
+        const double v = (double)l * 1048576.0 + (double)s * (1.0 / FORCE_SCALE);
+        if (!(fabs(v * FORCE_SCALE) < 9.0e18)) return to_fixed(v, FORCE_SCALE, status);
+        return s + l * (1ll << 52);
+    }
+};
+template <>
+struct LdsForce<double> {
+    double sum[3][TERM_THREADS];
+    __device__ __forceinline__ void clear(int c, int i) { sum[c][i] = 0.0; }
+    __device__ __forceinline__ void add(int c, int i, double v, unsigned*) { atomicAdd(&sum[c][i], v); }
+    __device__ __forceinline__ double total(int c, int i, unsigned*) const { return sum[c][i]; }
+};
 
 // The pair sums are added atomically, because the mesh may add into the same
 // accumulator from another stream meanwhile.
@@ -44,7 +86,7 @@ __global__ __launch_bounds__(TERM_THREADS) void k_fold(int ntiles, const Term* _
                                                        A* force, A* energy, int* order_a, int* order_b,
                                                        unsigned* status) {
     __shared__ double s_pos[3][TERM_THREADS], s_q[TERM_THREADS];
-    __shared__ A s_f[3][TERM_THREADS];
+    __shared__ LdsForce<A> s_f;
     __shared__ double s_e[TERM_THREADS / 64];
     __shared__ int s_kind[TERM_THREADS / 64];
     const int t = threadIdx.x;
@@ -74,7 +116,7 @@ __global__ __launch_bounds__(TERM_THREADS) void k_fold(int ntiles, const Term* _
     s_pos[1][t] = py;
     s_pos[2][t] = pz;
     s_q[t] = q;
-    for (int c = 0; c < 3; ++c) s_f[c][t] = (A)0;
+    for (int c = 0; c < 3; ++c) s_f.clear(c, t);
     __syncthreads();
     const int kind = term.kind_atoms >> 24;
     const int i = term.kind_atoms & 255, j = (term.kind_atoms >> 8) & 255, k = (term.kind_atoms >> 16) & 255;
@@ -87,7 +129,7 @@ __global__ __launch_bounds__(TERM_THREADS) void k_fold(int ntiles, const Term* _
             const double pk[3] = {s_pos[0][k], s_pos[1][k], s_pos[2][k]};
             e = angle_xyz(pi, pj, pk, term.p[0], term.p[1], fi, fk);
             for (int c = 0; c < 3; ++c) {
-                lds_force(&s_f[c][k], fk[c], status);
+                s_f.add(c, k, fk[c], status);
                 fk[c] += fi[c];
             }
         } else {
@@ -99,14 +141,16 @@ __global__ __launch_bounds__(TERM_THREADS) void k_fold(int ntiles, const Term* _
             for (int c = 0; c < 3; ++c) fk[c] = fi[c];
         }
         for (int c = 0; c < 3; ++c) {
-            lds_force(&s_f[c][i], fi[c], status);
-            lds_force(&s_f[c][j], -fk[c], status);
+            s_f.add(c, i, fi[c], status);
+            s_f.add(c, j, -fk[c], status);
         }
     }
     __syncthreads();
     if (a >= 0)
-        for (int c = 0; c < 3; ++c)
-            if (s_f[c][t] != (A)0) add_raw(force + 3 * (size_t)a + c, s_f[c][t]);
+        for (int c = 0; c < 3; ++c) {
+            const A v = s_f.total(c, t, status);
+            if (v != (A)0) add_raw(force + 3 * (size_t)a + c, v);
+        }
     if (energy) {
         // A wave's terms are of its first lane's kind; one add per kind and
         // workgroup (they meet on one address).
