@@ -110,8 +110,8 @@ __device__ __forceinline__ double pair_energy_fp64(double r2, double sig, double
 
 // Lane permutations by DPP inside each row of 16 lanes: quad_perm [1,0,3,2]
 // is lane ^ 1, quad_perm [3,2,1,0] is lane ^ 3, row_half_mirror is lane ^ 7
-// (each group of 8 reversed).
-constexpr int DPP_XOR1 = 0xB1, DPP_XOR3 = 0x1B, DPP_XOR7 = 0x141;
+// (each group of 8 reversed), row_ror:8 is lane ^ 8.
+constexpr int DPP_XOR1 = 0xB1, DPP_XOR3 = 0x1B, DPP_XOR7 = 0x141, DPP_XOR8 = 0x128;
 
 // Every control used here reads a lane of the same row, so no lane falls
 // back to an old value and the move needs none.
@@ -183,10 +183,25 @@ __device__ __forceinline__ unsigned valid_entries(const int* js, const unsigned 
 }
 
 // Sum over the eight groups (lanes l, l ^ 8, l ^ 16, ...).
-template <class T>
-__device__ __forceinline__ T group_sum(T v) {
+__device__ __forceinline__ double group_sum(double v) {
     for (int o = CLUSTER; o < 64; o <<= 1) v += __shfl_xor(v, o, 64);
     return v;
+}
+// Likewise, by register permutations: a swap of the odd rows (or the upper half) with a
+// copy's even rows (lower half) leaves the two partners' values in the two results.
+__device__ __forceinline__ long long group_sum(long long v) {
+    v += __double_as_longlong(dpp<DPP_XOR8>(__longlong_as_double(v)));
+    auto joined = [](unsigned lo, unsigned hi) { return (long long)(((unsigned long long)hi << 32) | lo); };
+    {
+        const unsigned lo = (unsigned)v, hi = (unsigned)((unsigned long long)v >> 32);
+        const auto l = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
+        const auto h = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+        v = joined(l[0], h[0]) + joined(l[1], h[1]);
+    }
+    const unsigned lo = (unsigned)v, hi = (unsigned)((unsigned long long)v >> 32);
+    const auto l = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
+    const auto h = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
+    return joined(l[0], h[0]) + joined(l[1], h[1]);
 }
 // A lane's force on its i-atom over a task.  Mixed form: each tile's FP32 sum is
 // rounded to multiples of 2^-32, the accumulators' step, which are added as
@@ -217,13 +232,15 @@ struct FixedForce {
             large[c] += small ? 0.0 : (double)f[c];
         }
     }
-    __device__ __forceinline__ long long total(int c, unsigned* status) const {
-        const long long s = group_sum(sum[c]);  // below 2^56
-        if (__ballot(large[c] != 0.0) == 0ull) return s;
+    __device__ __forceinline__ void totals(long long t[3], unsigned* status) const {
+        for (int c = 0; c < 3; ++c) t[c] = group_sum(sum[c]);  // below 2^56
+        if (__ballot(large[0] != 0.0 || large[1] != 0.0 || large[2] != 0.0) == 0ull) return;
         // The range is that of the whole task's force.
-        const double l = group_sum(large[c]);
-        if (!(fabs(l * FORCE_SCALE + (double)s) < 9.0e18)) return to_fixed(l + (double)s * (1.0 / FORCE_SCALE), FORCE_SCALE, status);
-        return s + (long long)(l * FORCE_SCALE);
+        for (int c = 0; c < 3; ++c) {
+            const double l = group_sum(large[c]);
+            if (fabs(l * FORCE_SCALE + (double)t[c]) < 9.0e18) t[c] += (long long)(l * FORCE_SCALE);
+            else t[c] = to_fixed(l + (double)t[c] * (1.0 / FORCE_SCALE), FORCE_SCALE, status);
+        }
     }
 };
 struct PlainForce {
@@ -233,7 +250,9 @@ struct PlainForce {
         x[1] += fy;
         x[2] += fz;
     }
-    __device__ __forceinline__ double total(int c, unsigned*) const { return group_sum(x[c]); }
+    __device__ __forceinline__ void totals(double t[3], unsigned*) const {
+        for (int c = 0; c < 3; ++c) t[c] = group_sum(x[c]);
+    }
 };
 __device__ __forceinline__ void add_total(long long* p, long long v) {
     if (v) atomicAdd(reinterpret_cast<unsigned long long*>(p), (unsigned long long)v);
@@ -566,11 +585,12 @@ __global__ __launch_bounds__(64) void k_pairs(const double* __restrict__ pos, co
             r0 = r1;
         }
         // i-forces: the eight groups' sums, in a fixed order.
-        const A tx = ftot.total(0, status), ty = ftot.total(1, status), tz = ftot.total(2, status);
+        A ft[3];
+        ftot.totals(ft, status);
         if (grp == 0 && ia >= 0) {
-            add_total(fslot + is, tx);
-            add_total(fslot + P.nslots + is, ty);
-            add_total(fslot + 2 * P.nslots + is, tz);
+            add_total(fslot + is, ft[0]);
+            add_total(fslot + P.nslots + is, ft[1]);
+            add_total(fslot + 2 * P.nslots + is, ft[2]);
         }
         if (ENERGY) {
             double etot = wave_sum(eacc);
