@@ -1325,6 +1325,7 @@ double NbOperator::mesh_charges(const double* pos, const double* box, double alp
     }
     const double saved_max = pme_.max_charge;
     pme_.max_charge = qmax;  // selects the spread's staging; the FP64 grid is exact either way
+    pme_.unordered = pme_.charges_only = true;  // these positions have no list
     const int phases = count > 0 ? (PME_SPREAD | PME_FFT) : PME_ALL;
     double* out = host_out_.at_least(std::max(3 * (size_t)n, (size_t)count));
     EvalResult* res = host_res_.at_least(1);
@@ -1332,10 +1333,8 @@ double NbOperator::mesh_charges(const double* pos, const double* box, double alp
     for (int attempt = 0; attempt < 8; ++attempt) {
         hipLaunchKernelGGL(k_mesh_begin, dim3((3 * n + 255) / 256), dim3(256), 0, s, n, in, pos_dev_.p, mesh_q_.p,
                            force_d_.p, energy_d_.p, status_.p);
-        pme_.unsorted = true;  // these positions have no list
         pme_run(pme_, MESH_F64, nl_, pos_dev_.p, mesh_q_.p, sys_dev_.p, nullptr, force_d_.p, nullptr, energy_d_.p,
                 status_.p, s, phases);
-        pme_.unsorted = false;
         // The potentials or the forces go straight to page-locked memory.
         if (count > 0) pme_potential_at(pme_, sys_dev_.p, pos_dev_.p, mesh_atoms_.p, count, out, s);
         const size_t n3 = count > 0 ? 0 : 3 * (size_t)n;
@@ -1587,6 +1586,9 @@ void NbOperator::compute(const double* pos, const double* box, bool direct, bool
     double* out = forces_dev_out ? forces_dev_out : (forces ? host_out_.at_least(n3) : nullptr);
     EvalResult* res = host_res_.at_least(1);
     const double lim = 0.5 * nl_.skin;
+    // Without a list check the order may be that of any earlier conformation.
+    pme_.unordered = pme_lj_.unordered = !direct;
+    pme_.charges_only = false;
     for (int attempt = 0; attempt < 6; ++attempt) {
         const double* src = attempt > 0 ? pos_dev_.p : (pos_dev_in ? pos_dev_in : host_in_.p);
         const double* built = direct ? nl_.pos_build.p : nullptr;

@@ -11,8 +11,13 @@ namespace ommhip {
 
 constexpr int CHARGE_PLANE_THREADS = 1024;
 constexpr int PLANE_POINTS = 6144;   // points of the largest plane
-// Every plane reads every position: 16,384 charges on 20 planes 64 us against 173 by
-// atomics (whole calls), and both grow with the charges.
+// Every plane reads every position, so the planes pay up to a product of planes and
+// charges: by planes and by tiles, whole calls in microseconds, 16,000 charges on 30
+// planes 134, 199; 60,000 on 64 363, 401; 60,000 on 512 (3.1e7) 576, 611; 32,000 on
+// 1,000 (3.2e7) 357, 363; but 60,000 on 1,000 (6e7) 507, 488.
+constexpr long long PLANE_WORK = 40000000;
+constexpr bool planes_pay(int planes, int charges) { return (long long)planes * charges <= PLANE_WORK; }
+// Charges of the allocation-free mesh (at most 64 planes), which has no tiles to change to.
 constexpr int PLANE_CHARGES = 65536;
 
 // s_plane[y * dims[2] + z] receives plane x (all threads of the workgroup call;

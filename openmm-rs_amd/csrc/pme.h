@@ -52,8 +52,9 @@ struct PmeDev {
     // Atom-owned spread (chunks of sorted atoms summed in LDS boxes) instead
     // of the tile-owned one; both write the same bits.
     bool spread_atoms = false;
-    // One system whose atoms no list has ordered (FP64 grids): a plane per workgroup.
-    bool unsorted = false;
+    // No list has put the atoms of this run in spatial order.  A mesh of charges
+    // alone (one system, FP64 grid) may then be spread plane by plane.
+    bool unordered = false, charges_only = false;
     int planes = 0, plane_points = 0;
     size_t fft_shmem[2][3] = {};  // dynamic LDS per axis
     // Matrix-core passes (dft.h), for the systems of dft_system: workgroup

@@ -1060,13 +1060,6 @@ void launch_spread_atoms(const PmeDev& pm, const NlistDev& nl, const int* order,
         hipLaunchKernelGGL(kernel, dim3(nl.nchunks * (PME_CHUNK / atoms)), dim3(ATOM_SPREAD_THREADS), 0, s,
                            nl.chunk_off.p, pm.nsys, order, pos, charge, sys, qgrid, status);
     };
-    if constexpr (std::is_same<G, double>::value) {
-        if (pm.unsorted && pm.plane_points <= PLANE_POINTS && pm.natoms <= PLANE_CHARGES) {
-            hipLaunchKernelGGL(k_spread_planes, dim3(pm.planes), dim3(CHARGE_PLANE_THREADS), 0, s, pm.natoms, pos, charge,
-                               sys, qgrid);
-            return;
-        }
-    }
     if (!order)
         hipLaunchKernelGGL((k_spread_direct<R, G, I32>), dim3((5 * pm.natoms + 255) / 256), dim3(256), 0, s, pm.natoms,
                            pos, charge, pm.atom_sys, sys, qgrid, status);
@@ -1077,6 +1070,19 @@ void launch_spread_atoms(const PmeDev& pm, const NlistDev& nl, const int* order,
     else
         chunks(k_spread_atoms<R, G, I32, 64>, 64);
 }
+
+// Atoms in no order spread by planes where those pay, else by tiles: chunks of them
+// fit no box, and each atom then adds to 125 points of the grid, which only few
+// atoms do sooner (reciprocal-only calls, by chunks and by tiles: 9,000 atoms 132, 150
+// us; 23,550 272, 216; 90,000 1,004, 684; charges on 100^3 points: 8,000 320, 334;
+// 16,000 392, 366).
+constexpr int UNORDERED_CHUNKS = 12000;
+template <class G>
+bool by_planes(const PmeDev& pm) {
+    return std::is_same<G, double>::value && pm.charges_only && pm.plane_points <= PLANE_POINTS &&
+           planes_pay(pm.planes, pm.natoms);
+}
+bool by_tiles(const PmeDev& pm) { return !pm.spread_atoms || (pm.unordered && pm.natoms > UNORDERED_CHUNKS); }
 
 template <class R, class G, class A>
 void run_t(PmeDev& pm, const NlistDev& nl, bool atom_order, const double* pos, const double* charge,
@@ -1092,7 +1098,11 @@ void run_t(PmeDev& pm, const NlistDev& nl, bool atom_order, const double* pos, c
     if (phases & PME_SPREAD) {
         const int* order = atom_order ? own : nl.sorted_atom.p;
         const int small = pm.max_charge <= SPREAD32_MAX_CHARGE ? 1 : 0;
-        if (pm.spread_atoms) {
+        if (by_planes<G>(pm)) {
+            if constexpr (std::is_same<G, double>::value)
+                hipLaunchKernelGGL(k_spread_planes, dim3(pm.planes), dim3(CHARGE_PLANE_THREADS), 0, s, pm.natoms, pos,
+                                   charge, sys, qgrid);
+        } else if (!by_tiles(pm)) {
             constexpr bool I32 = sizeof(R) == 4 && SpreadSum<R, G, false>::FIXED;
             if (I32 && small) launch_spread_atoms<R, G, I32>(pm, nl, order, pos, charge, sys, qgrid, status, s);
             else launch_spread_atoms<R, G, false>(pm, nl, order, pos, charge, sys, qgrid, status, s);
@@ -1111,7 +1121,7 @@ void run_t(PmeDev& pm, const NlistDev& nl, bool atom_order, const double* pos, c
     }
     if (phases & PME_FFT) {
         Cx<R>* cg = reinterpret_cast<Cx<R>*>(cgrid);
-        int* clear = (phases & PME_SPREAD) && !pm.spread_atoms ? pm.bin_count.p : nullptr;
+        int* clear = (phases & PME_SPREAD) && !by_planes<G>(pm) && by_tiles(pm) ? pm.bin_count.p : nullptr;
         constexpr int prec = sizeof(R) == 8 ? 1 : 0;
         if (pm.dft_blocks[prec][0] > 0) {
             launch_dft<R, G, A>(pm, sys, qgrid, cgrid, phi, roots, moduli, energy, status, s, clear, pm.ntiles);
