@@ -273,6 +273,13 @@ __host__ __device__ inline uint64_t pair_key(int32_t i, int32_t j) {
     return z ^ (z >> 31);
 }
 
+// Orders a wave's LDS accesses on either side, its other lanes' included, where the
+// wave's lanes hand values to one another through LDS.
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 __device__ __forceinline__ double wave_sum(double v) {
     for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
     return v;

@@ -243,12 +243,6 @@ __device__ __forceinline__ typename Mat<R>::V4 dft_rows(const R* b, int n, int r
     return total.total();
 }
 
-// Orders a wave's LDS writes before its other lanes' reads.
-__device__ __forceinline__ void wave_lds_fence() {
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
-
 // Every load of a workgroup is issued without a branch (indices past the end
 // read the last element and are masked when stored to LDS): behind a branch the
 // compiler waits for each load before the next.

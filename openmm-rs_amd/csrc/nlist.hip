@@ -917,7 +917,7 @@ __global__ __launch_bounds__(64 * CLIST_WAVES) void k_clist(
                 constexpr int NEAR_ROUND = 4;
                 if (pass)
                     s_near[wave][__popcll(m & below)] = make_float4(dcf[0], dcf[1], dcf[2], __int_as_float(J));
-                __builtin_amdgcn_wave_barrier();
+                wave_lds_fence();
                 struct Near {
                     float4 dc, q;
                     int2 range;
@@ -945,6 +945,7 @@ __global__ __launch_bounds__(64 * CLIST_WAVES) void k_clist(
 #pragma unroll
                     for (int u = 0; u < NEAR_ROUND / 2; ++u) e[u] = next[u];
                 }
+                wave_lds_fence();  // before the next line-up
                 return;
             }
             // Four passing blocks per round: lanes 0-31 take the first of

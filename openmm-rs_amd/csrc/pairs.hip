@@ -623,11 +623,6 @@ __global__ __launch_bounds__(64) void k_pairs(const double* __restrict__ pos, co
 constexpr int ENERGY_WAVES = 4;           // waves per workgroup
 constexpr int ENERGY_WORKGROUPS = 768;    // at most: three waves per SIMD of the chip
 
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
-
 template <int KIND>
 __global__ __launch_bounds__(64 * ENERGY_WAVES) void k_pair_energy(
     const double* __restrict__ pos, const double* __restrict__ qk, const double* __restrict__ sh,
@@ -696,7 +691,7 @@ __global__ __launch_bounds__(64 * ENERGY_WAVES) void k_pair_energy(
             s_js[lane] = live && e0.y >= 0 ? e0.x : INT_MAX;
             s_ja[lane] = e0.y;
             s_ex[lane] = (unsigned char)x0;
-            wave_sync();
+            wave_lds_fence();
             const unsigned present = valid_entries(s_js + grp * CLUSTER, s_ex + grp * CLUSTER, is, il);
             const unsigned vmask = ia >= 0 ? present : 0u;
             double eacc = 0.0;
@@ -726,7 +721,7 @@ __global__ __launch_bounds__(64 * ENERGY_WAVES) void k_pair_energy(
                         if constexpr ((KIND & PAIR_LJPME) != 0) ring[4][at] = si * sj.x;
                     }
                     waiting += __popcll(m);
-                    wave_sync();
+                    wave_lds_fence();
                     if (waiting < 64) continue;
                 } else if (waiting == 0) {
                     break;
@@ -739,11 +734,11 @@ __global__ __launch_bounds__(64 * ENERGY_WAVES) void k_pair_energy(
                 const int taken = min(waiting, 64);
                 head += taken;
                 waiting -= taken;
-                wave_sync();
+                wave_lds_fence();
             }
             const double et = wave_sum(eacc);
             esum += to_fixed(et, ENERGY_SCALE, status);
-            wave_sync();
+            wave_lds_fence();
             e0 = e1;
             x0 = x1;
         }
