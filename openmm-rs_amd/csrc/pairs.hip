@@ -482,15 +482,6 @@ __global__ __launch_bounds__(64) void k_pairs(const double* __restrict__ pos, co
                 }
                 return f;
             };
-            // Energy and statistics of an accepted pair (their variants only).
-            auto pair_extra = [&](const int slot, const R e) {
-                if (ENERGY) eacc += (double)e;
-                if (STATS) {
-                    const int ja = s_ja[slot];
-                    ++npair;
-                    hsum += pair_key(min(ia, ja), max(ia, ja));
-                }
-            };
             // Step k: lane (grp, il) pairs i-atom il with entry grp * 8 + (il ^ k);
             // each entry meets every i-atom of the cluster once over the 8 steps.
             // Pairs whose FP32 r^2 falls in the band around the cutoff are only
@@ -502,7 +493,10 @@ __global__ __launch_bounds__(64) void k_pairs(const double* __restrict__ pos, co
             // (away from the singularity at 0) and its force selected to zero.
             // The minimum-image choice is made once per tile, outside the
             // steps, so the eight steps form one straight block.
-            unsigned near = 0;
+            // Energies are selected and the statistics' pairs marked and counted
+            // afterwards: behind a branch in each step the FP64 forms needed up to 284
+            // registers, the rest beyond 256 in accumulation registers.
+            unsigned near = 0, taken = 0;
             auto pair_step = [&](const int k, auto MI) {
                 const int s8 = il ^ k;
                 const int slot = grp * CLUSTER + s8;
@@ -517,7 +511,8 @@ __global__ __launch_bounds__(64) void k_pairs(const double* __restrict__ pos, co
                 R e;
                 R f = pair_fe(pj.w, sj, in ? r2 : (R)1, e);
                 f = in ? f : (R)0;
-                if ((ENERGY || STATS) && in) pair_extra(slot, e);
+                if (ENERGY) eacc += in ? (double)e : 0.0;
+                if (STATS) taken |= in ? 1u << s8 : 0u;
                 fx += f * dx;
                 fy += f * dy;
                 fz += f * dz;
@@ -557,7 +552,8 @@ __global__ __launch_bounds__(64) void k_pairs(const double* __restrict__ pos, co
                         if (mi) delta(pj, dx, dy, dz, std::true_type{});
                         else delta(pj, dx, dy, dz, std::false_type{});
                         const R f = pair_fe(pj.w, s_se[slot], dx * dx + dy * dy + dz * dz, e);
-                        if (ENERGY || STATS) pair_extra(slot, e);
+                        if (ENERGY) eacc += (double)e;
+                        if (STATS) taken |= 1u << s8;
                         fx += f * dx;
                         fy += f * dy;
                         fz += f * dz;
@@ -568,6 +564,12 @@ __global__ __launch_bounds__(64) void k_pairs(const double* __restrict__ pos, co
                     }
                 }
             }
+            if (STATS)
+                for (; taken; taken &= taken - 1u) {
+                    const int ja = s_ja[grp * CLUSTER + __ffs(taken) - 1];
+                    ++npair;
+                    hsum += pair_key(min(ia, ja), max(ia, ja));
+                }
             // After step 7 the lane holds the accumulator of entry grp * 8 + (il ^ 7).
             const int jmine = grp * CLUSTER + (il ^ (CLUSTER - 1));
             if (s_ja[jmine] >= 0) {
