@@ -261,8 +261,15 @@ __device__ __forceinline__ void add_total(double* p, double v) {
     if (v != 0.0) unsafeAtomicAdd(p, v);
 }
 
+// FP64 forces with energies beside a mesh: one wave per SIMD, though the registers
+// allow two, so that the mesh's kernels find room beside them (9,000 atoms, a call
+// of energy and forces 481 us with two, 430 with one; the kernel alone 64 either way).
+constexpr int pair_waves_per_simd(int kind, bool energy) {
+    return energy && (kind & ELEC_MASK) == ELEC_EWALD ? 1 : 8;
+}
+
 template <class R, class A, int KIND, bool STATS, bool ENERGY>
-__global__ __launch_bounds__(64) void k_pairs(const double* __restrict__ pos, const R* __restrict__ qk,
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, pair_waves_per_simd(KIND, ENERGY)))) void k_pairs(const double* __restrict__ pos, const R* __restrict__ qk,
                                               const R* __restrict__ sh, const R* __restrict__ e2,
                                               const int* __restrict__ sorted_atom,
                                               const unsigned char* __restrict__ clist_ex,
