@@ -226,6 +226,12 @@ __device__ __forceinline__ long long to_fixed(double v, double scale, unsigned* 
     return (long long)s;
 }
 
+// Likewise to the nearest step, for sums of many parts of one sign: each cut off, they
+// lose half a step a part.
+__device__ __forceinline__ long long to_fixed_nearest(double v, double scale, unsigned* status) {
+    return to_fixed(rint(v * scale) / scale, scale, status);
+}
+
 __device__ __forceinline__ void add_fixed(long long* dst, double v, double scale, unsigned* status) {
     long long q = to_fixed(v, scale, status);
     if (q) atomicAdd(reinterpret_cast<unsigned long long*>(dst), (unsigned long long)q);

@@ -620,8 +620,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, pair_wave
 // pair set: FP64 offsets and parameters, the cutoff decided as the pair kernel
 // decides it (exactly, near the cutoff).  A kernel of its own: within the pair
 // kernel the FP64 values took its registers to one or two waves per SIMD.
-// Waves loop over tasks; each tile's sum is added in fixed point, so neither
-// the tasks' size nor their order changes the total.  Adds to one energy
+// Waves loop over tasks; each tile's sum is rounded to fixed point and added, so
+// neither the tasks' size nor their order changes the total.  Adds to one energy
 // serialise (12 ns each: one per task was 60 us at 9,000 atoms), so few waves
 // are launched and a workgroup adds once when its waves saw one system.
 // Bound: FP64 issue.  36% of a tile's slots are in range: they are lined up in
@@ -746,7 +746,7 @@ __global__ __launch_bounds__(64 * ENERGY_WAVES) void k_pair_energy(
                 wave_lds_fence();
             }
             const double et = wave_sum(eacc);
-            esum += to_fixed(et, ENERGY_SCALE, status);
+            esum += to_fixed_nearest(et, ENERGY_SCALE, status);
             wave_lds_fence();
             e0 = e1;
             x0 = x1;

@@ -35,6 +35,26 @@ def test_weak_forces_keep_the_accumulators_step(eps):
     assert worst <= 1.0
 
 
+def test_pair_energies_are_rounded_not_cut():
+    # Charges of one sign: every tile's energy is positive.  Some 8,000 tiles, rounded to a
+    # step each: 0.29 x sqrt(8,000) = 26 steps of scatter, of which 200 allow for several
+    # deviations and for the FP64 sums (1e-15 of 1e6 kJ/mol).  Cut to a step each they
+    # lose 4,000.
+    rng = np.random.default_rng(8)
+    f = ommhip.NonbondedForce()
+    f.set_nonbonded_method("CutoffPeriodic")
+    f.set_cutoff_distance(0.9)
+    for _ in range(9000):
+        f.add_particle(0.1, 0.3, 0.0)
+    pos, box, direct = rng.uniform(0.0, 4.48, (9000, 3)), 4.48 * np.eye(3), []
+    for precision in (ommhip.PRECISION_MIXED, ommhip.PRECISION_DOUBLE):
+        op = ommhip.GpuNonbondedForce(f, precision)
+        op.initialize(box)
+        direct.append(op.energy_parts(pos, box)[0])
+    print(direct, (direct[0] - direct[1]) / STEP)
+    assert abs(direct[0] - direct[1]) <= 200 * STEP
+
+
 def _one_against(offsets, eps):
     """An atom and partners that do not act on each other, at its position plus the offsets."""
     n = len(offsets)
