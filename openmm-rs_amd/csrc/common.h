@@ -317,23 +317,6 @@ __device__ __forceinline__ void wave_raise_flags(int* flag, bool moved, int si) 
     if (mixed && moved && si != lead && !__atomic_load_n(flag + 1 + si, __ATOMIC_RELAXED)) atomicOr(flag + 1 + si, 1);
 }
 
-// Adds each lane's energy v to slot `slot` of its system si (si < 0: lane
-// idle) in the per-system energy array: one atomic per wave when the active
-// lanes share a system, one per lane otherwise.  Called by all 64 lanes; a
-// null energy array (force-only evaluations) adds nothing.
-template <class A>
-__device__ __forceinline__ void wave_energy_add(A* energy, int si, int slot, double v, unsigned* status) {
-    if (!energy) return;  // force-only evaluation
-    const int lead = __shfl(si, 0, 64);  // lane 0 holds the lowest index, so it is active if any lane is
-    const bool uniform = __ballot(si >= 0 && si != lead) == 0ull;
-    if (uniform) {
-        const double t = wave_sum(v);
-        if ((threadIdx.x & 63) == 0 && lead >= 0 && t != 0.0) acc_add(energy + lead * E_SLOTS + slot, t, ENERGY_SCALE, status);
-    } else if (si >= 0 && v != 0.0) {
-        acc_add(energy + si * E_SLOTS + slot, v, ENERGY_SCALE, status);
-    }
-}
-
 // Reduced-triclinic minimum image in the reference's operation order
 // (harmonic_bond.rs:152-159): c, then b, then a; no fused multiply-add.
 __device__ __forceinline__ void min_image_exact(double d[3], const double* bv) {

@@ -5,7 +5,6 @@
 #include <climits>
 #include <cmath>
 #include <cstring>
-#include <functional>
 #include <random>
 #include <map>
 #include <numeric>

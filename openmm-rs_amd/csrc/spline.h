@@ -6,9 +6,6 @@
 
 namespace ommhip {
 
-// Order-5 cardinal B-spline weights and derivatives (pme.rs:151-174).  Which
-// products are fused is written out: the spreads' kernels have to agree in
-// every bit, and the compiler's own choice varies from kernel to kernel.
 // x / 3, correctly rounded (P. Markstein, IA-64 and Elementary Functions, 2000:
 // a quotient within an ulp, corrected by its exact remainder times the rounded
 // reciprocal), in three instructions instead of the general division's ten.
@@ -18,6 +15,9 @@ __device__ __forceinline__ R third(R x) {
     return fma(fma(q, (R)-3, x), r, q);
 }
 
+// Order-5 cardinal B-spline weights and derivatives (pme.rs:151-174).  Which
+// products are fused is written out: the spreads' kernels have to agree in
+// every bit, and the compiler's own choice varies from kernel to kernel.
 template <class R>
 __device__ __forceinline__ void spline5(R f, R w[5], R dw[5]) {
 #pragma clang fp contract(off)
