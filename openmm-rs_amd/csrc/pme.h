@@ -91,8 +91,8 @@ struct PmeDev {
 // FP64).  The dense products' work grows with n, the staged passes' with the
 // sum of n's prime factors (4 and 8 preferred).  Both transforms and the
 // convolution of n^3 points, staged then dense, microseconds:
-//   FP32: 19: 25, 14   55: 31, 21   72: 54, 39   96: 77, 71   120: 116, 104
-//         128: 129, 137   but 101: 228, 79 and 127: 430, 112
+//   FP32: 19: 25, 15   55: 31, 22   72: 54, 40   96: 77, 72   120: 114, 106
+//         128: 129, 138   but 101: 230, 80 and 127: 434, 113
 //   FP64: 19: 27, 17   55: 37, 27   64: 46, 40   72: 68, 70   96: 110, 120
 //         but 101: 403, 130
 // so every axis has at most 120 (FP32) or 64 points (FP64), or at most DFT_MAX

@@ -264,8 +264,9 @@ __global__ __launch_bounds__(SPREAD_THREADS) void k_spread_tiles(const int* __re
 constexpr int SPREAD_BOX_BYTES = 32768;
 constexpr int ATOM_SPREAD_WAVES = 4, ATOM_SPREAD_THREADS = 64 * ATOM_SPREAD_WAVES;
 // Smaller groups where that gives idle compute units work (chunks: time with 64,
-// 32 and 16 slots per workgroup, us): 15: 17, 12, 10; 141: 14, 11, 10; 368: 15, 14,
-// 20; 938: 24, 30, 40 (FP32 stencils).  FP64 ones at 360: 54, 43, 47.
+// 32 and 16 slots per workgroup, us).  FP32 stencils, 15: 16, 10, 9; 141: 13, 10, 10;
+// 235: 13, 11, 11; 368: 14, 13, 18; 469: 14, 16, 19; 938: 24, 27, 35.  FP64 ones, 282: 16,
+// 12, 18; 368: 16, 14, 19; 469: 19, 17, 21; 563: 17, 24, 27.
 constexpr int SPREAD_16_CHUNKS = 192, SPREAD_32_CHUNKS = 256, SPREAD_32_CHUNKS_F64 = 512;
 static_assert(PME_CHUNK == 64, "a wave of the atom-owned spread holds a chunk");
 

@@ -546,7 +546,8 @@ class GpuNonbondedForce:
         return (e.value if energy else None), bool(ev.value)
 
     def calc_forces(self, pos, box=None):
-        """Forces only (energy_out = NULL): the MD step's FP32 path."""
+        """Forces only (energy_out = NULL): no energies are evaluated; the mixed form's
+        pairs in FP32 and its mesh in FP64, as beside an energy."""
         p = _f64(pos).reshape(-1, 3)
         b, bp = _box_ptr(box)
         f = np.zeros_like(p)
