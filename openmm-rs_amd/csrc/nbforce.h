@@ -319,6 +319,7 @@ private:
     // Host-API scratch.
     DevBuf<double> pos_dev_;
     DevBuf<double> mesh_q_;  // mesh_charges: charges
+    DevBuf<double> out_dev_;  // forces on their way to an array that is not written in place
     DevBuf<int> mesh_atoms_;
     DevBuf<long long> force_fx_, energy_fx_;
     DevBuf<double> force_d_, energy_d_;

@@ -108,6 +108,34 @@ bool copy_finite(const double* src, double* dst, size_t n) {
     return worst != 0x7ff0000000000000ull;
 }
 
+// Whether one allocation of the current device holds the caller's array, so that kernels
+// may use it in place.  An array that leaves its allocations is an error here, before any
+// kernel touches it; other memory (host, another device) is left to the copy calls.
+bool device_array(const void* p, size_t bytes) {
+    hipPointerAttribute_t a{};
+    int device = 0;
+    if (hipPointerGetAttributes(&a, p) != hipSuccess || hipGetDevice(&device) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    if (a.type != hipMemoryTypeDevice || a.device != device) return false;
+    const char *at = static_cast<const char*>(p), *const end = at + bytes;
+    for (bool whole = true; at < end; whole = false) {
+        hipDeviceptr_t base = nullptr;
+        size_t size = 0;
+        if (hipMemGetAddressRange(&base, &size, const_cast<char*>(at)) != hipSuccess) {
+            (void)hipGetLastError();
+            if (whole) return false;
+            throw Error(OMM_ERR_INVALID, "a device array is shorter than its particles need");
+        }
+        const char* to = static_cast<const char*>(base) + size;
+        if (to >= end) return whole;
+        if (to <= at) return false;
+        at = to;  // the next of several mapped ranges, or past the array
+    }
+    return true;
+}
+
 void validate_particle(double q, double s, double e) {
     // nonbonded.rs:1252-1261
     if (!(std::isfinite(q) && std::isfinite(s) && std::isfinite(e) && s >= 0.0 && e >= 0.0))
@@ -1534,6 +1562,9 @@ void NbOperator::compute(const double* pos, const double* box, bool direct, bool
     if (!pos && !pos_dev_in) throw Error(OMM_ERR_INVALID, "positions must not be null");
     check_box(box);
     const int n = n_[0];
+    const size_t bytes = 3 * (size_t)n * sizeof(double);
+    const bool read_in_place = pos_dev_in && n > 0 && device_array(pos_dev_in, bytes);
+    const bool write_in_place = forces_dev_out && n > 0 && device_array(forces_dev_out, bytes);
     // Device positions: a non-periodic method chooses its virtual box from a
     // host copy; otherwise non-finite positions surface as non-finite forces.
     std::vector<double> host_pos;
@@ -1575,6 +1606,7 @@ void NbOperator::compute(const double* pos, const double* box, bool direct, bool
         // once the results are complete, as the host form does.
         OMM_HIP(hipEventRecord(ev_caller_, caller));
         OMM_HIP(hipStreamWaitEvent(s, ev_caller_, 0));
+        if (!read_in_place) OMM_HIP(hipMemcpyAsync(pos_dev_.p, pos_dev_in, bytes, hipMemcpyDeviceToDevice, s));
     }
     const bool want_stats = num_pairs || pair_hash;
     // Pair statistics are gathered by a force-only pass; energies by the
@@ -1583,14 +1615,17 @@ void NbOperator::compute(const double* pos, const double* box, bool direct, bool
     const int mode = mesh_mode(!want_stats);
     const NbSettings& c = cfg_[0];
     const size_t n3 = 3 * (size_t)n;
-    double* out = forces_dev_out ? forces_dev_out : (forces ? host_out_.at_least(n3) : nullptr);
+    const bool copy_out = forces_dev_out && !write_in_place;
+    if (copy_out) out_dev_.alloc_at_least(n3);
+    double* out = copy_out ? out_dev_.p : (forces_dev_out ? forces_dev_out : (forces ? host_out_.at_least(n3) : nullptr));
     EvalResult* res = host_res_.at_least(1);
     const double lim = 0.5 * nl_.skin;
     // Without a list check the order may be that of any earlier conformation.
     pme_.unordered = pme_lj_.unordered = !direct;
     pme_.charges_only = false;
     for (int attempt = 0; attempt < 6; ++attempt) {
-        const double* src = attempt > 0 ? pos_dev_.p : (pos_dev_in ? pos_dev_in : host_in_.p);
+        const double* src = attempt > 0 || (pos_dev_in && !read_in_place) ? pos_dev_.p
+                                                                          : (pos_dev_in ? pos_dev_in : host_in_.p);
         const double* built = direct ? nl_.pos_build.p : nullptr;
         const int rebuild = direct && (list_stale_ || attempt > 0) ? 1 : 0;
         const dim3 wgs((n + EVAL_WG - 1) / EVAL_WG);
@@ -1648,6 +1683,10 @@ void NbOperator::compute(const double* pos, const double* box, bool direct, bool
         if (st & ST_OVERFLOW) throw Error(OMM_ERR_OVERFLOW, "fixed-point force/energy accumulator overflow");
         const double* e = res->energy;
         if (forces) std::memcpy(forces, out, n3 * sizeof(double));
+        if (copy_out) {
+            OMM_HIP(hipMemcpyAsync(forces_dev_out, out, bytes, hipMemcpyDefault, s));
+            OMM_HIP(hipStreamSynchronize(s));
+        }
         if (want_stats) {
             if (num_pairs) *num_pairs = (int64_t)res->stats[0];
             if (pair_hash) *pair_hash = res->stats[1];
